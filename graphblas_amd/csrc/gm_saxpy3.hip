@@ -35,13 +35,25 @@
 
 #include "gm_internal.h"
 #include "gm_block.h"
+#include <cstring>
 
 namespace gm
 {
 
 constexpr int SX_NT = 256;
 constexpr uint32_t SX_EMPTY = 0xffffffffu;
-enum { BIN_SINGLE = 0, BIN_WS = 1, BIN_WL = 2, BIN_BLK = 3, BIN_GLB = 4, SX_NBINS = 5 };
+// BIN_HVY collects the rows beyond the LDS tables; k_sx_classify deals them out
+// to BIN_GLB (a hash table each) and BIN_DNS (spread over the device)
+enum { BIN_SINGLE = 0, BIN_WS = 1, BIN_WL = 2, BIN_BLK = 3, BIN_GLB = 4, BIN_DNS = 5, BIN_HVY = 6, SX_NBINS = 7 };
+// counters: the bins, then
+enum { CNT_SLOTS = 8,       // table slots of BIN_GLB
+       CNT_BIGSUM = 9,      // entries of the big rows (symbolic)
+       CNT_SMALL = 10,      // flops of the small rows
+       CNT_HFLOPS = 11,     // flops of BIN_HVY
+       CNT_NNZA = 12,       // nnz(A)
+       CNT_ERR = 13,        // the look-back's error flag
+       CNT_MAXLEN = 16,     // k_sx_maxlen's six results
+       SX_NCNT = 32 };
 enum { MODE_NONE = 0, MODE_MASK = 1, MODE_NOTMASK = 2 };
 
 struct SxArgs
@@ -60,7 +72,9 @@ struct SxArgs
     int64_t *Ci;
     void *Cx;
     uint32_t *rows;               // SX_NBINS x m row ids
-    unsigned long long *cnt;      // SX_NBINS bin counters, then global slot total
+    unsigned long long *cnt;      // bin counters and totals (CNT_*)
+    int64_t *hflops;              // per BIN_HVY row: its flops
+    const unsigned long long *rowf;   // NULL, or the rows' flops (few-row A)
     int64_t *gtab_off;            // per global-bin row: offset of its table
     int32_t *gtab_log2;           // per global-bin row: log2 of its table size
     uint32_t *gkeys;
@@ -206,11 +220,20 @@ __device__ __forceinline__ void sx_ordered_upd(typename S::Z *vals, int32_t slot
     }
 }
 
+} // namespace gm
+
+#include "gm_sx_push.h"
+
+namespace gm
+{
+
 //------------------------------------------------------------------------------
 // team-of-TG helpers (TG lanes of one wavefront work on one row)
 //------------------------------------------------------------------------------
 
 constexpr int TG = 8;          // lanes per row in the flop-count and fused kernels
+constexpr int FEW_ROWS = 256;             // A with at most this many rows: k_sx_rowflops
+constexpr int64_t FLOPS_TEAM_MAX = 256;   // longer rows of A: counted by the workgroup
 constexpr int FMAX = 64;       // largest flop count of a "small" row
 
 template <class T>
@@ -293,7 +316,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_maxlen(const int64_t *__restrict__
 //------------------------------------------------------------------------------
 // flops + binning: TG lanes per row (coalesced reads of A(i,:) and of the
 // B row pointers it names).  Rows with f <= fs are "small"; their flops are
-// summed into cnt[7] (capacity for the fused kernel) and they are listed in
+// summed into cnt[CNT_SMALL] (capacity for the fused kernel) and they are listed in
 // BIN_WS (used only when the fused kernel is not).  Larger rows go to the
 // single / wave1024 / block4096 / global bins.
 //------------------------------------------------------------------------------
@@ -302,24 +325,49 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
 {
     __shared__ unsigned int s_bc[SX_NBINS];
     __shared__ unsigned long long s_base[SX_NBINS];
-    __shared__ unsigned long long s_red[SX_NT / 64];
+    __shared__ unsigned long long s_red[SX_NT / 64 + 1];
+    __shared__ int s_long[SX_NT / TG], s_nlong;
     const int sub = threadIdx.x & (TG - 1);
     const int lane = threadIdx.x & 63;
     unsigned long long fsum = 0;          // flops of this thread's small rows
+    if (blockIdx.x == 0 && threadIdx.x == 0) g.cnt[CNT_NNZA] = (unsigned long long) g.Ap[g.m];
     for (int64_t base = (int64_t) blockIdx.x * (SX_NT / TG); base < g.m;
          base += (int64_t) gridDim.x * (SX_NT / TG))
     {
         const int64_t i = base + threadIdx.x / TG;
         int64_t f = 0, a0 = 0, a1 = 0;
+        if (threadIdx.x == 0) s_nlong = 0;
+        __syncthreads();
         if (i < g.m)
         {
             a0 = g.Ap[i];
             a1 = g.Ap[i + 1];
-            for (int64_t e = a0 + sub; e < a1; e += TG)
+            if (g.rowf) f = sub == 0 ? (int64_t) g.rowf[i] : 0;
+            else if (a1 - a0 > FLOPS_TEAM_MAX)
+            {
+                if (sub == 0) s_long[atomicAdd(&s_nlong, 1)] = threadIdx.x / TG;
+            }
+            else
+                for (int64_t e = a0 + sub; e < a1; e += TG)
+                {
+                    const int64_t k = g.Aj[e];
+                    f += g.Bp[k + 1] - g.Bp[k];
+                }
+        }
+        __syncthreads();
+        // the workgroup takes the tile's long rows together
+        for (int q = 0; q < s_nlong; q++)
+        {
+            const int64_t r = base + s_long[q], r1 = g.Ap[r + 1];
+            unsigned long long fl = 0;
+            #pragma unroll 4
+            for (int64_t e = g.Ap[r] + threadIdx.x; e < r1; e += SX_NT)
             {
                 const int64_t k = g.Aj[e];
-                f += g.Bp[k + 1] - g.Bp[k];
+                fl += (unsigned long long) (g.Bp[k + 1] - g.Bp[k]);
             }
+            const unsigned long long tot = block_sum<unsigned long long, SX_NT>(fl, s_red);
+            if (r == i && sub == 0) f = (int64_t) tot;
         }
         f = team_sum<int64_t>(f);
         int bin = -1;
@@ -338,7 +386,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
             else if (a1 - a0 == 1) bin = BIN_SINGLE;
             else if (t <= g.wl_max) bin = BIN_WL;
             else if (t <= g.blk_max) bin = BIN_BLK;
-            else bin = BIN_GLB;
+            else bin = BIN_HVY;
         }
         __syncthreads();
         // block-aggregated appends: LDS counters, one global atomic per bin
@@ -352,18 +400,10 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
         {
             const unsigned long long slot = s_base[bin] + local;
             g.rows[(int64_t) bin * g.m + (int64_t) slot] = (uint32_t) i;
-            if (bin == BIN_GLB)
+            if (bin == BIN_HVY)
             {
-                // table of 2^ceil(log2(2t)) slots, load factor <= 1/2, or a
-                // dense one of 2^ceil(log2(ncols)) (see SxArgs::table)
-                int lg = ilog2_ceil(2 * t);
-                const int lgd = ilog2_ceil(g.n);
-                const bool dn = (g.table == 0 && (((int64_t) 1 << lg) >= g.n / 12 || t >= g.n / 2)) ||
-                                (g.table == 2 && lgd <= lg + 4);
-                if (dn && lgd > lg) lg = lgd;
-                const unsigned long long sz = 1ull << lg;
-                g.gtab_off[slot] = (int64_t) atomicAdd(&g.cnt[SX_NBINS], sz);
-                g.gtab_log2[slot] = lg;
+                g.hflops[slot] = f;
+                atomicAdd(&g.cnt[CNT_HFLOPS], (unsigned long long) f);
             }
         }
         __syncthreads();
@@ -377,19 +417,61 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
     {
         unsigned long long tsum = 0;
         for (int w = 0; w < SX_NT / 64; w++) tsum += s_red[w];
-        if (tsum) atomicAdd(&g.cnt[7], tsum);
+        if (tsum) atomicAdd(&g.cnt[CNT_SMALL], tsum);
     }
 }
 
-// sum of the symbolic counts of the rows in the big bins -> cnt[6]
-__global__ __launch_bounds__(SX_NT) void k_sx_sum_big(SxArgs g)
+// Deals the heavy rows out.  A row takes a dense table (PUSH: the semiring and
+// the memory allow it, dmax rows at most) when its flops reach a quarter of
+// the columns, so that the table costs less than a hash table's inserts and
+// sort, or when it holds more than 1/512 of all heavy flops, so that one
+// workgroup on it would outlast the others, and at least 1/128 of the columns
+// (the table's clearing and compaction then stay below its updates).  Other
+// rows get a hash table of 2^ceil(log2(2t)) slots, load factor <= 1/2, or a
+// dense one of 2^ceil(log2(ncols)) slots (SxArgs::table).
+__global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops, int64_t dmax)
+{
+    const int64_t count = (int64_t) g.cnt[BIN_HVY];
+    const double total = (double) g.cnt[CNT_HFLOPS];
+    for (int64_t q = (int64_t) blockIdx.x * SX_NT + threadIdx.x; q < count; q += (int64_t) gridDim.x * SX_NT)
+    {
+        const uint32_t i = g.rows[(int64_t) BIN_HVY * g.m + q];
+        const int64_t f = g.hflops[q];
+        if (dmax > 0 && g.table != 1 && (f >= g.n / 4 || ((double) f * 512 > total && f >= g.n / 128)))
+        {
+            const int64_t d = (int64_t) atomicAdd(&g.cnt[BIN_DNS], 1ull);
+            if (d < dmax)
+            {
+                g.rows[(int64_t) BIN_DNS * g.m + d] = i;
+                dflops[d] = f;
+                continue;
+            }
+        }
+        int64_t t = f;
+        if (g.mode == MODE_MASK && g.Mp[i + 1] - g.Mp[i] < t) t = g.Mp[i + 1] - g.Mp[i];
+        if (t > g.n) t = g.n;
+        int lg = ilog2_ceil(2 * t);
+        const int lgd = ilog2_ceil(g.n);
+        const bool dn = (g.table == 0 && (((int64_t) 1 << lg) >= g.n / 12 || t >= g.n / 2)) ||
+                        (g.table == 2 && lgd <= lg + 4);
+        if (dn && lgd > lg) lg = lgd;
+        const int64_t slot = (int64_t) atomicAdd(&g.cnt[BIN_GLB], 1ull);
+        g.rows[(int64_t) BIN_GLB * g.m + slot] = i;
+        g.gtab_off[slot] = (int64_t) atomicAdd(&g.cnt[CNT_SLOTS], 1ull << lg);
+        g.gtab_log2[slot] = lg;
+    }
+}
+
+// sum of the symbolic counts of the rows in the big bins -> cnt[CNT_BIGSUM]
+__global__ __launch_bounds__(SX_NT) void k_sx_sum_big(SxArgs g, int64_t dmax)
 {
     __shared__ unsigned long long s_red[SX_NT / 64];
     unsigned long long sum = 0;
-    const int bins[4] = {BIN_SINGLE, BIN_WL, BIN_BLK, BIN_GLB};
-    for (int b = 0; b < 4; b++)
+    const int bins[5] = {BIN_SINGLE, BIN_WL, BIN_BLK, BIN_GLB, BIN_DNS};
+    for (int b = 0; b < 5; b++)
     {
-        const int64_t count = (int64_t) g.cnt[bins[b]];
+        int64_t count = (int64_t) g.cnt[bins[b]];
+        if (bins[b] == BIN_DNS && count > dmax) count = dmax;
         const uint32_t *list = g.rows + (int64_t) bins[b] * g.m;
         for (int64_t q = (int64_t) blockIdx.x * SX_NT + threadIdx.x; q < count;
              q += (int64_t) gridDim.x * SX_NT)
@@ -403,7 +485,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_sum_big(SxArgs g)
     {
         unsigned long long tsum = 0;
         for (int w = 0; w < SX_NT / 64; w++) tsum += s_red[w];
-        if (tsum) atomicAdd(&g.cnt[6], tsum);
+        if (tsum) atomicAdd(&g.cnt[CNT_BIGSUM], tsum);
     }
 }
 
@@ -1210,6 +1292,103 @@ static inline unsigned sx_grid(int64_t items, int64_t per_block, int64_t cap)
     return (unsigned) g;
 }
 
+// the dense rows' device arrays between their build and the writing of C
+struct SxPush
+{
+    PushArgs h;
+    DevBuf pre, coff, it_d, it_e, tab, bits, mbits, seg;
+};
+
+// bytes of one dense row
+template <class S>
+static double sx_push_row_bytes(int64_t n, bool masked)
+{
+    return (S::iso_out ? 0.0 : (double) sizeof(PuCell<S>) * (double) n) + (masked ? 0.25 : 0.125) * (double) n +
+           8.0 * (double) (n / PU_SEG + 1);
+}
+
+// tables, products and counts of the dense rows (their Cp entries)
+template <class S>
+static int sx_push_build(SxArgs &g, SxPush &p, int64_t D, int64_t nnzA, int64_t hflops)
+{
+    hipStream_t st = stream();
+    const int64_t cap = (int64_t) cu_count() * 8;
+    PushArgs &h = p.h;
+    h.D = D;
+    h.drow = g.rows + (int64_t) BIN_DNS * g.m;
+    h.nw = (g.n + 31) >> 5;
+    h.nseg = (g.n + PU_SEG - 1) / PU_SEG;
+    const int64_t items = hflops / PU_CH + D + 1;
+    const bool masked = g.mode != MODE_NONE;
+    if (!p.pre.alloc(sizeof(int64_t) * (nnzA + 1)) || !p.coff.alloc(sizeof(int64_t) * (D + 1)) ||
+        !p.it_d.alloc(sizeof(uint32_t) * items) || !p.it_e.alloc(sizeof(int64_t) * items) ||
+        (!S::iso_out && !p.tab.alloc(sizeof(PuCell<S>) * (size_t) (D * g.n))) ||
+        (PU_BITS<S> && !p.bits.alloc(sizeof(uint32_t) * (size_t) (D * h.nw))) ||
+        (masked && !p.mbits.alloc(sizeof(uint32_t) * (size_t) (D * h.nw))) ||
+        !p.seg.alloc(sizeof(int64_t) * (size_t) (D * h.nseg + 1)))
+        return set_error(GM_OUT_OF_MEMORY, "saxpy3: dense rows (%lld)", (long long) D);
+    h.pre = p.pre.as<int64_t>(); h.coff = p.coff.as<int64_t>();
+    h.it_d = p.it_d.as<uint32_t>(); h.it_e = p.it_e.as<int64_t>();
+    h.tab = p.tab.ptr; h.bits = p.bits.as<uint32_t>(); h.mbits = p.mbits.as<uint32_t>();
+    h.seg = p.seg.as<int64_t>();
+    ProfScope ps("sx_push");
+    k_sx_elen<<<sx_grid(nnzA, PU_NT, cap), PU_NT, 0, st>>>(g, nnzA, p.pre.as<int64_t>());
+    GM_TRY(scan_exclusive_i64(p.pre.as<int64_t>(), p.pre.as<int64_t>(), nnzA));
+    k_sx_push_chunks<<<sx_grid(D, PU_NT, cap), PU_NT, 0, st>>>(h);
+    GM_TRY(scan_exclusive_i64(h.coff, h.coff, D));
+    k_sx_push_items<<<sx_grid(items, PU_NT, cap), PU_NT, 0, st>>>(g, h);
+    k_sx_push_init<S><<<sx_grid(D * g.n, PU_NT * 8, cap * 2), PU_NT, 0, st>>>(h, D * g.n, D * h.nw, masked);
+    if (masked)
+    {
+        const dim3 grid(sx_grid(cap, D, 64), (unsigned) (D < 32768 ? D : 32768));
+        k_sx_push_mask<<<grid, PU_NT, 0, st>>>(g, h);
+    }
+    k_sx_push<S><<<sx_grid(items, 1, cap), PU_NT, 0, st>>>(g, h);
+    k_sx_push_count<S><<<sx_grid(D * h.nseg, 1, cap * 2), PU_NT, 0, st>>>(g, h);
+    GM_TRY(scan_exclusive_i64(h.seg, h.seg, D * h.nseg));
+    k_sx_push_rows<<<sx_grid(D, PU_NT, cap), PU_NT, 0, st>>>(g, h);
+    GM_HIP(hipGetLastError(), "sx_push");
+    return GM_SUCCESS;
+}
+
+template <class S>
+static int sx_push_write(SxArgs &g, SxPush &p)
+{
+    ProfScope ps("sx_push_write");
+    k_sx_push_write<S><<<sx_grid(p.h.D * p.h.nseg, 1, (int64_t) cu_count() * 16), PU_NT, 0, stream()>>>(g, p.h);
+    return check_hip(hipGetLastError(), "k_sx_push_write");
+}
+
+// flop count, binning and the dealing out of the heavy rows; hc receives the
+// counters
+static int sx_count(SxArgs &g, int64_t fs, int list_small, int64_t dmax, int64_t *dflops, int64_t *hc,
+                    unsigned long long *hp)
+{
+    hipStream_t st = stream();
+    DevBuf rowf;
+    {
+        ProfScope ps("sx_flops");
+        if (g.m <= FEW_ROWS)
+        {
+            // a few rows may be very long: each one over many workgroups
+            if (!rowf.alloc(sizeof(unsigned long long) * g.m)) return set_error(GM_OUT_OF_MEMORY, "saxpy3: flops");
+            k_sx_zero<<<1, FEW_ROWS, 0, st>>>(rowf.as<unsigned long long>(), (int) g.m);
+            const dim3 grid((unsigned) ((cu_count() * 4 + g.m - 1) / g.m), (unsigned) g.m);
+            k_sx_rowflops<<<grid, PU_NT, 0, st>>>(g, rowf.as<unsigned long long>());
+            g.rowf = rowf.as<unsigned long long>();
+        }
+        k_sx_flops<<<sx_grid(g.m, SX_NT / TG, (int64_t) cu_count() * 16), SX_NT, 0, st>>>(g, fs, list_small);
+        g.rowf = nullptr;
+        k_sx_classify<<<sx_grid(g.m, SX_NT, (int64_t) cu_count()), SX_NT, 0, st>>>(g, dflops, dmax);
+        GM_HIP(hipGetLastError(), "k_sx_flops");
+    }
+    GM_HIP(hipMemcpyAsync(hp, g.cnt, 16 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st), "bin counts");
+    GM_HIP(hipStreamSynchronize(st), "bin counts sync");
+    for (int t = 0; t < 16; t++) hc[t] = (int64_t) hp[t];
+    if (hc[BIN_DNS] > dmax) hc[BIN_DNS] = dmax;
+    return GM_SUCCESS;
+}
+
 // pattern-only instance used by the symbolic phase of every semiring
 using SxSym = SR<GM_ADD_ANY, GM_MULT_PAIR, uint8_t>;
 
@@ -1264,10 +1443,8 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     const size_t zs = sizeof(Z);
     const size_t entry_bytes = sizeof(int64_t) + (S::iso_out ? 0 : zs);
 
-    DevBuf Cp, rows, cnt, goff, glog;
-    if (!Cp.alloc(sizeof(int64_t) * (m + 1)) || !rows.alloc(sizeof(uint32_t) * SX_NBINS * (m > 0 ? m : 1)) ||
-        !cnt.alloc(sizeof(unsigned long long) * 16) || !goff.alloc(sizeof(int64_t) * (m > 0 ? m : 1)) ||
-        !glog.alloc(sizeof(int32_t) * (m > 0 ? m : 1)))
+    DevBuf Cp, cnt, lists;
+    if (!Cp.alloc(sizeof(int64_t) * (m + 1)) || !cnt.alloc(sizeof(unsigned long long) * SX_NCNT))
         return set_error(GM_OUT_OF_MEMORY, "saxpy3: workspace");
 
     SxArgs g;
@@ -1281,8 +1458,9 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     g.mask_struct = (mask_struct || !M || !M->x) ? 1 : 0;
     g.mode = !M ? MODE_NONE : (mask_comp ? MODE_NOTMASK : MODE_MASK);
     g.Cp = Cp.as<int64_t>(); g.Ci = nullptr; g.Cx = nullptr;
-    g.rows = rows.as<uint32_t>(); g.cnt = cnt.as<unsigned long long>();
-    g.gtab_off = goff.as<int64_t>(); g.gtab_log2 = glog.as<int32_t>();
+    g.rows = nullptr; g.cnt = cnt.as<unsigned long long>();
+    g.hflops = nullptr; g.rowf = nullptr;
+    g.gtab_off = nullptr; g.gtab_log2 = nullptr;
     g.gkeys = nullptr; g.gvals = nullptr; g.glist = nullptr;
     g.Bjx = nullptr;
     g.rec_lg = -1;
@@ -1301,8 +1479,12 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     // scan; it is used while that bound stays within a third of HBM
     const double budget = (double) device_hbm_bytes() / 3.0;
 
-    int64_t hc[16] = {0};
-    unsigned long long *hp = (unsigned long long *) pinned_scratch(16 * sizeof(unsigned long long));
+    // dense rows at most: their tables within 1/32 of HBM
+    int64_t dmax = 0;
+    if (SX_ANY_ORDER<S> && B->nrows < (int64_t) 0xffffffff)
+        dmax = (int64_t) ((double) device_hbm_bytes() / 32.0 / (sx_push_row_bytes<S>(n, M != nullptr) + 1.0));
+    int64_t hc[SX_NCNT] = {0};
+    unsigned long long *hp = (unsigned long long *) pinned_scratch(SX_NCNT * sizeof(unsigned long long));
     if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
     if (m == 0)
     {
@@ -1324,7 +1506,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     // together with its synchronisation.
     int64_t maxA = 0, maxB = 0, nnzA = 0, nnzB = -1;
     const bool probe_small = m * 8 >= B->nrows;
-    k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, 16);
+    k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
     GM_HIP(hipGetLastError(), "k_sx_fill_u64");
     if (probe_small)
     {
@@ -1332,17 +1514,17 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             ProfScope ps("sx_maxlen");
             const int64_t lim = m > B->nrows ? m : B->nrows;
             k_sx_maxlen<<<sx_grid((lim + 3) / 4, SX_NT, (int64_t) cu_count() * 8), SX_NT, 0, st>>>(
-                A->p, m, B->p, B->nrows, g.cnt + 8);
+                A->p, m, B->p, B->nrows, g.cnt + CNT_MAXLEN);
             GM_HIP(hipGetLastError(), "k_sx_maxlen");
         }
-        // counters 8..13: max |A(i,:)|, max |B(k,:)|, nnz(A), -, -, nnz(B)
-        GM_HIP(hipMemcpyAsync(hp + 8, g.cnt + 8, 6 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
+        // max |A(i,:)|, max |B(k,:)|, nnz(A), -, -, nnz(B)
+        GM_HIP(hipMemcpyAsync(hp, g.cnt + CNT_MAXLEN, 6 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
                "maxlen d2h");
         GM_HIP(hipStreamSynchronize(st), "maxlen sync");
-        maxA = (int64_t) hp[8];
-        maxB = (int64_t) hp[9];
-        nnzA = (int64_t) hp[10];
-        nnzB = (int64_t) hp[13];
+        maxA = (int64_t) hp[0];
+        maxB = (int64_t) hp[1];
+        nnzA = (int64_t) hp[2];
+        nnzB = (int64_t) hp[5];
     }
 
     bool fused = (mode != 2);
@@ -1351,36 +1533,31 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     int64_t cap_small = all_small ? nnzA * maxB : 0;
 
     // 2. flop count and binning (skipped when every row is small)
+    int64_t *dflops = nullptr;
     if (!all_small)
     {
-        {
-            ProfScope ps("sx_flops");
-            k_sx_flops<<<sx_grid(m, SX_NT / TG, (int64_t) cu_count() * 16), SX_NT, 0, st>>>(
-                g, fs, fused ? 0 : 1);
-            GM_HIP(hipGetLastError(), "k_sx_flops");
-        }
-        GM_HIP(hipMemcpyAsync(hp, g.cnt, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
-               "bin counts");
-        GM_HIP(hipStreamSynchronize(st), "bin counts sync");
-        for (int t = 0; t < 8; t++) hc[t] = (int64_t) hp[t];
-        cap_small = hc[7];
+        // the bins' row lists and the heavy rows' records, in one block
+        if (!lists.alloc((size_t) m * (3 * sizeof(int64_t) + (SX_NBINS + 1) * sizeof(uint32_t))))
+            return set_error(GM_OUT_OF_MEMORY, "saxpy3: row lists");
+        g.gtab_off = lists.as<int64_t>();
+        g.hflops = g.gtab_off + m;
+        dflops = g.hflops + m;
+        g.rows = (uint32_t *) (dflops + m);
+        g.gtab_log2 = (int32_t *) (g.rows + SX_NBINS * m);
+        GM_TRY(sx_count(g, fs, fused ? 0 : 1, dmax, dflops, hc, hp));
+        cap_small = hc[CNT_SMALL];
         if (fused && (double) cap_small * (double) entry_bytes > budget)
         {
             // too large to hold at the flop bound: redo the binning with the
             // small rows listed for the symbolic + numeric path
             fused = false;
-            k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, 16);
-            k_sx_flops<<<sx_grid(m, SX_NT / TG, (int64_t) cu_count() * 16), SX_NT, 0, st>>>(g, fs, 1);
-            GM_HIP(hipGetLastError(), "k_sx_flops");
-            GM_HIP(hipMemcpyAsync(hp, g.cnt, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
-                   "bin counts");
-            GM_HIP(hipStreamSynchronize(st), "bin counts sync");
-            for (int t = 0; t < 8; t++) hc[t] = (int64_t) hp[t];
+            k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
+            GM_TRY(sx_count(g, fs, 1, dmax, dflops, hc, hp));
         }
     }
 
     DevBuf gkeys, gvals, glist;
-    const int64_t gslots = hc[SX_NBINS];
+    const int64_t gslots = hc[CNT_SLOTS];
     if (gslots > 0)
     {
         if (!gkeys.alloc(sizeof(uint32_t) * gslots) || !gvals.alloc(zs * gslots) ||
@@ -1389,7 +1566,13 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
                              (long long) gslots);
         g.gkeys = gkeys.as<uint32_t>(); g.gvals = gvals.ptr; g.glist = glist.as<uint64_t>();
     }
-    const bool have_big = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB] > 0;
+    const int64_t nbig = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB] + hc[BIN_DNS];
+    const bool have_big = nbig > 0;
+    SxPush push;
+    memset(&push.h, 0, sizeof(push.h));
+    push.h.dflops = dflops;
+    if constexpr (SX_ANY_ORDER<S>)
+        if (hc[BIN_DNS] > 0) GM_TRY(sx_push_build<S>(g, push, hc[BIN_DNS], hc[CNT_NNZA], hc[CNT_HFLOPS]));
     int64_t nvals = 0;
     DevBuf Ci, Cx;
     if (fused)
@@ -1399,13 +1582,12 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         if (have_big)
         {
             GM_TRY((sx_launch_phase<SxSym, 0>(g, hc, true)));
-            const int64_t nbig = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB];
-            k_sx_sum_big<<<sx_grid(nbig, SX_NT, 512), SX_NT, 0, st>>>(g);
+            k_sx_sum_big<<<sx_grid(nbig, SX_NT, 512), SX_NT, 0, st>>>(g, dmax);
             GM_HIP(hipGetLastError(), "k_sx_sum_big");
-            GM_HIP(hipMemcpyAsync(hp + 6, g.cnt + 6, sizeof(unsigned long long),
+            GM_HIP(hipMemcpyAsync(hp, g.cnt + CNT_BIGSUM, sizeof(unsigned long long),
                                   hipMemcpyDeviceToHost, st), "big total");
             GM_HIP(hipStreamSynchronize(st), "big total sync");
-            big_total = (int64_t) hp[6];
+            big_total = (int64_t) hp[0];
         }
         const int64_t cap = cap_small + big_total;
         if (!Ci.alloc(sizeof(int64_t) * (cap > 0 ? cap : 1)) ||
@@ -1415,12 +1597,12 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         g.Cx = Cx.ptr;
         // 4. fused small-row kernel with the look-back scan over all rows
         const int64_t ntiles = (m + FUSED_ROWS - 1) / FUSED_ROWS;
-        DevBuf status, errf;
-        if (!status.alloc(sizeof(unsigned long long) * (ntiles + 1)) || !errf.alloc(sizeof(int)))
+        DevBuf status;
+        if (!status.alloc(sizeof(unsigned long long) * (ntiles + 1)))
             return set_error(GM_OUT_OF_MEMORY, "saxpy3: scan status");
         k_sx_fill_u64<<<sx_grid(ntiles + 1, 256, 1024), 256, 0, st>>>(
             status.as<unsigned long long>(), ntiles + 1);
-        k_sx_fill_u64<<<1, 64, 0, st>>>((unsigned long long *) g.cnt + 12, 1);
+        k_sx_fill_u64<<<1, 64, 0, st>>>((unsigned long long *) g.cnt + CNT_ERR, 1);
         GM_HIP(hipGetLastError(), "k_sx_fill_u64");
         // B's rows: from its row records when the operand carries them (one
         // aligned run per gathered row, no row pointers); else as 16-byte
@@ -1453,7 +1635,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             const int64_t gcap = (int64_t) cu_count() * 8 * 256 / FUSED_NT;
             const int64_t grid = ntiles < gcap ? ntiles : gcap;
             unsigned long long *stp = status.as<unsigned long long>();
-            int *errp = (int *) (g.cnt + 12);
+            int *errp = (int *) (g.cnt + CNT_ERR);
             const bool k32 = B->ncols <= ((int64_t) 1 << 26);
 #define GM_SX_FUSED(K, PKV) \
     k_sx_fused<S, K, FUSED_NT, PKV><<<(unsigned) grid, FUSED_NT, 0, st>>>(g, fs, stp, ntiles, errp)
@@ -1470,13 +1652,15 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             GM_HIP(hipGetLastError(), "k_sx_fused");
         }
         GM_HIP(hipMemcpyAsync(hp + 11, g.Cp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
-        GM_HIP(hipMemcpyAsync(hp + 12, g.cnt + 12, sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
+        GM_HIP(hipMemcpyAsync(hp + 12, g.cnt + CNT_ERR, sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
                "fused err");
         GM_HIP(hipStreamSynchronize(st), "fused sync");
         if (hp[12] != 0) return set_error(GM_PANIC, "saxpy3: look-back scan did not complete");
         nvals = (int64_t) hp[11];
         // 5. numeric phase of the big rows
         if (have_big && nvals > 0) GM_TRY((sx_launch_phase<S, 1>(g, hc, true)));
+        if constexpr (SX_ANY_ORDER<S>)
+            if (hc[BIN_DNS] > 0 && nvals > 0) GM_TRY(sx_push_write<S>(g, push));
     }
     else
     {
@@ -1492,6 +1676,8 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         g.Ci = Ci.as<int64_t>();
         g.Cx = Cx.ptr;
         if (nvals > 0) GM_TRY((sx_launch_phase<S, 1>(g, hc, false)));
+        if constexpr (SX_ANY_ORDER<S>)
+            if (hc[BIN_DNS] > 0 && nvals > 0) GM_TRY(sx_push_write<S>(g, push));
     }
     if (S::iso_out)
     {

@@ -275,3 +275,38 @@ def test_saxpy3_method_hints_grb_mxm(grb, axb):
     finally:
         d.free()
     assert_csr_equal(C.to_csr(), O.saxpy3("plus_times_fp64", A, B), fp_tol=FP_TOL, what=axb)
+
+
+@pytest.mark.parametrize("mask", ["none", "M", "!M"])
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("ncols", [1, 31, 2047, 2049, 5000])
+@pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GxB_PLUS_PAIR_INT32", "GxB_ANY_PAIR_BOOL",
+                                    "GxB_ANY_SECONDI_INT64", "GrB_PLUS_TIMES_SEMIRING_INT64",
+                                    "GrB_MIN_PLUS_SEMIRING_INT32", "GrB_MAX_PLUS_SEMIRING_INT32",
+                                    "GrB_MIN_PLUS_SEMIRING_FP64", "GrB_PLUS_TIMES_SEMIRING_FP64"])
+def test_saxpy3_spread_rows(grb, mask, mode, ncols, handle):
+    """Rows whose products are spread over the device: few long rows of A
+    (more than one LDS window of entries and more than one chunk of products),
+    empty rows of B inside them, columns on both sides of a segment's end,
+    values that cancel or equal the monoid's identity."""
+    print(f"[saxpy3] spread {handle} n={ncols} mode={mode} mask={mask}", flush=True)
+    rng = np.random.default_rng(ncols + 7 * mode + len(mask))
+    vt = _vals(handle)
+    K = 900
+    A = rand_csr(5, K, 0.6, rng, vt)
+    B = rand_csr(K, ncols, min(0.9, 30.0 / ncols), rng, vt, empty_rows=0.3)
+    if vt == "int64" and B.nnz:
+        B.x[::3] = 0
+    if vt == "int32" and B.nnz:
+        B.x[::5] = np.iinfo(np.int32).max if "MIN" in handle else np.iinfo(np.int32).min
+        A.x[:] = 0
+    if handle == "GrB_MIN_PLUS_SEMIRING_FP64" and B.nnz:
+        B.x[::4] = np.inf
+        B.x[1::4] *= -1.0
+    M = rand_csr(5, ncols, 0.4, rng, "int64") if mask != "none" else None
+    name, _ = SR[handle]
+    kw = {} if M is None else {"M": M, "mask_comp": mask == "!M", "mask_struct": False}
+    ref = O.saxpy3(name, A, B, **kw)
+    got = gm_saxpy3(handle, A, B, params=(8, 16, 32, mode), **kw)
+    tol = FP_TOL if handle == "GrB_PLUS_TIMES_SEMIRING_FP64" else None
+    assert_csr_equal(got, ref, fp_tol=tol, what=f"spread {handle}")
