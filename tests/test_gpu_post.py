@@ -224,3 +224,35 @@ def test_grb_mxm_axb_dot_hint(grb):
     assert rc == 0, capi.last_error()
     ref = O.saxpy3("plus_times_int64", A, B, M=M)
     assert_csr_equal(C.to_csr(), ref, what="axb dot")
+
+
+@pytest.mark.parametrize("mask", ["none", "M", "!M"])
+@pytest.mark.parametrize("nc,nt", [(0, 2048), (2047, 1), (2048, 2049), (4096, 0), (5000, 7000)])
+@pytest.mark.parametrize("rows", [1, 3])
+def test_accum_mask_long_rows(grb, rows, nc, nt, mask):
+    """Rows that span several tiles of entries, tiles that end with a row or
+    inside it, and an operand without entries."""
+    print(f"[post] accum rows={rows} nc={nc} nt={nt} mask={mask}", flush=True)
+    rng = np.random.default_rng(nc + nt + rows)
+    n = 12000
+
+    def long_rows(nnz):
+        key = np.sort(rng.choice(rows * n, size=nnz, replace=False))
+        p = np.searchsorted(key // n, np.arange(rows + 1)).astype(np.int64)
+        return W.Csr(rows, n, p, (key % n).astype(np.int64), rng.integers(-9, 9, nnz).astype(np.int64))
+    C, T = long_rows(nc), long_rows(nt)
+    M = long_rows(6000) if mask != "none" else None
+    for op, replace in ((1, False), (0, False), (0, True), (2, True)):
+        ref = O.accum_mask(C, M, T, mask_comp=mask == "!M", mask_struct=False, replace=replace, op=op,
+                           dtype=np.int64)
+        dC, dT = DevCsr(C, 8), DevCsr(T, 8)
+        dM = DevCsr(M, 8) if M is not None else None
+        out = capi.GmCsrOut()
+        rc = capi.lib().gm_accum_mask(ctypes.byref(out), ctypes.byref(dC.view),
+                                      ctypes.byref(dM.view) if dM else None, mask == "!M", False, replace,
+                                      ctypes.byref(dT.view), op)
+        assert rc == 0, capi.last_error()
+        assert_csr_equal(download(out, np.int64), ref, what=f"op={op} replace={replace}")
+        for d in (dC, dT, dM):
+            if d:
+                d.free()
