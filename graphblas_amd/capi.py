@@ -325,6 +325,9 @@ def lib():
         "gm_transpose": ([ctypes.POINTER(GmCsrOut), ctypes.POINTER(GmCsr)], ctypes.c_int),
         "gm_flopcount": ([ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(GmCsr), ctypes.POINTER(GmCsr)],
                          ctypes.c_int),
+        "gm_vxm_bt": ([ctypes.POINTER(GmCsrOut), ctypes.POINTER(GmCsr), ctypes.c_bool,
+                       ctypes.POINTER(GmCsr), ctypes.POINTER(GmCsr), I64,
+                       ctypes.POINTER(GmSemiring)], ctypes.c_int),
         "gm_nonempty_rows": ([ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(GmCsr)], ctypes.c_int),
         "gm_dot2": ([ctypes.POINTER(GmCsrOut), ctypes.POINTER(GmCsr), ctypes.c_bool, ctypes.c_bool,
                      ctypes.POINTER(GmCsr), ctypes.POINTER(GmCsr), ctypes.POINTER(GmSemiring),

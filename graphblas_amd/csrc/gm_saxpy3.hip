@@ -223,6 +223,7 @@ __device__ __forceinline__ void sx_ordered_upd(typename S::Z *vals, int32_t slot
 } // namespace gm
 
 #include "gm_sx_push.h"
+#include "gm_sx_pull.h"
 
 namespace gm
 {
@@ -1695,9 +1696,116 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     return GM_SUCCESS;
 }
 
+// C = A*B' or C<!M> = A*B' for a one-row A (gm_sx_pull.h)
+template <class S>
+static int vxm_bt_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_csr *A, const gm_csr *B,
+                      int64_t nnz)
+{
+    using Z = typename S::Z;
+    hipStream_t st = stream();
+    const int64_t n = B->nrows, k = A->ncols, cap = (int64_t) cu_count() * 8;
+    const int64_t nw = (n + 31) >> 5, kw = (k + 31) >> 5;
+    SxArgs g;
+    memset(&g, 0, sizeof(g));
+    g.m = 1; g.n = n;
+    g.Ap = A->p; g.Aj = A->j; g.Ax = A->x; g.a_iso = A->iso;
+    g.Bp = B->p; g.Bj = B->j; g.Bx = B->x; g.b_iso = B->iso;
+    if (M)
+    {
+        g.Mp = M->p; g.Mj = M->j; g.Mx = mask_struct ? nullptr : M->x;
+        g.msize = (int32_t) type_size(M->type); g.m_iso = M->iso;
+        g.mask_struct = (mask_struct || !M->x) ? 1 : 0;
+        g.mode = MODE_NOTMASK;
+    }
+    PushArgs h;
+    PullArgs p;
+    memset(&h, 0, sizeof(h));
+    memset(&p, 0, sizeof(p));
+    p.nnz = nnz;
+    p.nch = (nnz + PL_CH - 1) / PL_CH;
+    h.D = 1; h.nw = nw; h.all_bits = 1;
+    h.nseg = (n + PU_SEG - 1) / PU_SEG;
+    // cleared words: the row id, A's bits, the mask's, the result's bits or
+    // its 32-bit cells
+    const int64_t words = 2 + kw + (M ? nw : 0) + (PU_U32<S> ? n : nw);
+    DevBuf Cp, Ci, Cx, zero, val, tab, part, seg;
+    if (!Cp.alloc(2 * sizeof(int64_t)) || !Ci.alloc(sizeof(int64_t) * n) ||
+        !Cx.alloc(S::iso_out ? sizeof(Z) : sizeof(Z) * n) || !zero.alloc(sizeof(uint32_t) * (words + 1)) ||
+        (!S::pattern && !val.alloc(sizeof(Z) * k)) || (!PU_U32<S> && !S::iso_out && !tab.alloc(sizeof(Z) * n)) ||
+        !part.alloc((size_t) p.nch * (2 * sizeof(Z) + sizeof(int64_t) + 2) + 8) ||
+        !seg.alloc(sizeof(int64_t) * (h.nseg + 1)))
+        return set_error(GM_OUT_OF_MEMORY, "one-row product: workspace");
+    g.Cp = Cp.as<int64_t>(); g.Ci = Ci.as<int64_t>(); g.Cx = Cx.ptr;
+    uint32_t *w = zero.as<uint32_t>();
+    h.drow = w;
+    p.ubits = w + 2;
+    h.mbits = p.ubits + kw;
+    h.bits = h.mbits + (M ? nw : 0);
+    h.tab = PU_U32<S> ? (void *) h.bits : tab.ptr;
+    h.seg = seg.as<int64_t>();
+    p.uval = val.ptr;
+    p.lrow = part.as<int64_t>();
+    p.pz = p.lrow + p.nch;
+    p.pe = (uint8_t *) p.pz + 2 * sizeof(Z) * p.nch;
+    int64_t *hp = (int64_t *) pinned_scratch(sizeof(int64_t));
+    if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
+    {
+        ProfScope ps("sx_pull");
+        const int64_t zw = (words + 1) / 2;
+        k_sx_fill_u64<<<sx_grid(zw, 256, cap), 256, 0, st>>>(zero.as<unsigned long long>(), zw);
+        k_pull_scatter<S><<<sx_grid(k, PL_NT, cap), PL_NT, 0, st>>>(g, p);
+        if (M) k_sx_push_mask<<<dim3((unsigned) cu_count(), 1), PU_NT, 0, st>>>(g, h);
+        if (p.nch > 0)
+        {
+            k_pull<S><<<sx_grid(p.nch, 1, cap), PL_NT, 0, st>>>(g, h, p);
+            k_pull_fix<S><<<sx_grid(p.nch, PL_NT / 64, cap), PL_NT, 0, st>>>(g, h, p);
+        }
+        k_sx_push_count<S><<<sx_grid(h.nseg, 1, cap), PU_NT, 0, st>>>(g, h);
+        GM_TRY(scan_exclusive_i64(h.seg, h.seg, h.nseg));
+        k_pull_ptr<<<1, 64, 0, st>>>(g.Cp, h.seg, h.nseg);
+        k_sx_push_write<S><<<sx_grid(h.nseg, 1, cap), PU_NT, 0, st>>>(g, h);
+        if (S::iso_out) k_sx_iso_one<<<1, 1, 0, st>>>(Cx.ptr, (int) sizeof(Z));
+        GM_HIP(hipGetLastError(), "one-row product");
+    }
+    GM_HIP(hipMemcpyAsync(hp, g.Cp + 1, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
+    GM_HIP(hipStreamSynchronize(st), "one-row product sync");
+    C->nrows = 1;
+    C->ncols = n;
+    C->nvals = hp[0];
+    C->p = (int64_t *) Cp.release();
+    C->j = (int64_t *) Ci.release();
+    C->x = Cx.release();
+    C->iso = S::iso_out ? 1 : 0;
+    return GM_SUCCESS;
+}
+
 } // namespace gm
 
 using namespace gm;
+
+extern "C" int gm_vxm_bt(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_csr *A, const gm_csr *B,
+                         int64_t nnz_b, const gm_semiring *sr)
+{
+    if (!C || !A || !B || !sr) return set_error(GM_INVALID_VALUE, "gm_vxm_bt: NULL argument");
+    if (!semiring_supported(sr) || !operand_ok(sr, A) || !operand_ok(sr, B))
+        return set_error(GM_NO_VALUE, "gm_vxm_bt: case not handled by the GPU kernels");
+    // cells and counts are 32-bit; the dense vector is as long as the inner index
+    if (A->nrows != 1 || A->ncols != B->ncols || nnz_b < 0 || B->nrows < 1 || A->ncols < 1 ||
+        A->ncols >= (int64_t) 0xffffffff || B->nrows >= (int64_t) 0x7fffffff ||
+        (M && (M->nrows != 1 || M->ncols != B->nrows)))
+        return set_error(GM_NO_VALUE, "gm_vxm_bt: shape not handled");
+    GM_TRY(ensure_init());
+#define GM_VBT_CASE(ADD, MULT, ZC, Z)                                             \
+    if (sr->add_op == ADD && sr->mult_op == MULT && sr->ztype == ZC)              \
+    {                                                                             \
+        int rc = vxm_bt_run<SR<ADD, MULT, Z>>(C, M, mask_struct, A, B, nnz_b);    \
+        if (rc == GM_SUCCESS) C->type = ZC;                                       \
+        return rc;                                                                \
+    }
+    GM_SEMIRING_LIST(GM_VBT_CASE)
+#undef GM_VBT_CASE
+    return set_error(GM_NO_VALUE, "gm_vxm_bt: semiring not instantiated");
+}
 
 //------------------------------------------------------------------------------
 // total multiplies of C=A*B: the sum over A's entries (i,k) of |B(k,:)|.

@@ -57,6 +57,7 @@ struct PushArgs
     int64_t *it_e;                     //           its first product's A entry
     void *tab;                         // D x n cells
     uint32_t *bits, *mbits;            // D x nw presence / mask bits
+    int32_t all_bits;                  // every present cell has its bit (absent cells hold anything)
     int64_t nseg;
     int64_t *seg;                      // D x nseg + 1: scanned segment counts
 };
@@ -280,7 +281,7 @@ __device__ __forceinline__ bool pu_present(const PushArgs &h, int64_t n, int64_t
         else
         {
             z = ((const Z *) h.tab)[d * n + j];
-            return bit || (S::add != GM_ADD_PLUS && z != S::identity());
+            return bit || (S::add != GM_ADD_PLUS && !h.all_bits && z != S::identity());
         }
     }
 }

@@ -292,7 +292,14 @@ GrB_Info GrB_mxm(GrB_Matrix C, const GrB_Matrix Mask, const GrB_BinaryOp accum,
             }
         }
     }
-    if (method == GB_METHOD_SAXPY3 && (!Mask || mask_comp) && (b_tran || axb == GxB_AxB_DOT) &&
+    // a one-row A times B' reads B as it is held.  An ANY monoid with a
+    // positional multiplier asks the dot2 rule first: its witness k depends on
+    // the method (see above)
+    const bool any_k = sr.add_op == GM_ADD_ANY && sr.mult_op == GM_MULT_K;
+    const bool pull_ok = method == GB_METHOD_SAXPY3 && b_tran && va.nrows == 1 && axb == GxB_DEFAULT &&
+                         (!Mask || mask_comp);
+    bool pulled = false;
+    if (!(pull_ok && !any_k) && method == GB_METHOD_SAXPY3 && (!Mask || mask_comp) && (b_tran || axb == GxB_AxB_DOT) &&
         (axb == GxB_DEFAULT || axb == GxB_AxB_DOT))
     {
         // C = A*B' or C<!M> = A*B': every dot product of a small, dense
@@ -318,6 +325,20 @@ GrB_Info GrB_mxm(GrB_Matrix C, const GrB_Matrix Mask, const GrB_BinaryOp accum,
             method = GB_METHOD_DOT2;
         }
     }
+    if (pull_ok && method == GB_METHOD_SAXPY3)
+    {
+        rc = gm_vxm_bt(&R, Mask ? &vm : NULL, mstruct, &va, &vb, B->nvals, &sr);
+        pulled = (rc == GM_SUCCESS);
+        if (pulled && GB_burble)
+            printf("burble: GrB_mxm C%s=A*B' %s: one row, B as held (%lld entries)\n", Mask ? "<!M>" : "",
+                   GB_sr_name(&sr, nm, sizeof(nm)), (long long) B->nvals);
+        if (rc != GM_SUCCESS && rc != GM_NO_VALUE)
+        {
+            GB_free_out(&AT);
+            return GB_error(C, GB_from_gm(rc), "GrB_mxm: %s", gm_last_error());
+        }
+        rc = GM_SUCCESS;
+    }
     if (method == GB_METHOD_DOT3 && (Mask->nvals >= ((int64_t) 1 << 32) || Mask->nrows >= ((int64_t) 1 << 32)))
     {
         // the dot3 kernels number mask entries and rows with 32 bits: a larger
@@ -328,7 +349,7 @@ GrB_Info GrB_mxm(GrB_Matrix C, const GrB_Matrix Mask, const GrB_BinaryOp accum,
                    (long long) Mask->nvals);
         method = GB_METHOD_SAXPY3;
     }
-    if (b_tran != (method == GB_METHOD_DOT3 || method == GB_METHOD_DOT2))
+    if (!pulled && b_tran != (method == GB_METHOD_DOT3 || method == GB_METHOD_DOT2))
     {
         // saxpy3 needs B by rows, dot3 needs the rows of B' (B's columns)
         if (GB_burble) printf("burble: GrB_mxm: transpose B (%lld entries)\n", (long long) B->nvals);
@@ -340,7 +361,8 @@ GrB_Info GrB_mxm(GrB_Matrix C, const GrB_Matrix Mask, const GrB_BinaryOp accum,
         }
         vb = GB_view_of(&BT);
     }
-    if (method == GB_METHOD_DOT3)
+    if (pulled) { }
+    else if (method == GB_METHOD_DOT3)
     {
         if (GB_burble)
             printf("burble: GrB_mxm C<%sM>=A*B' %s: dot3 (masked dot product), M nnz %lld\n",

@@ -344,6 +344,15 @@ int gm_saxpy3(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_struct,
               const gm_csr *A, const gm_csr *B, const gm_semiring *sr,
               const gm_saxpy3_params *params);
 
+// C = A*B', or C<!M> = A*B' when M is given, for an A of one row (a vector) and
+// B by rows with nnz_b entries: the product GrB_mxv runs, without the transpose
+// of B that saxpy3 needs.  The result is saxpy3's (ANY keeps the largest k;
+// fp64 sums are tree sums).  Returns GM_NO_VALUE for a shape it does not take.
+// The reference transposes or uses its dot products here
+// (Source/mxm/GrB_mxv.c, GB_AxB_meta.c).
+int gm_vxm_bt(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_csr *A, const gm_csr *B,
+              int64_t nnz_b, const gm_semiring *sr);
+
 // *flops = multiplies of C=A*B without a mask: the sum over A's entries
 // (i,k) of |B(k,:)| (the total of GB_AxB_saxpy3_flopcount,
 // Source/mxm/GB_AxB_saxpy3_flopcount.c, taken over A's rows).  GrB_mxm uses

@@ -1,12 +1,14 @@
 """GrB_vxm / GrB_mxv (vectors as 1 x n rows on GrB_mxm's kernels) on the GPU
 against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import pyoracle as O
 from graphblas_amd import capi
 from graphblas_amd import workloads as W
-from helpers import assert_csr_equal, rand_csr
+from helpers import SR, ZT, DevCsr, assert_csr_equal, download, rand_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +90,46 @@ def test_vxm_transposed_with_accum_and_mask(grb):
     C0 = _row(w0i, w0x.astype(np.int64), 80)
     ref = O.accum_mask(C0, M, T, op=1, dtype=np.int64)
     assert_csr_equal(_got(w, 80), ref, what="w<m> += u'A'")
+
+
+@pytest.mark.parametrize("comp", [False, True])
+@pytest.mark.parametrize("shape", ["one row", "short", "hub", "chunk"])
+@pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GxB_PLUS_PAIR_INT32", "GxB_ANY_PAIR_BOOL",
+                                    "GxB_ANY_SECONDI_INT64", "GrB_PLUS_TIMES_SEMIRING_INT64",
+                                    "GrB_MIN_PLUS_SEMIRING_INT32", "GrB_MAX_PLUS_SEMIRING_INT32",
+                                    "GrB_MIN_PLUS_SEMIRING_FP64", "GrB_PLUS_TIMES_SEMIRING_FP64"])
+def test_vxm_bt(grb, handle, shape, comp):
+    """u'*B' without a transpose: one row, many short and empty rows, rows that
+    span several chunks of 2048 entries, and rows that end where a chunk ends."""
+    print(f"[vector] vxm_bt {handle} {shape} comp={comp}", flush=True)
+    rng = np.random.default_rng(len(handle) + len(shape))
+    K = 9000
+    lens = {"one row": [4096], "short": rng.integers(0, 9, 3000), "chunk": [2048, 0, 1, 2047, 64, 65, 1919, 2048],
+            "hub": np.where(np.arange(300) % 97 == 5, 8500, rng.integers(0, 40, 300))}[shape]
+    p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    j = np.concatenate([np.sort(rng.choice(K, size=int(l), replace=False)) for l in lens]).astype(np.int64)
+    n, name = len(lens), SR[handle][0]
+    vt = {"INT64": "int64", "INT32": "int32", "FP64": "fp64", "BOOL": "bool"}[handle.split("_")[-1]]
+
+    def vals(k):
+        return (rng.random(k) if vt == "fp64" else rng.integers(1, 100, k)).astype(
+            {"int64": np.int64, "int32": np.int32, "fp64": np.float64, "bool": np.uint8}[vt])
+    B = W.Csr(n, K, p, j, vals(len(j)))
+    ui = np.sort(rng.choice(K, size=K // 2, replace=False)).astype(np.int64)
+    U = _row(ui, vals(len(ui)), K)
+    M = _row(np.arange(0, n, 3), rng.integers(0, 2, len(range(0, n, 3))).astype(np.int64), n) if comp else None
+    code = SR[handle][1][2]
+    dU, dB = DevCsr(U, code), DevCsr(B, code)
+    dM = DevCsr(M, 8) if comp else None
+    out, sr = capi.GmCsrOut(), capi.GmSemiring(*SR[handle][1])
+    rc = capi.lib().gm_vxm_bt(ctypes.byref(out), ctypes.byref(dM.view) if comp else None, False,
+                              ctypes.byref(dU.view), ctypes.byref(dB.view), len(j), ctypes.byref(sr))
+    assert rc == 0, capi.last_error()
+    got = download(out, ZT[vt])
+    kw = {"M": M, "mask_comp": True, "mask_struct": False} if comp else {}
+    ref = O.saxpy3(name, U, O.transpose(B), **kw)
+    # tree sums of at most 8500 positive products against sequential ones
+    assert_csr_equal(got, ref, fp_tol=1e-12 if "PLUS_TIMES_SEMIRING_FP64" in handle else None, what=shape)
+    for d in (dU, dB, dM):
+        if d:
+            d.free()
