@@ -11,18 +11,20 @@
 //   saxpy5  C += A*B, C full, A bitmap/full, B sparse (GB_AxB_saxpy5.c),
 // both "+=" forms with the semiring's monoid as the accumulator and no mask.
 //
-// One kernel covers all three: a workgroup owns row i of C and a tile of
-// DN_TW columns, keeps the tile's accumulators, presence flags and mask in
-// LDS, and applies the row's terms A(i,k) B(k,j) for k ascending (the
-// reference's sequential order, so fp64 sums are bit-identical to it):
-//   B bitmap/full: each thread owns the tile's columns t, t+256, ... and
-//                  reads B(k, those columns) directly, so no two threads
-//                  touch one accumulator and no barrier is needed;
-//   B sparse:      the threads take the entries of B(k,:) inside the tile
-//                  (found by binary search), one barrier per k keeps the
-//                  updates of one column in k order.
+// Two kernels cover all three; both apply a row's terms A(i,k) B(k,j) for k
+// ascending (the reference's sequential order, so fp64 sums are bit-identical
+// to it):
+//   B bitmap/full: a lane owns one column of a row, its accumulator in a
+//                  register; B(k, the team's columns) is one coalesced read
+//                  (k_dn_rows);
+//   B sparse:      a workgroup owns row i and a tile of DN_TW columns with the
+//                  accumulators, presence flags and mask in LDS; the threads
+//                  take the entries of B(k,:) inside the tile (found by binary
+//                  search), one barrier per k keeps the updates of one column
+//                  in k order (k_dn_mxm).
 // ANY keeps the last writer (largest k), as the saxpy3 kernels do.
 
+#include <algorithm>
 #include <cstring>
 #include "gm_internal.h"
 #include "gm_block.h"
@@ -148,8 +150,297 @@ __device__ __forceinline__ void dn_apply(typename S::Z *acc, uint8_t *flag, int 
     else acc[c] = S::upd(acc[c], t);
 }
 
-// ASP / BSP: A / B sparse (else bitmap or full)
-template <class S, bool ASP, bool BSP>
+// a lane's value t of its team of G lanes; t is the same for the team
+template <class T, int G>
+__device__ __forceinline__ T dn_bcast(T v, int t)
+{
+    if constexpr (G == 64 && sizeof(T) == 8)
+    {
+        const uint64_t b = __builtin_bit_cast(uint64_t, v);
+        const uint32_t lo = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) b, t);
+        const uint32_t hi = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) (b >> 32), t);
+        return __builtin_bit_cast(T, ((uint64_t) hi << 32) | lo);
+    }
+    else if constexpr (G == 64 && sizeof(T) == 4)
+        return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), t));
+    else return shfl_any<T>(v, t, G);
+}
+
+// rows of a sparse A with more than DN_HUB entries
+constexpr int64_t DN_HUB = 512;
+
+__global__ __launch_bounds__(DN_NT) void k_dn_hubs(const int64_t *__restrict__ Ap, int64_t m, uint32_t *list,
+                                                   unsigned long long *cnt)
+{
+    for (int64_t i = (int64_t) blockIdx.x * DN_NT + threadIdx.x; i < m; i += (int64_t) gridDim.x * DN_NT)
+        if (Ap[i + 1] - Ap[i] > DN_HUB) list[atomicAdd(cnt, 1ull)] = (uint32_t) i;
+}
+
+// the result of entry (i,c): stored; returns 1 if C holds it
+template <class S>
+__device__ __forceinline__ int dn_put(const DnArgs &g, int64_t i, int64_t c, bool e, typename S::Z z)
+{
+    using Z = typename S::Z;
+    const int64_t d = i * g.n + c;
+    if (g.Cin)
+    {
+        // C full += T with the monoid
+        const Z cin = ((const Z *) g.Cin)[d];
+        ((Z *) g.Cx)[d] = e ? S::upd(cin, z) : cin;
+        return 1;
+    }
+    if (e && g.mkind)
+    {
+        bool in;
+        if (g.mkind == 2) in = (!g.Mb || g.Mb[d] != 0) && (g.mstruct || dn_mask_value(g.Mx, d, g.msize, g.m_iso));
+        else
+        {
+            const int64_t m1 = g.Mp[i + 1], q = lower_bound(g.Mj, g.Mp[i], m1, c);
+            in = q < m1 && g.Mj[q] == c && (g.mstruct || dn_mask_value(g.Mx, q, g.msize, g.m_iso));
+        }
+        e = in != (g.mcomp != 0);
+    }
+    g.Cb[d] = e ? 1 : 0;
+    if constexpr (!S::iso_out) ((Z *) g.Cx)[d] = e ? z : (Z) 0;
+    return e ? 1 : 0;
+}
+
+// B bitmap or full.  A team of G lanes (a power of two, G >= ncols or 64) takes
+// a row and G of its columns.  A row's terms are one serial chain (k
+// ascending), so what counts is how many reads of B's rows are in flight
+// before the first is used: DN_UN per team.  A hub row (DN_HUB entries and
+// more) would still be thousands of such steps, so its entries are taken by
+// the whole workgroup in stages of DN_STG products: while the first G lanes
+// add the stage in LDS, every thread has the next stage's products and the
+// one after's indices on their way.  Hubs go first, so the other rows fill
+// the device beside them.
+// RMAT n = 65536, 1.82M entries, times 64 full columns, fp64: 7.2 ms with a
+// workgroup per row, LDS accumulators and one read in flight; 2.2 ms without
+// the hub stages; 0.75 ms here.  B's rows, 931 MB, come from L2 and the
+// Infinity Cache.
+constexpr int DN_UN = 16;
+constexpr int DN_RT = 1024;                 // threads
+constexpr int DN_SPT = 8;                   // products of a stage per thread
+constexpr int DN_STG = DN_RT * DN_SPT;
+
+template <class S, bool ASP, int G>
+__global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const uint32_t *hubs,
+                                                   const unsigned long long *nhubs, unsigned long long *next)
+{
+    using Z = typename S::Z;
+    const Z *Ax = (const Z *) g.Ax;
+    const Z *Bx = (const Z *) g.Bx;
+    const int lane = threadIdx.x & 63, sub = lane & (G - 1), team = lane / G;
+    unsigned long long cnt = 0;
+    if constexpr (ASP)
+    {
+        constexpr int SE = DN_STG / G;          // entries of a stage
+        __shared__ Z s_t[2][DN_STG];
+        __shared__ uint8_t s_p[2][DN_STG];
+        __shared__ int64_t s_it;
+        const int64_t items = (int64_t) *nhubs * nseg;
+        while (items > 0)
+        {
+            if (threadIdx.x == 0) s_it = (int64_t) atomicAdd(next, 1ull);
+            __syncthreads();
+            const int64_t it = s_it;
+            __syncthreads();
+            if (it >= items) break;
+            const int64_t i = hubs[it / nseg], c0 = (it - it / nseg * nseg) * G;
+            const int64_t q0 = g.Ap[i], q1 = g.Ap[i + 1];
+            const int64_t stages = (q1 - q0 + SE - 1) / SE;
+            // this thread's products of a stage: entries er, er + DN_RT/G, ...,
+            // always of column c0 + sub
+            const int er = (int) threadIdx.x / G;
+            const bool col = c0 + sub < g.n;
+            int64_t k[DN_SPT];
+            Z a[DN_SPT], b[DN_SPT], t[DN_SPT];
+            bool p[DN_SPT];
+            auto entries = [&](int64_t s) {
+                #pragma unroll
+                for (int u = 0; u < DN_SPT; u++)
+                {
+                    const int64_t q = q0 + s * SE + u * (DN_RT / G) + er;
+                    k[u] = q < q1 ? g.Aj[q] : -1;
+                    a[u] = q < q1 ? S::geta(Ax, q, g.a_iso) : Z(0);
+                }
+            };
+            auto rows = [&]() {
+                #pragma unroll
+                for (int u = 0; u < DN_SPT; u++)
+                {
+                    p[u] = k[u] >= 0 && col;
+                    b[u] = Z(0);
+                    t[u] = Z(0);
+                    if (p[u])
+                    {
+                        const int64_t d = k[u] * g.n + c0 + sub;
+                        b[u] = S::geta(Bx, d, g.b_iso);
+                        if (g.Bb) p[u] = g.Bb[d] != 0;
+                    }
+                }
+            };
+            auto stage = [&](int buf) {
+                #pragma unroll
+                for (int u = 0; u < DN_SPT; u++)
+                {
+                    const int at = (u * (DN_RT / G) + er) * G + sub;
+                    s_t[buf][at] = t[u];
+                    s_p[buf][at] = p[u] ? 1 : 0;
+                }
+            };
+            auto products = [&]() {
+                #pragma unroll
+                for (int u = 0; u < DN_SPT; u++)
+                    if (p[u]) t[u] = S::mul(a[u], b[u], k[u]);
+            };
+            bool e = false;
+            Z z = S::identity();
+            entries(0);
+            rows();
+            products();
+            if (stages > 1) entries(1);
+            for (int64_t s = 0; s < stages; s++)
+            {
+                const int buf = (int) (s & 1);
+                stage(buf);
+                __syncthreads();
+                // the next stage's reads go out before this one is added
+                const bool more = s + 1 < stages;
+                if (more) rows();
+                if (threadIdx.x < G)
+                {
+                    const int64_t left = q1 - q0 - s * SE;
+                    const int n = (int) (left < SE ? left : SE);
+                    #pragma unroll 8
+                    for (int x = 0; x < n; x++)
+                    {
+                        const Z v = s_t[buf][x * G + sub];
+                        if (s_p[buf][x * G + sub])
+                        {
+                            z = e ? S::upd(z, v) : v;
+                            e = true;
+                        }
+                    }
+                }
+                if (more)
+                {
+                    products();
+                    if (s + 2 < stages) entries(s + 2);
+                }
+            }
+            if (threadIdx.x < G && col) cnt += (unsigned long long) dn_put<S>(g, i, c0 + sub, e, z);
+            __syncthreads();
+        }
+    }
+    constexpr int TPW = 64 / G, UN = DN_UN;
+    const int64_t nwaves = (int64_t) gridDim.x * (DN_RT / 64);
+    const int64_t items = (g.m + TPW - 1) / TPW * nseg;
+    // neighbouring workgroups take neighbouring rows: a wavefront's next row is nwaves away
+    for (int64_t it = (int64_t) (threadIdx.x >> 6) * gridDim.x + blockIdx.x; it < items; it += nwaves)
+    {
+        const int64_t grp = it / nseg;
+        const int64_t i = grp * TPW + team, c = (it - grp * nseg) * G + sub;
+        const bool own = i < g.m && c < g.n;
+        int64_t q0 = 0, q1 = 0;
+        if (i < g.m)
+        {
+            if constexpr (ASP)
+            {
+                q0 = g.Ap[i];
+                q1 = g.Ap[i + 1];
+                if (q1 - q0 > DN_HUB) continue;           // done above
+            }
+            else q1 = g.kdim;
+        }
+        bool e = false;
+        Z z = S::identity();
+        // G < UN: every lane reads the team's entries itself (one address per
+        // team); else the lanes read G of them and hand them round
+        constexpr int STEP = G < UN ? UN : G;
+        for (int64_t q = q0; q < q1; q += STEP)
+        {
+            const int nb = (int) (q1 - q < STEP ? q1 - q : STEP);
+            int64_t k = 0;
+            Z a = Z(0);
+            int ok = 1;
+            if (G >= UN && sub < nb)
+            {
+                if constexpr (ASP)
+                {
+                    k = g.Aj[q + sub];
+                    a = S::geta(Ax, q + sub, g.a_iso);
+                }
+                else
+                {
+                    k = q + sub;
+                    const int64_t d = i * g.kdim + k;
+                    ok = (!g.Ab || g.Ab[d] != 0) ? 1 : 0;
+                    if (ok) a = S::geta(Ax, d, g.a_iso);
+                }
+            }
+            for (int t0 = 0; t0 < nb; t0 += UN)
+            {
+                // past the entries: the last one's row again, not applied
+                Z av[UN], b[UN];
+                int64_t kv[UN];
+                bool p[UN];
+                #pragma unroll
+                for (int u = 0; u < UN; u++)
+                {
+                    const int t = t0 + u < nb ? t0 + u : nb - 1;
+                    int has = 1;
+                    if constexpr (G >= UN)
+                    {
+                        // by every lane: one outside the columns may hold the entry
+                        kv[u] = dn_bcast<int64_t, G>(k, t);
+                        av[u] = dn_bcast<Z, G>(a, t);
+                        if constexpr (!ASP) has = dn_bcast<int, G>(ok, t);
+                    }
+                    else if constexpr (ASP)
+                    {
+                        kv[u] = g.Aj[q + t];
+                        av[u] = S::geta(Ax, q + t, g.a_iso);
+                    }
+                    else
+                    {
+                        kv[u] = q + t;
+                        const int64_t d = i * g.kdim + kv[u];
+                        has = (!g.Ab || g.Ab[d] != 0) ? 1 : 0;
+                        av[u] = S::geta(Ax, d, g.a_iso);
+                    }
+                    p[u] = own && t0 + u < nb && has != 0;
+                }
+                #pragma unroll
+                for (int u = 0; u < UN; u++)
+                {
+                    b[u] = Z(0);
+                    if (own)
+                    {
+                        const int64_t d = kv[u] * g.n + c;
+                        if (g.Bb) p[u] = p[u] && g.Bb[d] != 0;
+                        b[u] = S::geta(Bx, d, g.b_iso);
+                    }
+                }
+                #pragma unroll
+                for (int u = 0; u < UN; u++)
+                    if (p[u])
+                    {
+                        const Z v = S::mul(av[u], b[u], kv[u]);
+                        z = e ? S::upd(z, v) : v;
+                        e = true;
+                    }
+            }
+        }
+        if (own) cnt += (unsigned long long) dn_put<S>(g, i, c, e, z);
+    }
+    #pragma unroll
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
+    if (lane == 0 && cnt) atomicAdd(g.nvals, cnt);
+}
+
+// B sparse; ASP: A sparse (else bitmap or full)
+template <class S, bool ASP>
 __global__ __launch_bounds__(DN_NT) void k_dn_mxm(DnArgs g)
 {
     using Z = typename S::Z;
@@ -216,18 +507,6 @@ __global__ __launch_bounds__(DN_NT) void k_dn_mxm(DnArgs g)
                 if (g.Ab && g.Ab[d] == 0) continue;          // uniform across the workgroup
                 a = S::geta(Ax, d, g.a_iso);
             }
-            if constexpr (!BSP)
-            {
-                // B(k, tile) by owned columns: no barrier
-                for (int c = threadIdx.x; c < w; c += DN_NT)
-                {
-                    const int64_t d = k * g.n + c0 + c;
-                    if (g.Bb && g.Bb[d] == 0) continue;
-                    if (!s_mask[c]) continue;
-                    dn_apply<S>(s_acc, s_flag, c, S::mul(a, S::geta(Bx, d, g.b_iso), k));
-                }
-            }
-            else
             {
                 const int64_t b0 = g.Bp[k], b1 = g.Bp[k + 1];
                 const int64_t lo = (b0 < b1 && g.Bj[b0] >= c0) ? b0 : lower_bound(g.Bj, b0, b1, c0);
@@ -268,7 +547,7 @@ __global__ __launch_bounds__(DN_NT) void k_dn_mxm(DnArgs g)
     }
 }
 
-__global__ void k_dn_zero_u64(unsigned long long *x) { if (threadIdx.x == 0 && blockIdx.x == 0) *x = 0; }
+__global__ void k_dn_zero_u64(unsigned long long *x, int n) { if ((int) threadIdx.x < n) x[threadIdx.x] = 0; }
 __global__ void k_dn_iso_one(void *x, int size)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0)
@@ -317,24 +596,48 @@ static int dn_mxm_run(gm_dense_out *C, const gm_csr *Ms, const gm_dense *Md, boo
     }
     const int64_t mn = g.m * g.n;
     const bool accum = (Cin != nullptr);
-    DevBuf Cb, Cx, cnt;
+    DevBuf Cb, Cx, cnt, hubs;
     if ((!accum && !Cb.alloc(mn > 0 ? mn : 1)) ||
         !Cx.alloc(S::iso_out && !accum ? sizeof(Z) : sizeof(Z) * (mn > 0 ? mn : 1)) ||
-        !cnt.alloc(sizeof(unsigned long long)))
+        !cnt.alloc(3 * sizeof(unsigned long long)))
         return set_error(GM_OUT_OF_MEMORY, "dense product: output");
     g.Cin = accum ? Cin->x : nullptr;
     g.Cb = accum ? nullptr : Cb.as<int8_t>();
     g.Cx = Cx.ptr;
     g.nvals = cnt.as<unsigned long long>();
-    k_dn_zero_u64<<<1, 64, 0, st>>>(g.nvals);
+    k_dn_zero_u64<<<1, 64, 0, st>>>(g.nvals, 3);
     if (mn > 0)
     {
         const int64_t items = g.m * ((g.n + DN_TW - 1) / DN_TW);
         ProfScope ps(accum ? (As ? "saxpy4" : "saxpy5") : "saxbit");
-        if (As && Bs) k_dn_mxm<S, true, true><<<dn_grid(items), DN_NT, 0, st>>>(g);
-        else if (As) k_dn_mxm<S, true, false><<<dn_grid(items), DN_NT, 0, st>>>(g);
-        else if (Bs) k_dn_mxm<S, false, true><<<dn_grid(items), DN_NT, 0, st>>>(g);
-        else k_dn_mxm<S, false, false><<<dn_grid(items), DN_NT, 0, st>>>(g);
+        if (As && Bs) k_dn_mxm<S, true><<<dn_grid(items), DN_NT, 0, st>>>(g);
+        else if (Bs) k_dn_mxm<S, false><<<dn_grid(items), DN_NT, 0, st>>>(g);
+        else
+        {
+            // the narrowest team that holds the columns, 64 lanes at most
+            int lg = 0;
+            while (lg < 6 && ((int64_t) 1 << lg) < g.n) lg++;
+            const int64_t nseg = (g.n + 63) / 64 > 0 ? (g.n + 63) / 64 : 1;
+            const int64_t teams = g.m * nseg, wgs = (teams + (DN_RT >> lg) - 1) / (DN_RT >> lg);
+            // at least a workgroup per CU while hubs may need one each
+            const unsigned grid = (unsigned) std::max<int64_t>(1, std::min<int64_t>(wgs, (int64_t) cu_count() * 2));
+            unsigned long long *ctr = g.nvals + 1;      // hub count, next hub item
+            if (As)
+            {
+                if (!hubs.alloc(sizeof(uint32_t) * g.m)) return set_error(GM_OUT_OF_MEMORY, "dense product: rows");
+                k_dn_hubs<<<dn_grid((g.m + DN_NT - 1) / DN_NT), DN_NT, 0, st>>>(g.Ap, g.m, hubs.as<uint32_t>(), ctr);
+            }
+#define GM_DN_ROWS(L)                                                                        \
+    case L:                                                                                  \
+        if (As) k_dn_rows<S, true, 1 << L><<<grid, DN_RT, 0, st>>>(g, nseg, hubs.as<uint32_t>(), ctr, ctr + 1); \
+        else k_dn_rows<S, false, 1 << L><<<grid, DN_RT, 0, st>>>(g, nseg, nullptr, ctr, ctr + 1); \
+        break;
+            switch (lg)
+            {
+                GM_DN_ROWS(0) GM_DN_ROWS(1) GM_DN_ROWS(2) GM_DN_ROWS(3) GM_DN_ROWS(4) GM_DN_ROWS(5) GM_DN_ROWS(6)
+            }
+#undef GM_DN_ROWS
+        }
         GM_HIP(hipGetLastError(), "k_dn_mxm");
     }
     if (S::iso_out && !accum)

@@ -217,3 +217,48 @@ def test_saxbit_cabi_errors(grb):
     rc = L.gm_saxbit(ctypes.byref(out), None, None, False, True, ctypes.byref(a), ctypes.byref(d),
                      ctypes.byref(a), None, ctypes.byref(sr), None)
     assert rc == capi.GrB_INVALID_VALUE
+
+
+@pytest.mark.parametrize("fa,fb", [("sparse", "full"), ("sparse", "bitmap"), ("bitmap", "full")])
+@pytest.mark.parametrize("n", [1, 2, 3, 31, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("handle", ["GrB_PLUS_TIMES_SEMIRING_FP64", "GrB_MIN_PLUS_SEMIRING_INT32",
+                                    "GxB_ANY_SECONDI_INT64", "GxB_ANY_PAIR_BOOL"])
+def test_saxbit_widths(grb, handle, n, fa, fb):
+    """Few dense columns: every team width and its remainders, rows without
+    entries, one entry, and more entries than a team reads at a time."""
+    print(f"[dense] saxbit width {n} {handle} A {fa} B {fb}", flush=True)
+    rng = np.random.default_rng(n + len(handle))
+    vt = VT.get(handle)
+    name, _ = SR[handle]
+    tn = TN[vt] if vt else "bool"
+    m, k = 77, 150
+    A = rand_csr(m, k, 0.3, rng, vt, empty_rows=0.2)
+    B = rand_csr(k, n, 1.0 if fb == "full" else 0.6, rng, vt)
+    Ad, Bd = _matrix(A, fa, tn), _matrix(B, fb, tn)
+    C = capi.Matrix(ZT[name], m, n)
+    capi.mxm_checked(C, None, handle, Ad, Bd)
+    ref = O.saxpy3(name, A, B)
+    # terms are added for k ascending: the same bits as the oracle
+    assert_csr_equal(C.to_csr(), ref, what=f"{handle} n={n}")
+
+
+@pytest.mark.parametrize("n", [1, 5, 64, 100])
+@pytest.mark.parametrize("handle", ["GrB_PLUS_TIMES_SEMIRING_FP64", "GrB_MIN_PLUS_SEMIRING_INT32"])
+def test_saxbit_hub_rows(grb, handle, n):
+    """Rows of A on both sides of the hub length and of a stage's end (8192
+    products: 128 entries for 64 columns, 8192 for one)."""
+    print(f"[dense] saxbit hubs {handle} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    vt = VT[handle]
+    name, _ = SR[handle]
+    k = 9000
+    lens = [0, 511, 512, 513, 640, 641, 8192, 8193, 9000, 3]
+    p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    j = np.concatenate([np.sort(rng.choice(k, size=l, replace=False)) for l in lens]).astype(np.int64)
+    x = rng.random(len(j)) if vt == "fp64" else rng.integers(-50, 50, len(j)).astype(np.int32)
+    A = Csr(len(lens), k, p, j, x)
+    for fb in ("full", "bitmap"):
+        B = rand_csr(k, n, 1.0 if fb == "full" else 0.5, rng, vt)
+        C = capi.Matrix(ZT[name], len(lens), n)
+        capi.mxm_checked(C, None, handle, capi.Matrix.from_csr(A, vt), _matrix(B, fb, vt))
+        assert_csr_equal(C.to_csr(), O.saxpy3(name, A, B), what=f"{handle} n={n} {fb}")
