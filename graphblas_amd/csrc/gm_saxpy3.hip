@@ -43,8 +43,10 @@ namespace gm
 constexpr int SX_NT = 256;
 constexpr uint32_t SX_EMPTY = 0xffffffffu;
 // BIN_HVY collects the rows beyond the LDS tables; k_sx_classify deals them out
-// to BIN_GLB (a hash table each) and BIN_DNS (spread over the device)
-enum { BIN_SINGLE = 0, BIN_WS = 1, BIN_WL = 2, BIN_BLK = 3, BIN_GLB = 4, BIN_DNS = 5, BIN_HVY = 6, SX_NBINS = 7 };
+// to BIN_GLB (a hash table each), BIN_DNS (products spread over the device) and
+// BIN_TIL (tiles of columns)
+enum { BIN_SINGLE = 0, BIN_WS = 1, BIN_WL = 2, BIN_BLK = 3, BIN_GLB = 4, BIN_DNS = 5, BIN_HVY = 6, BIN_TIL = 7,
+       SX_NBINS = 8 };
 // counters: the bins, then
 enum { CNT_SLOTS = 8,       // table slots of BIN_GLB
        CNT_BIGSUM = 9,      // entries of the big rows (symbolic)
@@ -52,6 +54,9 @@ enum { CNT_SLOTS = 8,       // table slots of BIN_GLB
        CNT_HFLOPS = 11,     // flops of BIN_HVY
        CNT_NNZA = 12,       // nnz(A)
        CNT_ERR = 13,        // the look-back's error flag
+       CNT_TILF = 14,       // BIN_TIL's very heavy rows (at the list's front; the others from its back)
+       CNT_TILA = 15,       // A's entries in BIN_TIL's rows
+       CNT_TILB = 22,       // BIN_TIL's other rows
        CNT_MAXLEN = 16,     // k_sx_maxlen's six results
        SX_NCNT = 32 };
 enum { MODE_NONE = 0, MODE_MASK = 1, MODE_NOTMASK = 2 };
@@ -224,6 +229,7 @@ __device__ __forceinline__ void sx_ordered_upd(typename S::Z *vals, int32_t slot
 
 #include "gm_sx_push.h"
 #include "gm_sx_pull.h"
+#include "gm_sx_tile.h"
 
 namespace gm
 {
@@ -422,29 +428,50 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
     }
 }
 
-// Deals the heavy rows out.  A row takes a dense table (PUSH: the semiring and
-// the memory allow it, dmax rows at most) when its flops reach a quarter of
-// the columns, so that the table costs less than a hash table's inserts and
-// sort, or when it holds more than 1/512 of all heavy flops, so that one
-// workgroup on it would outlast the others, and at least 1/128 of the columns
-// (the table's clearing and compaction then stay below its updates).  Other
-// rows get a hash table of 2^ceil(log2(2t)) slots, load factor <= 1/2, or a
-// dense one of 2^ceil(log2(ncols)) slots (SxArgs::table).
-__global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops, int64_t dmax)
+// Deals the heavy rows out, by flops f, entries la of A(i,:) and the columns n:
+//   dense table (BIN_DNS; the semiring allows any order, dmax rows at most): a
+//     row with more than 1/512 of all heavy flops, on which one workgroup
+//     would outlast the others, and at least n/128 flops, so that the table's
+//     clearing and compaction stay below its updates
+//   tiles (BIN_TIL, tmax rows at most): la * (n / TL_W) <= 4 f, where finding
+//     the parts of B's rows costs less than a hash table's inserts and sort
+//     (n = 40009: rows whose B rows hold 10 entries or more on average), and
+//     16 flops per tile; a very heavy fp64 row, whose order the dense table
+//     does not keep, up to 64 f
+//   dense table again: at least n/4 flops
+//   else a hash table of 2^ceil(log2(2t)) slots, load factor <= 1/2, or a
+//     dense one of 2^ceil(log2(ncols)) slots (SxArgs::table)
+__global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops, int64_t dmax, int64_t tmax)
 {
     const int64_t count = (int64_t) g.cnt[BIN_HVY];
     const double total = (double) g.cnt[CNT_HFLOPS];
+    const int64_t nt = (g.n + TL_W - 1) / TL_W;
     for (int64_t q = (int64_t) blockIdx.x * SX_NT + threadIdx.x; q < count; q += (int64_t) gridDim.x * SX_NT)
     {
         const uint32_t i = g.rows[(int64_t) BIN_HVY * g.m + q];
-        const int64_t f = g.hflops[q];
-        if (dmax > 0 && g.table != 1 && (f >= g.n / 4 || ((double) f * 512 > total && f >= g.n / 128)))
+        const int64_t f = g.hflops[q], la = g.Ap[i + 1] - g.Ap[i];
+        const bool most = (double) f * 512 > total;
+        const double search = (double) la * (double) nt;
+        const bool push = dmax > 0 && g.table != 1;
+        const bool tile = tmax > 0 && g.table != 1 && f >= 16 * nt &&
+                          (search <= 4.0 * (double) f || (!push && most && search <= 64.0 * (double) f));
+        if (push && ((most && f >= g.n / 128) || (!tile && f >= g.n / 4)))
         {
             const int64_t d = (int64_t) atomicAdd(&g.cnt[BIN_DNS], 1ull);
             if (d < dmax)
             {
                 g.rows[(int64_t) BIN_DNS * g.m + d] = i;
                 dflops[d] = f;
+                continue;
+            }
+        }
+        else if (tile)
+        {
+            if ((int64_t) atomicAdd(&g.cnt[BIN_TIL], 1ull) < tmax)
+            {
+                if (most) g.rows[(int64_t) BIN_TIL * g.m + atomicAdd(&g.cnt[CNT_TILF], 1ull)] = i;
+                else g.rows[(int64_t) (BIN_TIL + 1) * g.m - 1 - atomicAdd(&g.cnt[CNT_TILB], 1ull)] = i;
+                atomicAdd(&g.cnt[CNT_TILA], (unsigned long long) la);
                 continue;
             }
         }
@@ -468,12 +495,14 @@ __global__ __launch_bounds__(SX_NT) void k_sx_sum_big(SxArgs g, int64_t dmax)
 {
     __shared__ unsigned long long s_red[SX_NT / 64];
     unsigned long long sum = 0;
-    const int bins[5] = {BIN_SINGLE, BIN_WL, BIN_BLK, BIN_GLB, BIN_DNS};
-    for (int b = 0; b < 5; b++)
+    // (the tiled rows' two lists: from the front and from the back)
+    const int bins[7] = {BIN_SINGLE, BIN_WL, BIN_BLK, BIN_GLB, BIN_DNS, BIN_TIL, BIN_TIL};
+    for (int b = 0; b < 7; b++)
     {
-        int64_t count = (int64_t) g.cnt[bins[b]];
+        int64_t count = (int64_t) g.cnt[b < 5 ? bins[b] : b == 5 ? CNT_TILF : CNT_TILB];
         if (bins[b] == BIN_DNS && count > dmax) count = dmax;
         const uint32_t *list = g.rows + (int64_t) bins[b] * g.m;
+        if (b == 6) list += g.m - count;
         for (int64_t q = (int64_t) blockIdx.x * SX_NT + threadIdx.x; q < count;
              q += (int64_t) gridDim.x * SX_NT)
             sum += (unsigned long long) g.Cp[list[q]];
@@ -1360,9 +1389,64 @@ static int sx_push_write(SxArgs &g, SxPush &p)
     return check_hip(hipGetLastError(), "k_sx_push_write");
 }
 
+// the tiled rows' device arrays
+struct SxTile
+{
+    TileArgs t;
+    DevBuf tpos, bits, seg, next;
+};
+
+static int64_t sx_tile_row_bytes(int64_t n) { return (n + TL_W - 1) / TL_W * (TL_W / 8 + 8); }
+
+template <class S, int PHASE>
+static int sx_tile_run(SxArgs &g, TileArgs &t)
+{
+    hipStream_t st = stream();
+    ProfScope ps(PHASE == 0 ? "sx_tile_sym" : "sx_tile_num");
+    k_sx_zero<<<1, 64, 0, st>>>(t.next, 1);
+    const int64_t units = t.nf * t.nt + (t.T - t.nf) * ((t.nt + TL_RUN - 1) / TL_RUN);
+    k_sx_tile<S, PHASE><<<sx_grid(units, TL_NT / 64, (int64_t) cu_count() * 8), TL_NT, 0, st>>>(g, t);
+    return check_hip(hipGetLastError(), "k_sx_tile");
+}
+
+// bits and counts of the tiled rows (their Cp entries); kb: rows of B
+static int sx_tile_build(SxArgs &g, SxTile &x, const int64_t *hc, int64_t kb)
+{
+    hipStream_t st = stream();
+    const int64_t cap = (int64_t) cu_count() * 8;
+    TileArgs &t = x.t;
+    t.nf = hc[CNT_TILF];
+    t.T = hc[BIN_TIL];
+    t.nt = (g.n + TL_W - 1) / TL_W;
+    t.front = g.rows + (int64_t) BIN_TIL * g.m;
+    t.back = t.front + g.m - 1;
+    if (!x.bits.alloc((size_t) (t.T * t.nt) * (TL_W / 8)) || !x.seg.alloc(sizeof(int64_t) * (size_t) (t.T * t.nt + 1)) ||
+        !x.next.alloc(8))
+        return set_error(GM_OUT_OF_MEMORY, "saxpy3: tiled rows (%lld)", (long long) t.T);
+    t.bits = x.bits.as<uint64_t>();
+    t.seg = x.seg.as<int64_t>();
+    t.next = x.next.as<unsigned long long>();
+    t.tpos = nullptr;
+    // B's offsets at the tile ends, when the rows look up at least a quarter as
+    // many as there are and they fit 1 GB
+    if (4 * hc[CNT_TILA] >= kb && (double) kb * (double) (t.nt + 1) <= (double) (1 << 28) &&
+        x.tpos.alloc(sizeof(uint32_t) * (size_t) (kb * (t.nt + 1))))
+    {
+        ProfScope ps("sx_tile_pos");
+        k_sx_tile_pos<<<sx_grid(kb * (t.nt + 1), TL_NT, cap * 4), TL_NT, 0, st>>>(g.Bp, g.Bj, kb, t.nt,
+                                                                               x.tpos.as<uint32_t>());
+        GM_HIP(hipGetLastError(), "k_sx_tile_pos");
+        t.tpos = x.tpos.as<uint32_t>();
+    }
+    GM_TRY((sx_tile_run<SR<GM_ADD_ANY, GM_MULT_PAIR, uint8_t>, 0>(g, t)));
+    GM_TRY(scan_exclusive_i64(t.seg, t.seg, t.T * t.nt));
+    k_sx_tile_rows<<<sx_grid(t.T, TL_NT, cap), TL_NT, 0, st>>>(g, t);
+    return check_hip(hipGetLastError(), "k_sx_tile_rows");
+}
+
 // flop count, binning and the dealing out of the heavy rows; hc receives the
 // counters
-static int sx_count(SxArgs &g, int64_t fs, int list_small, int64_t dmax, int64_t *dflops, int64_t *hc,
+static int sx_count(SxArgs &g, int64_t fs, int list_small, int64_t dmax, int64_t tmax, int64_t *dflops, int64_t *hc,
                     unsigned long long *hp)
 {
     hipStream_t st = stream();
@@ -1380,13 +1464,14 @@ static int sx_count(SxArgs &g, int64_t fs, int list_small, int64_t dmax, int64_t
         }
         k_sx_flops<<<sx_grid(g.m, SX_NT / TG, (int64_t) cu_count() * 16), SX_NT, 0, st>>>(g, fs, list_small);
         g.rowf = nullptr;
-        k_sx_classify<<<sx_grid(g.m, SX_NT, (int64_t) cu_count()), SX_NT, 0, st>>>(g, dflops, dmax);
+        k_sx_classify<<<sx_grid(g.m, SX_NT, (int64_t) cu_count()), SX_NT, 0, st>>>(g, dflops, dmax, tmax);
         GM_HIP(hipGetLastError(), "k_sx_flops");
     }
-    GM_HIP(hipMemcpyAsync(hp, g.cnt, 16 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st), "bin counts");
+    GM_HIP(hipMemcpyAsync(hp, g.cnt, SX_NCNT * sizeof(unsigned long long), hipMemcpyDeviceToHost, st), "bin counts");
     GM_HIP(hipStreamSynchronize(st), "bin counts sync");
-    for (int t = 0; t < 16; t++) hc[t] = (int64_t) hp[t];
+    for (int t = 0; t < SX_NCNT; t++) hc[t] = (int64_t) hp[t];
     if (hc[BIN_DNS] > dmax) hc[BIN_DNS] = dmax;
+    hc[BIN_TIL] = hc[CNT_TILF] + hc[CNT_TILB];
     return GM_SUCCESS;
 }
 
@@ -1484,6 +1569,8 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     int64_t dmax = 0;
     if (SX_ANY_ORDER<S> && B->nrows < (int64_t) 0xffffffff)
         dmax = (int64_t) ((double) device_hbm_bytes() / 32.0 / (sx_push_row_bytes<S>(n, M != nullptr) + 1.0));
+    // tiled rows at most: their bits within 1/64 of HBM
+    const int64_t tmax = n > 0 ? device_hbm_bytes() / 64 / sx_tile_row_bytes(n) : 0;
     int64_t hc[SX_NCNT] = {0};
     unsigned long long *hp = (unsigned long long *) pinned_scratch(SX_NCNT * sizeof(unsigned long long));
     if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
@@ -1545,7 +1632,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         dflops = g.hflops + m;
         g.rows = (uint32_t *) (dflops + m);
         g.gtab_log2 = (int32_t *) (g.rows + SX_NBINS * m);
-        GM_TRY(sx_count(g, fs, fused ? 0 : 1, dmax, dflops, hc, hp));
+        GM_TRY(sx_count(g, fs, fused ? 0 : 1, dmax, tmax, dflops, hc, hp));
         cap_small = hc[CNT_SMALL];
         if (fused && (double) cap_small * (double) entry_bytes > budget)
         {
@@ -1553,7 +1640,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             // small rows listed for the symbolic + numeric path
             fused = false;
             k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
-            GM_TRY(sx_count(g, fs, 1, dmax, dflops, hc, hp));
+            GM_TRY(sx_count(g, fs, 1, dmax, tmax, dflops, hc, hp));
         }
     }
 
@@ -1567,8 +1654,11 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
                              (long long) gslots);
         g.gkeys = gkeys.as<uint32_t>(); g.gvals = gvals.ptr; g.glist = glist.as<uint64_t>();
     }
-    const int64_t nbig = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB] + hc[BIN_DNS];
+    const int64_t nbig = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB] + hc[BIN_DNS] +
+                         hc[BIN_TIL];
     const bool have_big = nbig > 0;
+    SxTile tiles;
+    if (hc[BIN_TIL] > 0) GM_TRY(sx_tile_build(g, tiles, hc, B->nrows));
     SxPush push;
     memset(&push.h, 0, sizeof(push.h));
     push.h.dflops = dflops;
@@ -1660,6 +1750,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         nvals = (int64_t) hp[11];
         // 5. numeric phase of the big rows
         if (have_big && nvals > 0) GM_TRY((sx_launch_phase<S, 1>(g, hc, true)));
+        if (hc[BIN_TIL] > 0 && nvals > 0) GM_TRY((sx_tile_run<S, 1>(g, tiles.t)));
         if constexpr (SX_ANY_ORDER<S>)
             if (hc[BIN_DNS] > 0 && nvals > 0) GM_TRY(sx_push_write<S>(g, push));
     }
@@ -1677,6 +1768,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         g.Ci = Ci.as<int64_t>();
         g.Cx = Cx.ptr;
         if (nvals > 0) GM_TRY((sx_launch_phase<S, 1>(g, hc, false)));
+        if (hc[BIN_TIL] > 0 && nvals > 0) GM_TRY((sx_tile_run<S, 1>(g, tiles.t)));
         if constexpr (SX_ANY_ORDER<S>)
             if (hc[BIN_DNS] > 0 && nvals > 0) GM_TRY(sx_push_write<S>(g, push));
     }
