@@ -42,6 +42,7 @@ constexpr int D3_P1_PER_THREAD = 4;   // entries per thread per phase1 tile
 constexpr int D3_P1_TILE = D3_NT * D3_P1_PER_THREAD;
 constexpr int D3_CT_IPT = 8;          // compaction items per thread
 constexpr int D3_CT_TILE = D3_NT * D3_CT_IPT;
+constexpr int64_t CT_SUM_MAX = 512;   // at most so many tiles add up the counts before them themselves
 
 // Probe indexes of the long rows of one operand (rows of length >= T).  A row
 // with column range [lo, hi] gets
@@ -909,21 +910,6 @@ __device__ __forceinline__ void team_task(const Dot3Args &g, uint64_t w, int lan
     if (lane == 0) d3_store<S>(g, p, e, z);
 }
 
-// the bin's entries in their appended order, strided over the grid
-template <class S, int G>
-__global__ __launch_bounds__(D3_NT) void k_dot3_team(Dot3Args g, int bin)
-{
-    const int64_t count = (int64_t) g.bin_cnt[bin];
-    const uint64_t *list = g.bins + (int64_t) bin * g.mnz;
-    constexpr int TPB = D3_NT / G;
-    __shared__ uint32_t s_lists[TPB][StageCap<G>::value];
-    const int lane = threadIdx.x & (G - 1);
-    uint32_t *sl = s_lists[threadIdx.x / G];
-    for (int64_t q = (int64_t) blockIdx.x * TPB + threadIdx.x / G; q < count;
-         q += (int64_t) gridDim.x * TPB)
-        team_task<S, G>(g, list[q], lane, sl);
-}
-
 // The bin's entries sorted by the row whose probe index they read.  The list
 // is cut into 8 regions, one per XCD (workgroups are dispatched to the 8 XCDs
 // round-robin, so workgroup b runs on XCD b mod 8): an XCD's workgroups take
@@ -985,15 +971,25 @@ __device__ __forceinline__ void block_task(const Dot3Args &g, uint64_t w, typena
     __syncthreads();
 }
 
+// the three bins' entries in their appended order, strided over the grid: one
+// launch for small problems, where a launch costs as much as its work
 template <class S>
-__global__ __launch_bounds__(D3_NT) void k_dot3_block(Dot3Args g)
+__global__ __launch_bounds__(D3_NT) void k_dot3_teams(Dot3Args g)
 {
     using Z = typename S::Z;
+    __shared__ uint32_t s_lists[(D3_NT / 16) * StageCap<16>::value];
     __shared__ Z s_z[D3_NT / 64];
     __shared__ int s_e[D3_NT / 64];
-    const int64_t count = (int64_t) g.bin_cnt[2];
-    const uint64_t *list = g.bins + 2 * g.mnz;
-    for (int64_t q = blockIdx.x; q < count; q += gridDim.x) block_task<S>(g, list[q], s_z, s_e);
+    static_assert((D3_NT / 64) * StageCap<64>::value <= (D3_NT / 16) * StageCap<16>::value, "staging lists");
+    const int64_t n0 = (int64_t) g.bin_cnt[0], n1 = (int64_t) g.bin_cnt[1], n2 = (int64_t) g.bin_cnt[2];
+    for (int64_t q = blockIdx.x; q < n2; q += gridDim.x) block_task<S>(g, g.bins[2 * g.mnz + q], s_z, s_e);
+    for (int64_t q = (int64_t) blockIdx.x * (D3_NT / 64) + threadIdx.x / 64; q < n1;
+         q += (int64_t) gridDim.x * (D3_NT / 64))
+        team_task<S, 64>(g, g.bins[g.mnz + q], threadIdx.x & 63, s_lists + threadIdx.x / 64 * StageCap<64>::value);
+    __syncthreads();
+    for (int64_t q = (int64_t) blockIdx.x * (D3_NT / 16) + threadIdx.x / 16; q < n0;
+         q += (int64_t) gridDim.x * (D3_NT / 16))
+        team_task<S, 16>(g, g.bins[q], threadIdx.x & 15, s_lists + threadIdx.x / 16 * StageCap<16>::value);
 }
 
 // the heaviest bin sorted by probed row, over the same 8 XCD regions as the
@@ -1844,16 +1840,26 @@ template <class Z, bool ISO>
 __global__ __launch_bounds__(D3_NT) void k_dot3_compact(const int64_t *__restrict__ Mp,
     const int64_t *__restrict__ Mj, int64_t m_nrows, int64_t mnz,
     const uint8_t *__restrict__ live, const Z *__restrict__ W,
-    const int64_t *__restrict__ tile_off, int64_t *__restrict__ Cp,
-    int64_t *__restrict__ Ci, Z *__restrict__ Cx)
+    const int64_t *__restrict__ tile_off, int scanned, int64_t *__restrict__ Cp,
+    int64_t *__restrict__ Ci, Z *__restrict__ Cx, int64_t *total)
 {
     constexpr int NW = D3_NT / 64;
     static_assert(D3_CT_IPT * NW <= 64, "one wavefront scans the per-step counts");
     __shared__ int32_t s_pre[D3_CT_TILE + 1];
     __shared__ int32_t s_cnt[D3_CT_IPT * NW];
     __shared__ int64_t s_row0;
+    __shared__ int64_t s_sum[NW + 1];
     const int64_t t0 = (int64_t) blockIdx.x * D3_CT_TILE;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    // entries of the tiles before: from the scan, or added up here
+    int64_t off;
+    if (scanned) off = tile_off[blockIdx.x];
+    else
+    {
+        int64_t s = 0;
+        for (int64_t t = threadIdx.x; t < (int64_t) blockIdx.x; t += D3_NT) s += tile_off[t];
+        off = block_sum<int64_t, D3_NT>(s, s_sum);
+    }
     if (threadIdx.x == 0)
     {
         // first row whose start lies at or after t0
@@ -1891,7 +1897,7 @@ __global__ __launch_bounds__(D3_NT) void k_dot3_compact(const int64_t *__restric
         if (lane == 63) s_pre[D3_CT_TILE] = incl;
     }
     __syncthreads();
-    const int64_t off = tile_off[blockIdx.x];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = off + s_pre[D3_CT_TILE];
     const unsigned long long below = (1ull << lane) - 1ull;
     #pragma unroll
     for (int t = 0; t < D3_CT_IPT; t++)
@@ -1947,85 +1953,146 @@ __global__ void k_zero_u64(unsigned long long *x, int n)
 
 constexpr int BM_HIST = 64;
 
-// words needed by eligible rows, bucketed by floor(log2(row length))
-__global__ __launch_bounds__(D3_NT) void k_d3_bm_hist(const int64_t *__restrict__ Xp,
-                                                      const int64_t *__restrict__ Xj, int64_t nrows,
+// words needed by eligible rows of A and B, bucketed by floor(log2(row length))
+__global__ __launch_bounds__(D3_NT) void k_d3_bm_hist(const int64_t *__restrict__ Ap, const int64_t *__restrict__ Aj,
+                                                      int64_t nA, const int64_t *__restrict__ Bp,
+                                                      const int64_t *__restrict__ Bj, int64_t nB,
                                                       int64_t minlen, unsigned long long *hist)
 {
     // per-workgroup histogram in LDS, then one atomic per nonzero bucket
-    __shared__ unsigned long long s_h[64];
-    if (threadIdx.x < 64) s_h[threadIdx.x] = 0;
+    __shared__ unsigned long long s_h[BM_HIST];
+    if (threadIdx.x < BM_HIST) s_h[threadIdx.x] = 0;
     __syncthreads();
-    for (int64_t r = (int64_t) blockIdx.x * D3_NT + threadIdx.x; r < nrows;
+    for (int64_t r = (int64_t) blockIdx.x * D3_NT + threadIdx.x; r < nA + nB;
          r += (int64_t) gridDim.x * D3_NT)
     {
-        const int64_t p0 = Xp[r], len = Xp[r + 1] - p0;
+        const int64_t *Xp = r < nA ? Ap + r : Bp + (r - nA);
+        const int64_t *Xj = r < nA ? Aj : Bj;
+        const int64_t p0 = Xp[0], len = Xp[1] - p0;
         if (len < minlen) continue;
         const int64_t lo = Xj[p0], hi = Xj[p0 + len - 1];
         const int b = 63 - __clzll((unsigned long long) len);
         atomicAdd(&s_h[b], (unsigned long long) px_units(len, lo, hi));
     }
     __syncthreads();
-    if (threadIdx.x < 64 && s_h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], s_h[threadIdx.x]);
+    if (threadIdx.x < BM_HIST && s_h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], s_h[threadIdx.x]);
 }
 
-// word offsets of the eligible rows (atomic bump) and the list of them
-__global__ __launch_bounds__(D3_NT) void k_d3_bm_assign(const int64_t *__restrict__ Xp,
-                                                        const int64_t *__restrict__ Xj, int64_t nrows,
-                                                        int64_t T, int64_t *off,
-                                                        unsigned long long *wctr,
-                                                        unsigned long long *lctr, uint32_t *list)
+constexpr int PREP_IPT = 4;
+
+// Rows r < nA are A's, the others B's row r - nA (nB = 0 when the operands are
+// one matrix).  In one pass: the unit offsets of the indexed rows (length >= T),
+// the list of them, every row's summary (when desc), and the largest column
+// span of a row.  A workgroup takes PREP_IPT * 256 rows at a time and makes one
+// reservation for them: with one per wavefront the two shared counters took
+// 1.4 ms of the pass at RMAT 22 (8.4M rows); it takes 0.42 ms here.
+__global__ __launch_bounds__(D3_NT) void k_d3_prep(const int64_t *__restrict__ Ap, const int64_t *__restrict__ Aj,
+                                                   int64_t nA, const int64_t *__restrict__ Bp,
+                                                   const int64_t *__restrict__ Bj, int64_t nB, int64_t T,
+                                                   int64_t *off, unsigned long long *wctr,
+                                                   unsigned long long *lctr, uint64_t *list, RowDesc *desc,
+                                                   unsigned long long *maxspan)
 {
-    // one reservation per wavefront for its rows' units and list slots;
-    // every lane of a wavefront runs the same iterations
+    __shared__ unsigned long long s_scan[D3_NT / 64 + 1], s_base[2];
     const int lane = threadIdx.x & 63;
-    for (int64_t r0 = (int64_t) blockIdx.x * D3_NT; r0 < nrows; r0 += (int64_t) gridDim.x * D3_NT)
+    const int64_t n = nA + nB;
+    unsigned long long ms = 0;
+    for (int64_t r0 = (int64_t) blockIdx.x * D3_NT * PREP_IPT; r0 < n; r0 += (int64_t) gridDim.x * D3_NT * PREP_IPT)
     {
-        const int64_t r = r0 + threadIdx.x;
-        bool take = false;
-        unsigned long long u = 0;
-        if (r < nrows)
+        int64_t p0[PREP_IPT], len[PREP_IPT], lo[PREP_IPT], hi[PREP_IPT];
+        // units taken << 16 | rows taken, of this thread's rows
+        unsigned long long take = 0;
+        #pragma unroll
+        for (int v = 0; v < PREP_IPT; v++)
         {
-            const int64_t p0 = Xp[r], len = Xp[r + 1] - p0;
-            if (len >= T)
+            const int64_t r = r0 + v * D3_NT + threadIdx.x;
+            p0[v] = 0; len[v] = 0; lo[v] = 0; hi[v] = -1;
+            if (r < n)
             {
-                take = true;
-                u = (unsigned long long) px_units(len, Xj[p0], Xj[p0 + len - 1]);
+                const int64_t *Xp = r < nA ? Ap + r : Bp + (r - nA);
+                p0[v] = Xp[0];
+                len[v] = Xp[1] - p0[v];
             }
         }
-        unsigned long long inc = u;
         #pragma unroll
-        for (int o = 1; o < 64; o <<= 1)
+        for (int v = 0; v < PREP_IPT; v++)
         {
-            const unsigned long long t = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += t;
+            const int64_t r = r0 + v * D3_NT + threadIdx.x;
+            if (len[v] > 0)
+            {
+                const int64_t *Xj = r < nA ? Aj : Bj;
+                lo[v] = Xj[p0[v]];
+                hi[v] = Xj[p0[v] + len[v] - 1];
+            }
         }
-        const unsigned long long total = __shfl(inc, 63, 64);
-        const unsigned long long mask = __ballot(take);
-        unsigned long long wbase = 0, lbase = 0;
-        if (lane == 0 && mask != 0)
+        #pragma unroll
+        for (int v = 0; v < PREP_IPT; v++)
         {
-            wbase = atomicAdd(wctr, total);
-            lbase = atomicAdd(lctr, (unsigned long long) __popcll(mask));
+            if (len[v] >= T && r0 + v * D3_NT + threadIdx.x < n)
+                take += ((unsigned long long) px_units(len[v], lo[v], hi[v]) << 16) + 1;
+            const unsigned long long sp = (unsigned long long) (hi[v] - lo[v] + 1);
+            ms = sp > ms ? sp : ms;
         }
-        wbase = __shfl(wbase, 0, 64);
-        lbase = __shfl(lbase, 0, 64);
-        if (take)
+        unsigned long long base = 0, at = 0;
+        if (__syncthreads_or(take != 0))
         {
-            off[r] = (int64_t) (wbase + inc - u);
-            list[lbase + (unsigned long long) __popcll(mask & ((1ull << lane) - 1ull))] = (uint32_t) r;
+            unsigned long long total;
+            const unsigned long long pre = block_exclusive_scan<unsigned long long, D3_NT>(take, s_scan, &total);
+            if (threadIdx.x == 0)
+            {
+                s_base[0] = atomicAdd(wctr, total >> 16);
+                s_base[1] = atomicAdd(lctr, total & 0xffffull);
+            }
+            __syncthreads();
+            base = s_base[0] + (pre >> 16);
+            at = s_base[1] + (pre & 0xffffull);
+        }
+        #pragma unroll
+        for (int v = 0; v < PREP_IPT; v++)
+        {
+            const int64_t r = r0 + v * D3_NT + threadIdx.x;
+            if (r >= n) continue;
+            const bool tk = len[v] >= T;
+            if (tk)
+            {
+                off[r] = (int64_t) base;
+                list[at++] = (uint64_t) r;
+            }
+            if (desc)
+            {
+                RowDesc d;
+                d.p0 = p0[v];
+                d.off = tk ? (int64_t) base : 0;
+                d.len = (int32_t) len[v];
+                d.lo = (int32_t) lo[v];
+                d.hi = (int32_t) hi[v];
+                d.kind = tk ? (bm_eligible(0, len[v], lo[v], hi[v]) ? 0 : hx_log2(len[v])) : -1;
+                desc[r] = d;
+            }
+            if (tk) base += (unsigned long long) px_units(len[v], lo[v], hi[v]);
         }
     }
+    // wavefront maximum, then an atomic only where it raises the value seen so far
+    #pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+    {
+        const unsigned long long t = __shfl_xor(ms, o, 64);
+        ms = t > ms ? t : ms;
+    }
+    if (lane == 0 && ms > __hip_atomic_load(maxspan, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(maxspan, ms);
 }
 
 // One workgroup per listed row: clear its words, then OR in its elements.
 // Elements are sorted, so the lanes holding one word are contiguous: a
 // segmented OR across the wavefront leaves one atomic per word per chunk.
 // rank[w] (when requested) = number of row entries before word w.
-__global__ __launch_bounds__(D3_NT) void k_d3_bm_build(const int64_t *__restrict__ Xp,
-                                                       const int64_t *__restrict__ Xj,
+__global__ __launch_bounds__(D3_NT) void k_d3_bm_build(const int64_t *__restrict__ Ap,
+                                                       const int64_t *__restrict__ Aj, int64_t nA,
+                                                       const int64_t *__restrict__ Bp,
+                                                       const int64_t *__restrict__ Bj,
                                                        const int64_t *__restrict__ off,
-                                                       const uint32_t *__restrict__ list,
+                                                       const uint64_t *__restrict__ list,
                                                        const unsigned long long *lctr,
                                                        unsigned long long *words, uint32_t *rank)
 {
@@ -2033,8 +2100,10 @@ __global__ __launch_bounds__(D3_NT) void k_d3_bm_build(const int64_t *__restrict
     const int64_t count = (int64_t) *lctr;
     for (int64_t q = blockIdx.x; q < count; q += gridDim.x)
     {
-        const int64_t r = list[q];
-        const int64_t p0 = Xp[r], p1 = Xp[r + 1];
+        const int64_t r = (int64_t) list[q];
+        const int64_t *Xp = r < nA ? Ap + r : Bp + (r - nA);
+        const int64_t *Xj = r < nA ? Aj : Bj;
+        const int64_t p0 = Xp[0], p1 = Xp[1];
         const int64_t lo = Xj[p0], hi = Xj[p1 - 1];
         const int64_t o = off[r];
         if (!bm_eligible(0, p1 - p0, lo, hi))
@@ -2128,50 +2197,6 @@ __global__ __launch_bounds__(D3_NT) void k_d3_chunkpos(const int64_t *__restrict
     }
 }
 
-// one summary per row (off: the probe index offsets, or NULL when the
-// operand has none; rows of length >= T have an index)
-__global__ __launch_bounds__(D3_NT) void k_d3_desc(const int64_t *__restrict__ Xp,
-                                                   const int64_t *__restrict__ Xj, int64_t nrows,
-                                                   int64_t T, const int64_t *__restrict__ off,
-                                                   RowDesc *__restrict__ out,
-                                                   unsigned long long *maxspan)
-{
-    unsigned long long ms = 0;
-    // every lane of a wavefront runs the same number of iterations
-    for (int64_t r0 = (int64_t) blockIdx.x * D3_NT; r0 < nrows; r0 += (int64_t) gridDim.x * D3_NT)
-    {
-        const int64_t r = r0 + threadIdx.x;
-        if (r >= nrows) continue;
-        const int64_t p0 = Xp[r], len = Xp[r + 1] - p0;
-        RowDesc d;
-        d.p0 = p0;
-        d.off = 0;
-        d.len = (int32_t) len;
-        d.lo = len > 0 ? (int32_t) Xj[p0] : 0;
-        d.hi = len > 0 ? (int32_t) Xj[p0 + len - 1] : -1;
-        d.kind = -1;
-        if (off && len >= T)
-        {
-            d.off = off[r];
-            d.kind = bm_eligible(0, len, d.lo, d.hi) ? 0 : hx_log2(len);
-        }
-        out[r] = d;
-        const unsigned long long sp = len > 0 ? (unsigned long long) (d.hi - d.lo + 1) : 0ull;
-        ms = sp > ms ? sp : ms;
-    }
-    // largest column span of a row: wavefront maximum, then an atomic only
-    // where it raises the value seen so far
-    #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-    {
-        const unsigned long long t = __shfl_xor(ms, o, 64);
-        ms = t > ms ? t : ms;
-    }
-    if ((threadIdx.x & 63) == 0 &&
-        ms > __hip_atomic_load(maxspan, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(maxspan, ms);
-}
-
 static inline unsigned grid_for(int64_t work_items, int64_t per_block, int64_t cap)
 {
     int64_t g = (work_items + per_block - 1) / per_block;
@@ -2180,86 +2205,132 @@ static inline unsigned grid_for(int64_t work_items, int64_t per_block, int64_t c
     return (unsigned) g;
 }
 
-// Decide which rows get bitmaps (longest first, within a budget of HBM),
-// then build them.  A and B share bitmaps when they are the same matrix.
-static int dot3_bitmaps(Dot3Args &g, const gm_csr *A, const gm_csr *B, bool need_rank,
-                        int64_t minlen, DevBuf &offA, DevBuf &offB, DevBuf &words, DevBuf &rank,
-                        DevBuf &list, DevBuf &ctr)
+// A call's entry counts and its counters (D3C_*), cleared
+struct D3Front
+{
+    DevBuf ctr;
+    int64_t mnz = 0, nza = 0, nzb = 0;
+};
+enum { D3C_BINS = 0,          // three bin counts, then the largest column span of a row
+       D3C_UNITS = 4,         // index units taken
+       D3C_LISTED = 5,        // indexed rows
+       D3C_HIST = 64,         // BM_HIST length buckets
+       D3C_N = 128 };
+
+// clears the counters and brings the three entry counts to the host (written
+// there by the kernel: no copy to queue)
+__global__ __launch_bounds__(D3C_N) void k_d3_front(unsigned long long *ctr, const int64_t *Mp, int64_t mn,
+                                                    const int64_t *Ap, int64_t an, const int64_t *Bp, int64_t bn,
+                                                    int64_t *host)
+{
+    ctr[threadIdx.x] = 0;
+    if (threadIdx.x == 0) host[0] = Mp[mn];
+    if (threadIdx.x == 1) host[1] = (Ap && an > 0) ? Ap[an] : 0;
+    if (threadIdx.x == 2) host[2] = (Bp && bn > 0) ? Bp[bn] : 0;
+}
+
+static int dot3_front(D3Front &f, const gm_csr *M, const gm_csr *A, const gm_csr *B)
+{
+    if (M->nrows <= 0 || !M->p) return GM_SUCCESS;
+    hipStream_t st = stream();
+    int64_t *hp = (int64_t *) pinned_scratch(3 * sizeof(int64_t));
+    if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
+    if (!f.ctr.alloc(D3C_N * sizeof(unsigned long long))) return set_error(GM_OUT_OF_MEMORY, "dot3: counters");
+    k_d3_front<<<1, D3C_N, 0, st>>>(f.ctr.as<unsigned long long>(), M->p, M->nrows, A->p, A->nrows, B->p, B->nrows,
+                                    hp);
+    GM_HIP(hipGetLastError(), "k_d3_front");
+    GM_HIP(hipStreamSynchronize(st), "dot3 sizes sync");
+    f.mnz = hp[0];
+    f.nza = hp[1];
+    f.nzb = hp[2];
+    return GM_SUCCESS;
+}
+
+// Decide which rows get bitmaps (longest first, within a budget of HBM), build
+// them, and write the row summaries (desc).  A and B share both when they are
+// the same matrix.  Operands whose indexes are sure to fit 64 MB -- a row's
+// takes at most 32 units per entry, and at most 4 per entry or the columns'
+// bitmap -- need no histogram and no wait for it.
+static int dot3_bitmaps(Dot3Args &g, D3Front &f, const gm_csr *A, const gm_csr *B, bool need_rank,
+                        int64_t minlen, int64_t *off, uint64_t *list, RowDesc *desc, DevBuf &words)
 {
     hipStream_t st = stream();
     const bool shared = (A->p == B->p && A->j == B->j && A->nrows == B->nrows);
-    if (!ctr.alloc(sizeof(unsigned long long) * (2 * BM_HIST + 8)))
-        return set_error(GM_OUT_OF_MEMORY, "dot3: bitmap counters");
-    unsigned long long *c = ctr.as<unsigned long long>();
-    k_zero_u64<<<1, 64, 0, st>>>(c, 64);
-    k_zero_u64<<<1, 64, 0, st>>>(c + 64, 64);
-    k_zero_u64<<<1, 64, 0, st>>>(c + 128, 8);
+    const int64_t nA = A->nrows, nB = shared ? 0 : B->nrows;
+    unsigned long long *c = f.ctr.as<unsigned long long>();
     const int64_t gcap = (int64_t) cu_count() * 8;
-    {
-        ProfScope ps("dot3_bm_hist");
-        k_d3_bm_hist<<<grid_for(A->nrows, D3_NT, gcap), D3_NT, 0, st>>>(A->p, A->j, A->nrows, minlen, c);
-        if (!shared)
-            k_d3_bm_hist<<<grid_for(B->nrows, D3_NT, gcap), D3_NT, 0, st>>>(B->p, B->j, B->nrows,
-                                                                            minlen, c + BM_HIST);
-        GM_HIP(hipGetLastError(), "k_d3_bm_hist");
-    }
-    unsigned long long *h = (unsigned long long *) pinned_scratch(sizeof(unsigned long long) * 2 * BM_HIST);
-    if (!h) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
-    GM_HIP(hipMemcpyAsync(h, c, sizeof(unsigned long long) * 2 * BM_HIST, hipMemcpyDeviceToHost, st),
-           "bitmap histogram");
-    GM_HIP(hipStreamSynchronize(st), "bitmap histogram sync");
     const double wbytes = 8.0 + (need_rank ? 4.0 : 0.0);
-    double budget = (double) device_hbm_bytes() / 16.0;
-    if (budget > 16e9) budget = 16e9;
-    // smallest length bucket whose cumulative words fit the budget
-    int b0 = -1;
-    double acc = 0;
-    for (int b = BM_HIST - 1; b >= 0; b--)
+    int64_t T = INT64_MAX, total_words = 0;
+    if (minlen > 0)
     {
-        const double wb = (double) (h[b] + h[BM_HIST + b]) * wbytes;
-        if (wb == 0) continue;
-        if (acc + wb > budget) break;
-        acc += wb;
-        b0 = b;
-    }
-    if (b0 < 0) return GM_SUCCESS;               // no row qualifies
-    int64_t T = (int64_t) 1 << b0;
-    if (T < minlen) T = minlen;
-    const int64_t total_words = (int64_t) (acc / wbytes) + 1;
-    if (!offA.alloc(sizeof(int64_t) * (A->nrows > 0 ? A->nrows : 1)) ||
-        (!shared && !offB.alloc(sizeof(int64_t) * (B->nrows > 0 ? B->nrows : 1))) ||
-        !words.alloc(sizeof(uint64_t) * total_words) ||
-        (need_rank && !rank.alloc(sizeof(uint32_t) * total_words)) ||
-        !list.alloc(sizeof(uint32_t) * ((A->nrows + (shared ? 0 : B->nrows)) > 0
-                                        ? (A->nrows + (shared ? 0 : B->nrows)) : 1)))
-        return set_error(GM_OUT_OF_MEMORY, "dot3: bitmaps (%lld words)", (long long) total_words);
-    uint32_t *lst = list.as<uint32_t>();
-    // c[128]: word bump shared by A and B; c[129] / c[130]: rows of A / B listed
-    {
-        ProfScope ps("dot3_bm_build");
-        unsigned long long *dw = words.as<unsigned long long>();
-        uint32_t *rk = need_rank ? rank.as<uint32_t>() : nullptr;
-        k_d3_bm_assign<<<grid_for(A->nrows, D3_NT, gcap), D3_NT, 0, st>>>(
-            A->p, A->j, A->nrows, T, offA.as<int64_t>(), c + 128, c + 129, lst);
-        GM_HIP(hipGetLastError(), "k_d3_bm_assign");
-        k_d3_bm_build<<<(unsigned) gcap, D3_NT, 0, st>>>(A->p, A->j, offA.as<int64_t>(), lst, c + 129,
-                                                         dw, rk);
-        GM_HIP(hipGetLastError(), "k_d3_bm_build");
-        if (!shared)
+        const double nz = (double) f.nza + (shared ? 0.0 : (double) f.nzb);
+        const double bound = std::min(32.0 * nz, 4.0 * nz + (nz / (double) minlen + 1.0) * ((double) A->ncols / 64.0 + 2.0));
+        if (bound * wbytes <= (double) (64 << 20))
         {
-            k_d3_bm_assign<<<grid_for(B->nrows, D3_NT, gcap), D3_NT, 0, st>>>(
-                B->p, B->j, B->nrows, T, offB.as<int64_t>(), c + 128, c + 130, lst + A->nrows);
-            GM_HIP(hipGetLastError(), "k_d3_bm_assign");
-            k_d3_bm_build<<<(unsigned) gcap, D3_NT, 0, st>>>(B->p, B->j, offB.as<int64_t>(),
-                                                             lst + A->nrows, c + 130, dw, rk);
-            GM_HIP(hipGetLastError(), "k_d3_bm_build");
+            T = minlen;
+            total_words = (int64_t) bound + 1;
+        }
+        else
+        {
+            {
+                ProfScope ps("dot3_bm_hist");
+                k_d3_bm_hist<<<grid_for(nA + nB, D3_NT, gcap), D3_NT, 0, st>>>(A->p, A->j, nA, B->p, B->j, nB, minlen,
+                                                                              c + D3C_HIST);
+                GM_HIP(hipGetLastError(), "k_d3_bm_hist");
+            }
+            unsigned long long *h = (unsigned long long *) pinned_scratch(sizeof(unsigned long long) * BM_HIST);
+            if (!h) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
+            GM_HIP(hipMemcpyAsync(h, c + D3C_HIST, sizeof(unsigned long long) * BM_HIST, hipMemcpyDeviceToHost, st),
+                   "bitmap histogram");
+            GM_HIP(hipStreamSynchronize(st), "bitmap histogram sync");
+            double budget = (double) device_hbm_bytes() / 16.0;
+            if (budget > 16e9) budget = 16e9;
+            // smallest length bucket whose cumulative words fit the budget
+            int b0 = -1;
+            double acc = 0;
+            for (int b = BM_HIST - 1; b >= 0; b--)
+            {
+                const double wb = (double) h[b] * wbytes;
+                if (wb == 0) continue;
+                if (acc + wb > budget) break;
+                acc += wb;
+                b0 = b;
+            }
+            if (b0 >= 0)
+            {
+                T = (int64_t) 1 << b0;
+                if (T < minlen) T = minlen;
+                total_words = (int64_t) (acc / wbytes) + 1;
+            }
         }
     }
-    g.bA = RowBits{T, offA.as<int64_t>(), (const uint64_t *) words.ptr,
-                   need_rank ? rank.as<uint32_t>() : nullptr};
-    g.bB = shared ? g.bA
-                  : RowBits{T, offB.as<int64_t>(), (const uint64_t *) words.ptr,
-                            need_rank ? rank.as<uint32_t>() : nullptr};
+    if (T != INT64_MAX && !words.alloc((sizeof(uint64_t) + (need_rank ? sizeof(uint32_t) : 0)) * total_words))
+        return set_error(GM_OUT_OF_MEMORY, "dot3: bitmaps (%lld words)", (long long) total_words);
+    unsigned long long *dw = words.as<unsigned long long>();
+    uint32_t *rk = (need_rank && T != INT64_MAX) ? (uint32_t *) (dw + total_words) : nullptr;
+    if (T != INT64_MAX || desc)
+    {
+        ProfScope ps("dot3_prep");
+        k_d3_prep<<<grid_for(nA + nB, D3_NT * PREP_IPT, gcap), D3_NT, 0, st>>>(A->p, A->j, nA, B->p, B->j, nB, T, off,
+                                                                       c + D3C_UNITS, c + D3C_LISTED, list, desc,
+                                                                       c + D3C_BINS + 3);
+        GM_HIP(hipGetLastError(), "k_d3_prep");
+    }
+    if (T != INT64_MAX)
+    {
+        ProfScope ps("dot3_bm_build");
+        const int64_t most = (f.nza + (shared ? 0 : f.nzb)) / T + 1;      // rows that long at most
+        k_d3_bm_build<<<grid_for(most, 1, gcap), D3_NT, 0, st>>>(A->p, A->j, nA, B->p, B->j, off, list, c + D3C_LISTED,
+                                                                 dw, rk);
+        GM_HIP(hipGetLastError(), "k_d3_bm_build");
+        g.bA = RowBits{T, off, (const uint64_t *) words.ptr, rk};
+        g.bB = shared ? g.bA : RowBits{T, off + nA, (const uint64_t *) words.ptr, rk};
+    }
+    if (desc)
+    {
+        g.dA = desc;
+        g.dB = shared ? desc : desc + nA;
+    }
     return GM_SUCCESS;
 }
 
@@ -2267,17 +2338,14 @@ static int dot3_bitmaps(Dot3Args &g, const gm_csr *A, const gm_csr *B, bool need
 // of (key, entry) pairs) and run them with the XCD-regioned kernels.  The
 // bins' keys must have been written by phase1 (g.bkeys != NULL).
 template <class S>
-static int dot3_grouped_teams(Dot3Args &g, const gm_csr *A, const gm_csr *B)
+static int dot3_grouped_teams(Dot3Args &g, const D3Front &f, const gm_csr *A, const gm_csr *B)
 {
     const int64_t nkeys = A->nrows + B->nrows;
     hipStream_t st = stream();
-    unsigned long long *hc = (unsigned long long *) pinned_scratch(6 * sizeof(unsigned long long));
+    unsigned long long *hc = (unsigned long long *) pinned_scratch(4 * sizeof(unsigned long long));
     if (!hc) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
     GM_HIP(hipMemcpyAsync(hc, g.bin_cnt, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
            "bin counts");
-    // the operands' entry counts (32-bit column copies for the chunk kernel)
-    GM_HIP(hipMemcpyAsync(hc + 4, A->p + A->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(A)");
-    GM_HIP(hipMemcpyAsync(hc + 5, B->p + B->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(B)");
     GM_HIP(hipStreamSynchronize(st), "bin counts sync");
     const int64_t cnt[3] = {(int64_t) hc[0], (int64_t) hc[1], (int64_t) hc[2]};
     // every row spans at most L1_BITS columns: whole bitmaps fit in LDS
@@ -2336,7 +2404,7 @@ static int dot3_grouped_teams(Dot3Args &g, const gm_csr *A, const gm_csr *B)
     if (LC_NARROW && g.cols32 && g.dA != nullptr &&
         ((small && (cnt[0] > 0 || cnt[1] > 0)) || (lds && (lds_chunk || cnt[0] > 0))))
     {
-        const int64_t nza = (int64_t) hc[4], nzb = shared ? 0 : (int64_t) hc[5];
+        const int64_t nza = f.nza, nzb = shared ? 0 : f.nzb;
         if (narA.alloc(sizeof(uint32_t) * (nza > 0 ? nza : 1)) &&
             (shared || narB.alloc(sizeof(uint32_t) * (nzb > 0 ? nzb : 1))))
         {
@@ -2463,35 +2531,29 @@ static int dot3_grouped_teams(Dot3Args &g, const gm_csr *A, const gm_csr *B)
 
 template <class S>
 static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_csr *A,
-                    const gm_csr *B, const gm_dot3_params *prm, int64_t mnz_known = -1)
+                    const gm_csr *B, const gm_dot3_params *prm, D3Front *front = nullptr)
 {
     using Z = typename S::Z;
     hipStream_t st = stream();
     const int64_t n = M->nrows;
-    int64_t Mnz = (n > 0) ? mnz_known : 0;
-    if (Mnz < 0)
+    D3Front own;
+    if (!front)
     {
-        // nnz(M) from its last row pointer
-        int64_t *hp = (int64_t *) pinned_scratch(sizeof(int64_t));
-        if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
-        GM_HIP(hipMemcpyAsync(hp, M->p + n, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(M)");
-        GM_HIP(hipStreamSynchronize(st), "nnz(M) sync");
-        Mnz = *hp;
+        GM_TRY(dot3_front(own, M, A, B));
+        front = &own;
     }
+    const int64_t Mnz = front->mnz;
     if (Mnz >= ((int64_t) 1 << 32) || n >= ((int64_t) 1 << 32))
         return set_error(GM_NO_VALUE, "dot3: nnz(M) or nrows beyond 2^32");
 
     const size_t zs = sizeof(Z);
-    DevBuf Cp, Ci, Cx, W, live, bins, cnt;
+    DevBuf Cp, Ci, Cx, work;
     if (!Cp.alloc(sizeof(int64_t) * (n + 1)) || !Ci.alloc(sizeof(int64_t) * (Mnz > 0 ? Mnz : 1)) ||
         !Cx.alloc(S::iso_out ? zs : zs * (Mnz > 0 ? Mnz : 1)))
         return set_error(GM_OUT_OF_MEMORY, "dot3: output");
     int64_t nvals = 0;
     if (Mnz > 0)
     {
-        if (!W.alloc(S::iso_out ? 8 : zs * Mnz) || !live.alloc(Mnz) ||
-            !bins.alloc(sizeof(uint64_t) * 3 * Mnz) || !cnt.alloc(4 * sizeof(unsigned long long)))
-            return set_error(GM_OUT_OF_MEMORY, "dot3: workspace");
         Dot3Args g;
         g.Mp = M->p; g.Mj = M->j; g.Mx = mask_struct ? nullptr : M->x;
         g.msize = (int32_t) type_size(M->type); g.m_iso = M->iso; g.mask_struct = mask_struct ? 1 : 0;
@@ -2499,59 +2561,46 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         g.m_nrows = n; g.mnz = Mnz;
         g.Ap = A->p; g.Aj = A->j; g.Ax = A->x; g.a_iso = A->iso;
         g.Bp = B->p; g.Bj = B->j; g.Bx = B->x; g.b_iso = B->iso;
-        g.W = W.ptr; g.live = live.as<uint8_t>(); g.bins = bins.as<uint64_t>();
-        g.bin_cnt = cnt.as<unsigned long long>();
+        g.bin_cnt = front->ctr.as<unsigned long long>() + D3C_BINS;
         g.cols32 = (A->ncols < ((int64_t) 1 << 32)) ? 1 : 0;
-        g.bkeys = nullptr;
         g.key_nA = A->nrows;
         // group deferred entries by probed row: explicit, or by default for
         // masks large enough that the sort pays for itself
         const gm_dot3_params tu = dot3_tuned();
         const int64_t order = (prm && prm->order) ? prm->order : tu.order;
         const bool grouped = (order == 2) || (order == 0 && Mnz >= ((int64_t) 1 << 20));
-        DevBuf bkeys;
-        if (grouped)
-        {
-            if (!bkeys.alloc(sizeof(uint64_t) * 3 * Mnz))
-                return set_error(GM_OUT_OF_MEMORY, "dot3: grouping keys");
-            g.bkeys = bkeys.as<uint64_t>();
-        }
         g.thread_max = pick_param(prm ? prm->thread_max : 0, tu.thread_max, 8);
         g.team16_max = pick_param(prm ? prm->team16_max : 0, tu.team16_max, 512);
         g.wave_max = pick_param(prm ? prm->wave_max : 0, tu.wave_max, 4096);
         const int64_t cap = (int64_t) cu_count() * 16;
         g.bA = RowBits{INT64_MAX, nullptr, nullptr, nullptr};
         g.bB = g.bA;
-        DevBuf bm_offA, bm_offB, bm_words, bm_rank, bm_list, bm_ctr;
+        g.dA = nullptr;
+        g.dB = nullptr;
         int64_t minlen = (prm && prm->bitmap_min_len != 0) ? prm->bitmap_min_len
                        : (tu.bitmap_min_len != 0 ? tu.bitmap_min_len : 128);
         if (A->ncols >= ((int64_t) 1 << 32)) minlen = -1;   // hash keys are 32-bit columns
-        if (minlen > 0)
-            GM_TRY(dot3_bitmaps(g, A, B, !S::pattern, minlen, bm_offA, bm_offB, bm_words, bm_rank,
-                                bm_list, bm_ctr));
-        k_zero_u64<<<1, 64, 0, st>>>(g.bin_cnt, 4);
-        // row summaries for pair setup (columns must fit 31 bits); bin_cnt[3]
-        // receives the largest column span of a row
-        g.dA = nullptr;
-        g.dB = nullptr;
-        DevBuf descA, descB;
-        if (A->ncols < ((int64_t) 1 << 31))
-        {
-            const bool shared = (A->p == B->p && A->j == B->j && A->nrows == B->nrows);
-            if (descA.alloc(sizeof(RowDesc) * (A->nrows > 0 ? A->nrows : 1)) &&
-                (shared || descB.alloc(sizeof(RowDesc) * (B->nrows > 0 ? B->nrows : 1))))
-            {
-                ProfScope ps("dot3_desc");
-                k_d3_desc<<<grid_for(A->nrows, D3_NT, cap), D3_NT, 0, st>>>(
-                    A->p, A->j, A->nrows, g.bA.T, g.bA.off, descA.as<RowDesc>(), g.bin_cnt + 3);
-                if (!shared)
-                    k_d3_desc<<<grid_for(B->nrows, D3_NT, cap), D3_NT, 0, st>>>(
-                        B->p, B->j, B->nrows, g.bB.T, g.bB.off, descB.as<RowDesc>(), g.bin_cnt + 3);
-                GM_HIP(hipGetLastError(), "k_d3_desc");
-                g.dA = descA.as<RowDesc>();
-                g.dB = shared ? g.dA : descB.as<RowDesc>();
-            }
-        }
+        // the workspace in one block: row summaries (columns below 2^31), bins,
+        // grouping keys, index offsets and list, tile offsets, results, flags
+        const bool shared = (A->p == B->p && A->j == B->j && A->nrows == B->nrows);
+        const bool use_desc = A->ncols < ((int64_t) 1 << 31);
+        const size_t nr = (size_t) A->nrows + (shared ? 0 : (size_t) B->nrows);
+        const int64_t ntiles = (Mnz + D3_CT_TILE - 1) / D3_CT_TILE;
+        const size_t wbytes = S::iso_out ? 0 : (zs * (size_t) Mnz + 7) / 8 * 8;
+        if (!work.alloc((use_desc ? sizeof(RowDesc) * nr : 0) + 8 * 3 * (size_t) Mnz * (grouped ? 2 : 1) + 16 * nr +
+                        8 * (size_t) (ntiles + 1) + wbytes + (size_t) Mnz))
+            return set_error(GM_OUT_OF_MEMORY, "dot3: workspace");
+        RowDesc *desc = use_desc ? work.as<RowDesc>() : nullptr;
+        g.bins = use_desc ? (uint64_t *) (desc + nr) : work.as<uint64_t>();
+        uint64_t *at = g.bins + 3 * (size_t) Mnz;
+        g.bkeys = grouped ? at : nullptr;
+        if (grouped) at += 3 * (size_t) Mnz;
+        int64_t *off = (int64_t *) at, *toff = off + 2 * nr;
+        uint64_t *list = at + nr;
+        g.W = toff + ntiles + 1;
+        g.live = (uint8_t *) g.W + wbytes;
+        DevBuf words;
+        GM_TRY(dot3_bitmaps(g, *front, A, B, !S::pattern, minlen, off, list, desc, words));
         // whole rows to the row kernel: mask rows with at least row_min
         // entries whose A row spans fewer than RM_BITS columns
         const int64_t row_min = (prm && prm->row_min != 0) ? prm->row_min
@@ -2577,26 +2626,13 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         }
         if (grouped)
         {
-            GM_TRY(dot3_grouped_teams<S>(g, A, B));
+            GM_TRY(dot3_grouped_teams<S>(g, *front, A, B));
         }
         else
         {
-            {
-                ProfScope ps("dot3_team16");
-                k_dot3_team<S, 16><<<(unsigned) (cu_count() * 8), D3_NT, 0, st>>>(g, 0);
-                GM_HIP(hipGetLastError(), "k_dot3_team16");
-            }
-            {
-                ProfScope ps("dot3_wave");
-                k_dot3_team<S, 64><<<(unsigned) (cu_count() * 8), D3_NT, 0, st>>>(g, 1);
-                GM_HIP(hipGetLastError(), "k_dot3_wave");
-            }
-        }
-        if (!grouped)
-        {
-            ProfScope ps("dot3_block");
-            k_dot3_block<S><<<(unsigned) (cu_count() * 8), D3_NT, 0, st>>>(g);
-            GM_HIP(hipGetLastError(), "k_dot3_block");
+            ProfScope ps("dot3_teams");
+            k_dot3_teams<S><<<grid_for(Mnz, D3_NT / 16, (int64_t) cu_count() * 8), D3_NT, 0, st>>>(g);
+            GM_HIP(hipGetLastError(), "k_dot3_teams");
         }
         if (g.rowmode)
         {
@@ -2605,28 +2641,23 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
                 g, rm_rows.as<uint32_t>(), rm_cnt.as<unsigned long long>());
             GM_HIP(hipGetLastError(), "k_dot3_rows");
         }
-        // compaction
-        const int64_t ntiles = (Mnz + D3_CT_TILE - 1) / D3_CT_TILE;
-        DevBuf toff;
-        if (!toff.alloc(sizeof(int64_t) * (ntiles + 1)))
-            return set_error(GM_OUT_OF_MEMORY, "dot3: compaction workspace");
+        // compaction; the entry count comes to the host with the last tile
         {
             ProfScope ps("dot3_tile_count");
-            k_dot3_tile_count<<<(unsigned) ntiles, D3_NT, 0, st>>>(live.as<uint8_t>(), Mnz,
-                                                                   toff.as<int64_t>());
+            k_dot3_tile_count<<<(unsigned) ntiles, D3_NT, 0, st>>>(g.live, Mnz, toff);
             GM_HIP(hipGetLastError(), "k_dot3_tile_count");
         }
-        GM_TRY(scan_exclusive_i64(toff.as<int64_t>(), toff.as<int64_t>(), ntiles));
+        const bool scanned = ntiles > CT_SUM_MAX;
+        if (scanned) GM_TRY(scan_exclusive_i64(toff, toff, ntiles));
+        int64_t *hp = (int64_t *) pinned_scratch(sizeof(int64_t));
+        if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
         {
             ProfScope ps("dot3_compact");
             k_dot3_compact<Z, S::iso_out><<<(unsigned) ntiles, D3_NT, 0, st>>>(
-                M->p, M->j, n, Mnz, live.as<uint8_t>(), (const Z *) W.ptr, toff.as<int64_t>(),
-                Cp.as<int64_t>(), Ci.as<int64_t>(), (Z *) Cx.ptr);
+                M->p, M->j, n, Mnz, g.live, (const Z *) g.W, toff, scanned ? 1 : 0,
+                Cp.as<int64_t>(), Ci.as<int64_t>(), (Z *) Cx.ptr, hp);
             GM_HIP(hipGetLastError(), "k_dot3_compact");
         }
-        int64_t *hp = (int64_t *) pinned_scratch(sizeof(int64_t));
-        GM_HIP(hipMemcpyAsync(hp, toff.as<int64_t>() + ntiles, sizeof(int64_t),
-                              hipMemcpyDeviceToHost, st), "nvals");
         GM_HIP(hipStreamSynchronize(st), "dot3 sync");
         nvals = *hp;
     }
@@ -2844,13 +2875,13 @@ extern "C" int gm_AxB_dot3(gm_csr_out *C, const gm_csr *M, bool mask_struct, con
 
 static int dot3_dispatch(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_csr *A,
                          const gm_csr *B, const gm_semiring *sr, const gm_dot3_params *params,
-                         int64_t mnz_known = -1)
+                         D3Front *front = nullptr)
 {
     int rc = GM_NO_VALUE;
 #define GM_DOT3_CASE(ADD, MULT, ZC, Z)                                         \
     if (sr->add_op == ADD && sr->mult_op == MULT && sr->ztype == ZC)           \
     {                                                                          \
-        rc = dot3_run<SR<ADD, MULT, Z>>(C, M, mask_struct, A, B, params, mnz_known); \
+        rc = dot3_run<SR<ADD, MULT, Z>>(C, M, mask_struct, A, B, params, front); \
         if (rc == GM_SUCCESS) C->type = ZC;                                    \
         return rc;                                                             \
     }
@@ -2999,20 +3030,12 @@ extern "C" int gm_dot3(gm_csr_out *C, const gm_csr *M, bool mask_struct, const g
     if (!gm_dot3_branch(M, mask_struct, A, B, sr))
         return set_error(GM_NO_VALUE, "gm_dot3: case not handled by the GPU kernels");
     GM_TRY(ensure_init());
-    int64_t mnz = -1;
-    if (M->nrows > 0 && M->p)
-    {
-        int64_t *hp = (int64_t *) pinned_scratch(sizeof(int64_t));
-        if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
-        hipStream_t st = stream();
-        GM_HIP(hipMemcpyAsync(hp, M->p + M->nrows, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(M)");
-        GM_HIP(hipStreamSynchronize(st), "nnz(M) sync");
-        mnz = *hp;
-        const int64_t slice_max = g_dot3_slice_max;
-        if (mnz >= slice_max || M->nrows >= ((int64_t) 1 << 31))
-            return dot3_sliced(C, M, mask_struct, A, B, sr, params, slice_max);
-    }
-    return dot3_dispatch(C, M, mask_struct, A, B, sr, params, mnz);
+    D3Front front;
+    GM_TRY(dot3_front(front, M, A, B));
+    const int64_t slice_max = g_dot3_slice_max;
+    if (front.mnz >= slice_max || M->nrows >= ((int64_t) 1 << 31))
+        return dot3_sliced(C, M, mask_struct, A, B, sr, params, slice_max);
+    return dot3_dispatch(C, M, mask_struct, A, B, sr, params, &front);
 }
 
 // sums over the mask entries (i,j) of min(|A(i,:)|, |B(j,:)|) and of
