@@ -309,3 +309,34 @@ def test_dot3_row_slices(grb, slice_max):
         assert_csr_equal(C.to_csr(), ref, what="sliced tricount")
     finally:
         L.gm_debug_dot3_slice_max(0)
+
+
+@pytest.mark.parametrize("valued", [False, True])
+@pytest.mark.parametrize("handle", list(SR))
+def test_dot3_no_long_rows(grb, handle, valued):
+    """Operands whose rows are all shorter than the index length and too large
+    for the no-histogram case: rows of 0, 1 and 127 entries, mask rows with
+    more entries than a wavefront takes, and stretches of more than 64 empty
+    mask rows."""
+    print(f"[dot3] no long rows {handle} valued={valued}", flush=True)
+    rng = np.random.default_rng(len(handle))
+    vt = _vals(handle)
+
+    def rows(lens, ncols, values):
+        p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        j = np.concatenate([np.sort(rng.choice(ncols, size=int(l), replace=False)) for l in lens]).astype(np.int64)
+        x = {"fp64": rng.random(len(j)), "int32": rng.integers(-50, 50, len(j)).astype(np.int32),
+             "int64": rng.integers(-50, 50, len(j)).astype(np.int64)}.get(values)
+        return W.Csr(len(lens), ncols, p, j, x)
+    n, K = 3001, 700
+    A = rows(rng.choice([0, 1, 30, 64, 65, 100, 127], n, p=[.05, .05, .2, .2, .2, .2, .1]), K, vt)
+    B = rows(rng.choice([0, 1, 15, 16, 17, 64, 127], n, p=[.05, .05, .1, .1, .1, .3, .3]), K, vt)
+    assert 32 * 8 * (A.nnz + B.nnz) > 64 << 20
+    ml = rng.integers(0, 6, n)
+    ml[100:400] = 0
+    ml[500] = 1000
+    M = rows(ml, n, "int64" if valued else None)
+    name, _ = SR[handle]
+    ref = O.dot3(name, M, A, B, mask_struct=not valued)
+    got = gm_dot3(handle, M, A, B, mask_struct=not valued)
+    assert_csr_equal(got, ref, fp_tol=FP_TOL if "fp64" in name else None, what=handle)
