@@ -6,6 +6,7 @@ through the C-ABI (gm_dot3) and through the drop-in GrB_mxm.
 """
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import pyoracle as O
 from graphblas_amd import capi
@@ -340,3 +341,47 @@ def test_dot3_no_long_rows(grb, handle, valued):
     ref = O.dot3(name, M, A, B, mask_struct=not valued)
     got = gm_dot3(handle, M, A, B, mask_struct=not valued)
     assert_csr_equal(got, ref, fp_tol=FP_TOL if "fp64" in name else None, what=handle)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("mask", ["structural", "valued", "A"])
+@pytest.mark.parametrize("handle", list(SR))
+def test_dot3_one_matrix(grb, handle, mask, order):
+    """C<M> = A*A' with a mask that is symmetric but for a few entries, whose
+    values (valued mask) differ between the two sides, with diagonal entries:
+    each pair computed once, the others alone; and the mask that is A itself."""
+    import ctypes
+    from helpers import ZT, download
+    print(f"[dot3] one matrix {handle} {mask} order={order}", flush=True)
+    rng = np.random.default_rng(len(handle) + order)
+    vt = _vals(handle)
+    G = W.rmat_sym(11, 40, seed=5)
+    n = G.nrows
+    A = W.Csr(n, n, G.p, G.j, {"fp64": rng.random(G.nnz), "int32": rng.integers(-50, 50, G.nnz).astype(np.int32),
+                               "int64": rng.integers(-50, 50, G.nnz).astype(np.int64)}.get(vt))
+    if mask == "A":
+        M = G
+    else:
+        m = G.to_scipy() + sp.eye(n)
+        drop = rng.choice(m.nnz, size=m.nnz // 20, replace=False)
+        m = m.tocsr()
+        m.data[:] = 1
+        m.data[drop] = 0
+        m.eliminate_zeros()
+        M = W.Csr.from_scipy(m, keep_values=False)
+        if mask == "valued":
+            M.x = (rng.random(M.nnz) < 0.7).astype(np.int64)
+    assert M.nnz >= 1 << 16
+    name, trip = SR[handle]
+    dA = DevCsr(A, trip[2])
+    dM = dA if mask == "A" else DevCsr(M, 8)
+    out, sr = capi.GmCsrOut(), capi.GmSemiring(*trip)
+    prm = capi.GmDot3Params(0, 0, 0, 0, order, 0)
+    rc = capi.lib().gm_dot3(ctypes.byref(out), ctypes.byref(dM.view), mask != "valued", ctypes.byref(dA.view),
+                            ctypes.byref(dA.view), ctypes.byref(sr), ctypes.byref(prm))
+    assert rc == 0, capi.last_error()
+    got = download(out, ZT[{8: "int64", 6: "int32", 1: "bool", 11: "fp64"}[trip[2]]])
+    ref = O.dot3(name, M, A, A, mask_struct=mask != "valued")
+    assert_csr_equal(got, ref, fp_tol=FP_TOL if "fp64" in name else None, what=f"{handle} {mask}")
+    for d in (dA, dM):
+        d.free()
