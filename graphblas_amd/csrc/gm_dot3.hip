@@ -1456,10 +1456,17 @@ __global__ __launch_bounds__(LC_NT) void k_dot3_lds(Dot3Args g, const uint64_t *
 // short rows against it: lane l takes elements l, l+G, ... of the 32-bit
 // column copy (eight loads in flight) and the partials combine in lane
 // order, as in the global probe.  Other entries run the team kernel's own
-// path, without LDS staging: the kernel keeps its LDS small and its
+// path, without LDS staging (an entry of two rows without an index counts as
+// a probe of A(i,:), whose run it sorts into): the kernel keeps its LDS small and its
 // registers capped at eight wavefronts per SIMD, because it is bound by the
 // latency of its entries' loads (4096-graph batch: 16-lane bin 387 -> 291
-// ms, wavefront bin 220 -> 164 ms).
+// ms, wavefront bin 220 -> 164 ms).  The probe arithmetic is 32-bit: one
+// unsigned compare for the long row's range.  With the entries of two rows
+// without an index looked up too, the 16-lane bin of a 256-graph batch went
+// from 6.8 to 5.3 ms (plus_pair int32) and from 11.8 to 9.9 ms (min_plus int32).
+// A valued semiring's hit reads its two values from memory: with the long
+// row's values in LDS and the short row's read beside its columns the
+// latter took 13.1 ms (five wavefronts per SIMD, and most elements miss).
 constexpr int L1_BITS = 1 << 16;
 constexpr int L1_WORDS = L1_BITS / 64;
 constexpr int L1_SLICE = 256;
@@ -1475,7 +1482,7 @@ __global__ __launch_bounds__(D3_NT) __attribute__((amdgpu_waves_per_eu(8))) void
     constexpr int TPB = D3_NT / G;
     constexpr bool RANK = !S::pattern;
     __shared__ uint64_t s_bits[L1_WORDS];
-    __shared__ uint32_t s_rank[RANK ? L1_WORDS : 1];
+    __shared__ uint16_t s_rank[RANK ? L1_WORDS : 1];       // positions below 2^16, as the span is
     __shared__ uint64_t s_key[L1_SLICE];
     // every slice entry's short row (start, length) and probe direction
     // (0: none, 1: into A's row, 2: into B's row), set up together at the
@@ -1513,9 +1520,11 @@ __global__ __launch_bounds__(D3_NT) __attribute__((amdgpu_waves_per_eu(8))) void
                     const int64_t i = (int64_t) (w >> 32), p = (int64_t) (w & 0xffffffffull);
                     Pair P;
                     (void) d3_pair(g, i, g.Mj[p], P);
-                    if (!P.empty && P.probe != 0)
+                    if (!P.empty)
                     {
-                        dir = (int8_t) P.probe;
+                        // neither row indexed: the run's row is A(i,:), B(j,:) is
+                        // looked up in it instead of merged with it
+                        dir = P.probe ? (int8_t) P.probe : (int8_t) 1;
                         const bool shortA = (P.probe == 2);
                         s_sp0[t] = shortA ? P.pa : P.pb;
                         s_slen[t] = (uint32_t) (shortA ? P.pa_end - P.pa : P.pb_end - P.pb);
@@ -1553,7 +1562,7 @@ __global__ __launch_bounds__(D3_NT) __attribute__((amdgpu_waves_per_eu(8))) void
                         {
                             // the first entry of its word records its position
                             if (e == d.p0 || ((Lj[e - 1] - d.lo) >> 6) != wd)
-                                s_rank[wd] = (uint32_t) (e - d.p0);
+                                s_rank[wd] = (uint16_t) (e - d.p0);
                         }
                     }
                     __syncthreads();
@@ -1576,18 +1585,57 @@ __global__ __launch_bounds__(D3_NT) __attribute__((amdgpu_waves_per_eu(8))) void
                     // steps of UN elements per lane, loads issued together (past
                     // the end: the last element again, no branch around the
                     // loads); the lane stops after a step past the long row's range
-                    constexpr int UN = N32 ? 8 : 4;
-                    const uint32_t *Sj32 = shortA ? A32 : B32;
-                    for (int64_t q0s = s0 + lane; q0s < s1; q0s += UN * G)
+                    if constexpr (N32)
+                    {
+                        constexpr int UN = 8;
+                        const uint32_t *S32 = (shortA ? A32 : B32) + s0;
+                        const Z *Sx = shortA ? Ax : Bx, *Lx = shortA ? Bx : Ax;
+                        const int32_t s_iso = shortA ? g.a_iso : g.b_iso, l_iso = shortA ? g.b_iso : g.a_iso;
+                        const uint32_t len = s_slen[t], lo = (uint32_t) d.lo, span = (uint32_t) (d.hi - d.lo);
+                        for (uint32_t q = lane; q < len; q += UN * G)
+                        {
+                            uint32_t raw[UN];
+                            #pragma unroll
+                            for (int u = 0; u < UN; u++) raw[u] = S32[q + u * G < len ? q + u * G : len - 1];
+                            #pragma unroll
+                            for (int u = 0; u < UN; u++)
+                            {
+                                // below the long row's first column: wraps above the span
+                                const uint32_t dd = raw[u] - lo;
+                                const bool in = q + u * G < len && dd <= span;
+                                const uint32_t w = ((const uint32_t *) s_bits)[in ? dd >> 5 : 0];
+                                const bool hit = in && ((w >> (dd & 31)) & 1u);
+                                if constexpr (S::add == GM_ADD_PLUS && S::mult == GM_MULT_PAIR) cnt += hit ? 1u : 0u;
+                                else if (hit)
+                                {
+                                    Z tz;
+                                    if constexpr (RANK)
+                                    {
+                                        const uint64_t word = s_bits[dd >> 6];
+                                        const int pos = (int) s_rank[dd >> 6] +
+                                                        __popcll(word & ((1ull << (dd & 63)) - 1ull));
+                                        // (multipliers with values commute)
+                                        tz = S::mul(S::geta(Sx, s0 + q + u * G, s_iso),
+                                                    S::geta(Lx, d.p0 + pos, l_iso), 0);
+                                    }
+                                    else tz = S::mul(Z(1), Z(1), (int64_t) raw[u]);
+                                    if (!e) { z = tz; e = true; }
+                                    else if constexpr (S::any_min_k) { if (tz < z) z = tz; }
+                                    else z = S::upd(z, tz);
+                                }
+                            }
+                            if (raw[UN - 1] > (uint32_t) d.hi) break;
+                        }
+                    }
+                    constexpr int UN = 4;
+                    for (int64_t q0s = s0 + lane; !N32 && q0s < s1; q0s += UN * G)
                     {
                         int64_t xs[UN];
                         #pragma unroll
                         for (int u = 0; u < UN; u++)
                         {
                             const int64_t qq = q0s + u * G;
-                            const int64_t qc = qq < s1 ? qq : s1 - 1;
-                            if constexpr (N32) xs[u] = (int64_t) Sj32[qc];
-                            else xs[u] = Sj[qc];
+                            xs[u] = Sj[qq < s1 ? qq : s1 - 1];
                         }
                         #pragma unroll
                         for (int u = 0; u < UN; u++)
