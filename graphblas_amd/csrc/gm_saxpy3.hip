@@ -432,7 +432,10 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
 //   dense table (BIN_DNS; the semiring allows any order, dmax rows at most): a
 //     row with more than 1/512 of all heavy flops, on which one workgroup
 //     would outlast the others, and at least n/128 flops, so that the table's
-//     clearing and compaction stay below its updates
+//     clearing and compaction stay below its updates; or a row whose own
+//     workgroup (50 ns a flop) would take longer than tables for all the
+//     heavy rows (2.5e-6 us a column): 20000 f >= heavy rows * n (second BFS
+//     level of 64 searches, RMAT 20: 1.34 -> 0.90 ms)
 //   tiles (BIN_TIL, tmax rows at most): la * (n / TL_W) <= 4 f, where finding
 //     the parts of B's rows costs less than a hash table's inserts and sort
 //     (n = 40009: rows whose B rows hold 10 entries or more on average), and
@@ -455,7 +458,8 @@ __global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops
         const bool push = dmax > 0 && g.table != 1;
         const bool tile = tmax > 0 && g.table != 1 && f >= 16 * nt &&
                           (search <= 4.0 * (double) f || (!push && most && search <= 64.0 * (double) f));
-        if (push && ((most && f >= g.n / 128) || (!tile && f >= g.n / 4)))
+        if (push && ((most && f >= g.n / 128) || (!tile && f >= g.n / 4) ||
+                     20000.0 * (double) f >= (double) count * (double) g.n))
         {
             const int64_t d = (int64_t) atomicAdd(&g.cnt[BIN_DNS], 1ull);
             if (d < dmax)
@@ -523,6 +527,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_sum_big(SxArgs g, int64_t dmax)
 // single-entry rows: C(i,:) = A(i,k) (x) B(k,:) filtered by the mask
 //------------------------------------------------------------------------------
 
+constexpr int SINGLE_UN = 8;
 template <class S, int PHASE>
 __global__ __launch_bounds__(SX_NT) void k_sx_single(SxArgs g)
 {
@@ -547,28 +552,38 @@ __global__ __launch_bounds__(SX_NT) void k_sx_single(SxArgs g)
         const int64_t cbase = PHASE ? g.Cp[i] : 0;
         const int64_t cend = PHASE ? g.Cp[i + 1] : 0;
         int64_t run = 0;
-        for (int64_t c0 = b0; c0 < b1; c0 += 64)
+        // SINGLE_UN windows of 64 entries, their reads out together
+        for (int64_t c0 = b0; c0 < b1; c0 += 64 * SINGLE_UN)
         {
-            const int64_t pb = c0 + lane;
-            bool ok = false;
-            int64_t j = 0;
-            if (pb < b1)
+            int64_t j[SINGLE_UN];
+            Z x[SINGLE_UN];
+            bool ok[SINGLE_UN];
+            #pragma unroll
+            for (int u = 0; u < SINGLE_UN; u++)
             {
-                j = g.Bj[pb];
-                ok = sx_mask_ok(g, pm0, pm1, j);
+                const int64_t pb = c0 + u * 64 + lane;
+                ok[u] = pb < b1;
+                j[u] = g.Bj[ok[u] ? pb : b1 - 1];
+                x[u] = Z(0);
+                if constexpr (PHASE == 1 && !S::iso_out) x[u] = S::geta((const Z *) g.Bx, ok[u] ? pb : b1 - 1, g.b_iso);
             }
-            const unsigned long long bal = __ballot(ok);
-            if (PHASE == 1 && ok)
+            #pragma unroll
+            for (int u = 0; u < SINGLE_UN; u++) ok[u] = ok[u] && sx_mask_ok(g, pm0, pm1, j[u]);
+            #pragma unroll
+            for (int u = 0; u < SINGLE_UN; u++)
             {
-                const int64_t pos = cbase + run + __popcll(bal & ((1ull << lane) - 1ull));
-                if (pos < cend)
+                const unsigned long long bal = __ballot(ok[u]);
+                if (PHASE == 1 && ok[u])
                 {
-                    g.Ci[pos] = j;
-                    if constexpr (!S::iso_out)
-                        ((Z *) g.Cx)[pos] = S::mul(av, S::geta((const Z *) g.Bx, pb, g.b_iso), k);
+                    const int64_t pos = cbase + run + __popcll(bal & ((1ull << lane) - 1ull));
+                    if (pos < cend)
+                    {
+                        g.Ci[pos] = j[u];
+                        if constexpr (!S::iso_out) ((Z *) g.Cx)[pos] = S::mul(av, x[u], k);
+                    }
                 }
+                run += __popcll(bal);
             }
-            run += __popcll(bal);
         }
         if (PHASE == 0 && lane == 0) g.Cp[i] = run;
     }
