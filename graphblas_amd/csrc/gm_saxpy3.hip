@@ -328,6 +328,16 @@ __global__ __launch_bounds__(SX_NT) void k_sx_maxlen(const int64_t *__restrict__
 // single / wave1024 / block4096 / global bins.
 //------------------------------------------------------------------------------
 
+// A row of f flops from la entries of A is cut into tiles (gm_sx_tile.h) when
+// finding the parts of B's rows costs less than a hash table's inserts and sort:
+// la * (n / TL_W) <= 4 f (n = 40009: rows whose B rows hold 10 entries or more
+// on average), with 16 flops per tile at least.
+__device__ __forceinline__ bool sx_tiled(const SxArgs &g, int64_t f, int64_t la)
+{
+    const int64_t nt = (g.n + TL_W - 1) / TL_W;
+    return g.table != 1 && f >= 16 * nt && (double) la * (double) nt <= 4.0 * (double) f;
+}
+
 __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int list_small)
 {
     __shared__ unsigned int s_bc[SX_NBINS];
@@ -392,7 +402,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
             else if (f <= fs) { bin = list_small ? BIN_WS : -1; fsum += (unsigned long long) f; }
             else if (a1 - a0 == 1) bin = BIN_SINGLE;
             else if (t <= g.wl_max) bin = BIN_WL;
-            else if (t <= g.blk_max) bin = BIN_BLK;
+            else if (t <= g.blk_max && !sx_tiled(g, f, a1 - a0)) bin = BIN_BLK;
             else bin = BIN_HVY;
         }
         __syncthreads();
@@ -436,11 +446,8 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
 //     workgroup (50 ns a flop) would take longer than tables for all the
 //     heavy rows (2.5e-6 us a column): 20000 f >= heavy rows * n (second BFS
 //     level of 64 searches, RMAT 20: 1.34 -> 0.90 ms)
-//   tiles (BIN_TIL, tmax rows at most): la * (n / TL_W) <= 4 f, where finding
-//     the parts of B's rows costs less than a hash table's inserts and sort
-//     (n = 40009: rows whose B rows hold 10 entries or more on average), and
-//     16 flops per tile; a very heavy fp64 row, whose order the dense table
-//     does not keep, up to 64 f
+//   tiles (BIN_TIL, tmax rows at most): sx_tiled, or for a very heavy fp64 row,
+//     whose order the dense table does not keep, la * (n / TL_W) <= 64 f
 //   dense table again: at least n/4 flops
 //   else a hash table of 2^ceil(log2(2t)) slots, load factor <= 1/2, or a
 //     dense one of 2^ceil(log2(ncols)) slots (SxArgs::table)
@@ -454,10 +461,10 @@ __global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops
         const uint32_t i = g.rows[(int64_t) BIN_HVY * g.m + q];
         const int64_t f = g.hflops[q], la = g.Ap[i + 1] - g.Ap[i];
         const bool most = (double) f * 512 > total;
-        const double search = (double) la * (double) nt;
         const bool push = dmax > 0 && g.table != 1;
-        const bool tile = tmax > 0 && g.table != 1 && f >= 16 * nt &&
-                          (search <= 4.0 * (double) f || (!push && most && search <= 64.0 * (double) f));
+        const bool tile = tmax > 0 && g.table != 1 &&
+                          (sx_tiled(g, f, la) ||
+                           (!push && most && f >= 16 * nt && (double) la * (double) nt <= 64.0 * (double) f));
         if (push && ((most && f >= g.n / 128) || (!tile && f >= g.n / 4) ||
                      20000.0 * (double) f >= (double) count * (double) g.n))
         {
@@ -1418,7 +1425,7 @@ static int sx_tile_run(SxArgs &g, TileArgs &t)
 {
     hipStream_t st = stream();
     ProfScope ps(PHASE == 0 ? "sx_tile_sym" : "sx_tile_num");
-    k_sx_zero<<<1, 64, 0, st>>>(t.next, 1);
+    if (PHASE == 1) k_sx_zero<<<1, 128, 0, st>>>(t.next, 128);
     const int64_t units = t.nf * t.nt + (t.T - t.nf) * ((t.nt + TL_RUN - 1) / TL_RUN);
     k_sx_tile<S, PHASE><<<sx_grid(units, TL_NT / 64, (int64_t) cu_count() * 8), TL_NT, 0, st>>>(g, t);
     return check_hip(hipGetLastError(), "k_sx_tile");
@@ -1436,7 +1443,7 @@ static int sx_tile_build(SxArgs &g, SxTile &x, const int64_t *hc, int64_t kb)
     t.front = g.rows + (int64_t) BIN_TIL * g.m;
     t.back = t.front + g.m - 1;
     if (!x.bits.alloc((size_t) (t.T * t.nt) * (TL_W / 8)) || !x.seg.alloc(sizeof(int64_t) * (size_t) (t.T * t.nt + 1)) ||
-        !x.next.alloc(8))
+        !x.next.alloc(128 * sizeof(unsigned long long)))
         return set_error(GM_OUT_OF_MEMORY, "saxpy3: tiled rows (%lld)", (long long) t.T);
     t.bits = x.bits.as<uint64_t>();
     t.seg = x.seg.as<int64_t>();

@@ -18,7 +18,7 @@
 // Bound by the latency of its dependent steps (A entry, offsets, products,
 // LDS), covered by 16 wavefronts per CU.  RMAT square, n = 40009, 0.47M entries,
 // 59.8M entries of C, fp64: 30.3 ms with a workgroup and a table in HBM per
-// row, 5.4 ms here for the call.
+// row, 4.3 ms here for the call.
 #pragma once
 
 namespace gm
@@ -36,7 +36,7 @@ struct TileArgs
     const uint32_t *tpos;              // NULL, or nrows(B) x (nt + 1) offsets of B's rows
     uint64_t *bits;                    // T x nt x (TL_W / 64)
     int64_t *seg;                      // T x nt + 1: scanned tile counts
-    unsigned long long *next;
+    unsigned long long *next;          // eight counters, 128 bytes apart
 };
 
 __device__ __forceinline__ int64_t tl_row(const TileArgs &t, int64_t q)
@@ -75,11 +75,29 @@ __global__ __launch_bounds__(TL_NT) void k_sx_tile(SxArgs g, TileArgs t)
     if constexpr (VALS && !SX_ANY_ORDER<S>)
         for (int x = lane; x < SX_OWN; x += 64) s_own[wv][x] = 0xffffffffu;
     wave_sync();
+    // The symbolic phase's units are dealt out by stride (80000 units from one
+    // counter: 1.74 ms, 1.03 ms by stride); the numeric phase's, whose work
+    // varies more (by stride 3.06 ms, one counter 2.52 ms), from eight counters,
+    // one for the units of each remainder by 8, a workgroup's own first.
+    int64_t su = (int64_t) blockIdx.x + (int64_t) wv * gridDim.x;
+    int rem = (int) (blockIdx.x & 7), left = 8;
     while (true)
     {
-        int64_t u = 0;
-        if (lane == 0) u = (int64_t) atomicAdd(t.next, 1ull);
-        u = __shfl(u, 0, 64);
+        int64_t u = su;
+        if constexpr (PHASE == 0) su += (int64_t) gridDim.x * NWV;
+        else
+        {
+            u = units;
+            while (left > 0)
+            {
+                int64_t k = 0;
+                if (lane == 0) k = (int64_t) atomicAdd(&t.next[16 * rem], 1ull);
+                u = __shfl(k, 0, 64) * 8 + rem;
+                if (u < units) break;
+                rem = (rem + 1) & 7;
+                left--;
+            }
+        }
         if (u >= units) break;
         const bool heavy = u < hunits;
         const int64_t v = u - hunits;
