@@ -38,8 +38,11 @@ namespace gm
 {
 
 constexpr int D3_NT = 256;            // threads per workgroup everywhere here
-constexpr int D3_P1_PER_THREAD = 4;   // entries per thread per phase1 tile
-constexpr int D3_P1_TILE = D3_NT * D3_P1_PER_THREAD;
+// entries per thread of a phase1 tile: four, or one for masks below 2^18
+// entries, whose tiles would leave most of the device idle (16000 mask entries:
+// tiles of 1024 left a call at 104 us, tiles of 256 at 91)
+constexpr int D3_P1_PER_THREAD = 4;
+constexpr int64_t D3_P1_SMALL = 1 << 18;
 constexpr int D3_CT_IPT = 8;          // compaction items per thread
 constexpr int D3_CT_TILE = D3_NT * D3_CT_IPT;
 constexpr int64_t CT_SUM_MAX = 512;   // at most so many tiles add up the counts before them themselves
@@ -771,25 +774,26 @@ __device__ __forceinline__ void d3_store(const Dot3Args &g, int64_t p, bool e, t
 // phase1: classify every mask entry, finish the small ones
 //------------------------------------------------------------------------------
 
-template <class S>
+template <class S, int PT>
 __global__ __launch_bounds__(D3_NT) void k_dot3_phase1(Dot3Args g)
 {
     using Z = typename S::Z;
+    constexpr int TILE = D3_NT * PT;       // entries
     __shared__ int64_t s_rows[2];
     // the tile's row pointers Mp[r0 .. r1+1], when the window is short
-    __shared__ int64_t s_mp[D3_P1_TILE + 2];
+    __shared__ int64_t s_mp[TILE + 2];
     // the tile's binned entries: bin (-1: none), record, grouping key; the
     // wavefronts' ballots per bin, their offsets in the tile, the bases
-    __shared__ int8_t s_bin[D3_P1_TILE];
-    __shared__ uint64_t s_rec[D3_P1_TILE], s_bkey[D3_P1_TILE];
-    __shared__ unsigned long long s_mb[D3_P1_PER_THREAD][D3_NT / 64][3];
-    __shared__ unsigned long long s_pre[D3_P1_PER_THREAD][D3_NT / 64][3];
+    __shared__ int8_t s_bin[TILE];
+    __shared__ uint64_t s_rec[TILE], s_bkey[TILE];
+    __shared__ unsigned long long s_mb[PT][D3_NT / 64][3];
+    __shared__ unsigned long long s_pre[PT][D3_NT / 64][3];
     __shared__ unsigned long long s_base[3];
-    const int64_t ntiles = (g.mnz + D3_P1_TILE - 1) / D3_P1_TILE;
+    const int64_t ntiles = (g.mnz + TILE - 1) / TILE;
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
     {
-        const int64_t t0 = tile * D3_P1_TILE;
-        const int64_t t1 = (t0 + D3_P1_TILE < g.mnz) ? t0 + D3_P1_TILE : g.mnz;
+        const int64_t t0 = tile * TILE;
+        const int64_t t1 = (t0 + TILE < g.mnz) ? t0 + TILE : g.mnz;
         if (threadIdx.x < 2)
         {
             // row containing entry t0 (thread 0) / t1-1 (thread 1)
@@ -804,12 +808,12 @@ __global__ __launch_bounds__(D3_NT) void k_dot3_phase1(Dot3Args g)
         }
         __syncthreads();
         const int64_t r0 = s_rows[0], r1 = s_rows[1];
-        const bool lds_rows = (r1 - r0 + 2) <= (int64_t) (D3_P1_TILE + 2);
+        const bool lds_rows = (r1 - r0 + 2) <= (int64_t) (TILE + 2);
         if (lds_rows)
             for (int64_t t = threadIdx.x; t <= r1 - r0 + 1; t += D3_NT) s_mp[t] = g.Mp[r0 + t];
         __syncthreads();
         #pragma unroll 1
-        for (int u = 0; u < D3_P1_PER_THREAD; u++)
+        for (int u = 0; u < PT; u++)
         {
             const int64_t p = t0 + (int64_t) u * D3_NT + threadIdx.x;
             const bool valid = p < t1;
@@ -896,7 +900,7 @@ __global__ __launch_bounds__(D3_NT) void k_dot3_phase1(Dot3Args g)
         {
             const int b = (int) threadIdx.x;
             unsigned long long run = 0;
-            for (int u = 0; u < D3_P1_PER_THREAD; u++)
+            for (int u = 0; u < PT; u++)
                 for (int w = 0; w < D3_NT / 64; w++)
                 {
                     s_pre[u][w][b] = run;
@@ -906,7 +910,7 @@ __global__ __launch_bounds__(D3_NT) void k_dot3_phase1(Dot3Args g)
         }
         __syncthreads();
         #pragma unroll
-        for (int u = 0; u < D3_P1_PER_THREAD; u++)
+        for (int u = 0; u < PT; u++)
         {
             const int tslot = u * D3_NT + (int) threadIdx.x;
             const int b = s_bin[tslot];
@@ -2882,7 +2886,10 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         else
         {
             ProfScope ps("dot3_phase1");
-            k_dot3_phase1<S><<<grid_for(Mnz, D3_P1_TILE, cap), D3_NT, 0, st>>>(g);
+            if (Mnz < D3_P1_SMALL)
+                k_dot3_phase1<S, 1><<<grid_for(Mnz, D3_NT, cap), D3_NT, 0, st>>>(g);
+            else
+                k_dot3_phase1<S, D3_P1_PER_THREAD><<<grid_for(Mnz, D3_NT * D3_P1_PER_THREAD, cap), D3_NT, 0, st>>>(g);
             GM_HIP(hipGetLastError(), "k_dot3_phase1");
         }
         if (no_long) { }

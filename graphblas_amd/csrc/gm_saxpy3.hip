@@ -53,7 +53,6 @@ enum { CNT_SLOTS = 8,       // table slots of BIN_GLB
        CNT_SMALL = 10,      // flops of the small rows
        CNT_HFLOPS = 11,     // flops of BIN_HVY
        CNT_NNZA = 12,       // nnz(A)
-       CNT_ERR = 13,        // the look-back's error flag
        CNT_TILF = 14,       // BIN_TIL's very heavy rows (at the list's front; the others from its back)
        CNT_TILA = 15,       // A's entries in BIN_TIL's rows
        CNT_TILB = 22,       // BIN_TIL's other rows
@@ -962,9 +961,7 @@ constexpr int LB_WIN = 1;            // look-back window: LB_WIN x 64 predecesso
 // PK: 0 B read from Bp/Bj/Bx, 1 from the packed pairs, 2 from the row records
 template <class S, class K, int NT, int PK>
 __global__ __launch_bounds__(NT, sizeof(K) == 4 ? SX_FUSED_WAVES : 3)
-void k_sx_fused(SxArgs g, int64_t fs,
-                                                         unsigned long long *status, int64_t ntiles,
-                                                         int *err)
+void k_sx_fused(SxArgs g, int64_t fs, unsigned long long *status, int64_t ntiles, int64_t *host)
 {
     using Z = typename S::Z;
     constexpr int FUSED_ROWS = NT / TG;
@@ -1287,7 +1284,8 @@ void k_sx_fused(SxArgs g, int64_t fs,
                         // a predecessor has not published yet
                         if (++spins > LB_SPIN_LIMIT)
                         {
-                            if (lane == 0) atomicExch(err, 1);
+                            if (lane == 0)
+                                __hip_atomic_store(&host[1], (int64_t) 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                             break;
                         }
                         __builtin_amdgcn_s_sleep(1);
@@ -1313,7 +1311,12 @@ void k_sx_fused(SxArgs g, int64_t fs,
         const int64_t prefix = s_prefix;
         const int64_t total = s_off[FUSED_ROWS];
         if (sub == 0 && i < g.m) g.Cp[i] = prefix + s_off[team];
-        if (tile == ntiles - 1 && threadIdx.x == 0) g.Cp[g.m] = prefix + total;
+        if (tile == ntiles - 1 && threadIdx.x == 0)
+        {
+            // the host reads nnz(C) there after its wait: no copy to queue
+            g.Cp[g.m] = prefix + total;
+            host[0] = prefix + total;
+        }
         // each team copies its own small row: the row's entries are
         // contiguous in C, its lanes store consecutive ones
         if (!big && i < g.m)
@@ -1552,7 +1555,10 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     const size_t entry_bytes = sizeof(int64_t) + (S::iso_out ? 0 : zs);
 
     DevBuf Cp, cnt, lists;
-    if (!Cp.alloc(sizeof(int64_t) * (m + 1)) || !cnt.alloc(sizeof(unsigned long long) * SX_NCNT))
+    // the counters and the fused kernel's tile status words, cleared together
+    const int64_t ntiles = (m + FUSED_ROWS - 1) / FUSED_ROWS;
+    if (!Cp.alloc(sizeof(int64_t) * (m + 1)) ||
+        !cnt.alloc(sizeof(unsigned long long) * (size_t) (SX_NCNT + ntiles + 1)))
         return set_error(GM_OUT_OF_MEMORY, "saxpy3: workspace");
 
     SxArgs g;
@@ -1616,7 +1622,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     // together with its synchronisation.
     int64_t maxA = 0, maxB = 0, nnzA = 0, nnzB = -1;
     const bool probe_small = m * 8 >= B->nrows;
-    k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
+    k_sx_fill_u64<<<sx_grid(SX_NCNT + ntiles + 1, 256, 1024), 256, 0, st>>>(g.cnt, SX_NCNT + ntiles + 1);
     GM_HIP(hipGetLastError(), "k_sx_fill_u64");
     if (probe_small)
     {
@@ -1709,14 +1715,6 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         g.Ci = Ci.as<int64_t>();
         g.Cx = Cx.ptr;
         // 4. fused small-row kernel with the look-back scan over all rows
-        const int64_t ntiles = (m + FUSED_ROWS - 1) / FUSED_ROWS;
-        DevBuf status;
-        if (!status.alloc(sizeof(unsigned long long) * (ntiles + 1)))
-            return set_error(GM_OUT_OF_MEMORY, "saxpy3: scan status");
-        k_sx_fill_u64<<<sx_grid(ntiles + 1, 256, 1024), 256, 0, st>>>(
-            status.as<unsigned long long>(), ntiles + 1);
-        k_sx_fill_u64<<<1, 64, 0, st>>>((unsigned long long *) g.cnt + CNT_ERR, 1);
-        GM_HIP(hipGetLastError(), "k_sx_fill_u64");
         // B's rows: from its row records when the operand carries them (one
         // aligned run per gathered row, no row pointers); else as 16-byte
         // (column, value) pairs when its rows are gathered at least about once
@@ -1747,11 +1745,13 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             ProfScope ps("sx_fused");
             const int64_t gcap = (int64_t) cu_count() * 8 * 256 / FUSED_NT;
             const int64_t grid = ntiles < gcap ? ntiles : gcap;
-            unsigned long long *stp = status.as<unsigned long long>();
-            int *errp = (int *) (g.cnt + CNT_ERR);
+            unsigned long long *stp = g.cnt + SX_NCNT;
+            int64_t *host = (int64_t *) hp;         // nnz(C), look-back error
+            host[0] = 0;
+            host[1] = 0;
             const bool k32 = B->ncols <= ((int64_t) 1 << 26);
 #define GM_SX_FUSED(K, PKV) \
-    k_sx_fused<S, K, FUSED_NT, PKV><<<(unsigned) grid, FUSED_NT, 0, st>>>(g, fs, stp, ntiles, errp)
+    k_sx_fused<S, K, FUSED_NT, PKV><<<(unsigned) grid, FUSED_NT, 0, st>>>(g, fs, stp, ntiles, host)
             if constexpr (SX_PACK_OK<S>)
             {
                 if (pk == 2 && k32) GM_SX_FUSED(uint32_t, 2);
@@ -1764,12 +1764,9 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
 #undef GM_SX_FUSED
             GM_HIP(hipGetLastError(), "k_sx_fused");
         }
-        GM_HIP(hipMemcpyAsync(hp + 11, g.Cp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
-        GM_HIP(hipMemcpyAsync(hp + 12, g.cnt + CNT_ERR, sizeof(unsigned long long), hipMemcpyDeviceToHost, st),
-               "fused err");
         GM_HIP(hipStreamSynchronize(st), "fused sync");
-        if (hp[12] != 0) return set_error(GM_PANIC, "saxpy3: look-back scan did not complete");
-        nvals = (int64_t) hp[11];
+        if (hp[1] != 0) return set_error(GM_PANIC, "saxpy3: look-back scan did not complete");
+        nvals = (int64_t) hp[0];
         // 5. numeric phase of the big rows
         if (have_big && nvals > 0) GM_TRY((sx_launch_phase<S, 1>(g, hc, true)));
         if (hc[BIN_TIL] > 0 && nvals > 0) GM_TRY((sx_tile_run<S, 1>(g, tiles.t)));
