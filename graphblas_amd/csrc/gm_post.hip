@@ -317,7 +317,7 @@ __global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g)
 
 template <class Z>
 static int accum_mask_run(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bool mask_comp,
-                          bool mask_struct, bool replace, const gm_csr *T, int32_t op)
+                          bool mask_struct, bool replace, const gm_csr *T, int32_t op, int64_t nc, int64_t nt)
 {
     hipStream_t st = stream();
     const int64_t m = T->nrows;
@@ -338,10 +338,15 @@ static int accum_mask_run(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bool 
     g.op = op;
     int64_t *hp = (int64_t *) pinned_scratch(2 * sizeof(int64_t));
     if (!hp) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
-    hp[0] = 0;
-    if (g.Cp) GM_HIP(hipMemcpyAsync(hp, g.Cp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
-    GM_HIP(hipMemcpyAsync(hp + 1, g.Tp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(T)");
-    GM_HIP(hipStreamSynchronize(st), "accum sizes sync");
+    const bool known = nc >= 0 && nt >= 0;
+    hp[0] = g.Cp && known ? nc : 0;
+    hp[1] = nt;
+    if (!known)
+    {
+        if (g.Cp) GM_HIP(hipMemcpyAsync(hp, g.Cp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
+        GM_HIP(hipMemcpyAsync(hp + 1, g.Tp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(T)");
+        GM_HIP(hipStreamSynchronize(st), "accum sizes sync");
+    }
     g.nc = hp[0];
     g.nt = hp[1];
     g.ntc = g.nc / AC_TILE + 1;
@@ -474,6 +479,12 @@ extern "C" int gm_transpose(gm_csr_out *T, const gm_csr *A)
 extern "C" int gm_accum_mask(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bool mask_comp,
                              bool mask_struct, bool replace, const gm_csr *T, int32_t accum_op)
 {
+    return gm_accum_mask_sized(O, C, -1, M, mask_comp, mask_struct, replace, T, -1, accum_op);
+}
+
+extern "C" int gm_accum_mask_sized(gm_csr_out *O, const gm_csr *C, int64_t nc, const gm_csr *M, bool mask_comp,
+                                   bool mask_struct, bool replace, const gm_csr *T, int64_t nt, int32_t accum_op)
+{
     if (!O || !T || !T->p) return set_error(GM_INVALID_VALUE, "gm_accum_mask: NULL argument");
     if (C && C->p && (C->nrows != T->nrows || C->ncols != T->ncols || C->type != T->type))
         return set_error(GM_INVALID_VALUE, "gm_accum_mask: C and T differ in shape or type");
@@ -486,10 +497,10 @@ extern "C" int gm_accum_mask(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bo
     GM_TRY(ensure_init());
     switch (T->type)
     {
-        case GM_BOOL: return accum_mask_run<uint8_t>(O, C, M, mask_comp, mask_struct, replace, T, accum_op);
-        case GM_INT32: return accum_mask_run<int32_t>(O, C, M, mask_comp, mask_struct, replace, T, accum_op);
-        case GM_INT64: return accum_mask_run<int64_t>(O, C, M, mask_comp, mask_struct, replace, T, accum_op);
-        case GM_FP64: return accum_mask_run<double>(O, C, M, mask_comp, mask_struct, replace, T, accum_op);
+        case GM_BOOL: return accum_mask_run<uint8_t>(O, C, M, mask_comp, mask_struct, replace, T, accum_op, nc, nt);
+        case GM_INT32: return accum_mask_run<int32_t>(O, C, M, mask_comp, mask_struct, replace, T, accum_op, nc, nt);
+        case GM_INT64: return accum_mask_run<int64_t>(O, C, M, mask_comp, mask_struct, replace, T, accum_op, nc, nt);
+        case GM_FP64: return accum_mask_run<double>(O, C, M, mask_comp, mask_struct, replace, T, accum_op, nc, nt);
         default: return set_error(GM_NO_VALUE, "gm_accum_mask: type %d not supported", T->type);
     }
 }

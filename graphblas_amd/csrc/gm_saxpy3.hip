@@ -53,6 +53,7 @@ enum { CNT_SLOTS = 8,       // table slots of BIN_GLB
        CNT_SMALL = 10,      // flops of the small rows
        CNT_HFLOPS = 11,     // flops of BIN_HVY
        CNT_NNZA = 12,       // nnz(A)
+       CNT_BIGT = 13,       // most entries the big rows can have
        CNT_TILF = 14,       // BIN_TIL's very heavy rows (at the list's front; the others from its back)
        CNT_TILA = 15,       // A's entries in BIN_TIL's rows
        CNT_TILB = 22,       // BIN_TIL's other rows
@@ -238,6 +239,7 @@ namespace gm
 //------------------------------------------------------------------------------
 
 constexpr int TG = 8;          // lanes per row in the flop-count and fused kernels
+constexpr int64_t BIG_BOUND_MAX = (int64_t) 64 << 20;   // bytes of C held at the big rows' bound
 constexpr int FEW_ROWS = 256;             // A with at most this many rows: k_sx_rowflops
 constexpr int64_t FLOPS_TEAM_MAX = 256;   // longer rows of A: counted by the workgroup
 constexpr int FMAX = 64;       // largest flop count of a "small" row
@@ -344,8 +346,8 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
     __shared__ unsigned long long s_red[SX_NT / 64 + 1];
     __shared__ int s_long[SX_NT / TG], s_nlong;
     const int sub = threadIdx.x & (TG - 1);
-    const int lane = threadIdx.x & 63;
     unsigned long long fsum = 0;          // flops of this thread's small rows
+    unsigned long long bsum = 0;          // size bounds of its big rows
     if (blockIdx.x == 0 && threadIdx.x == 0) g.cnt[CNT_NNZA] = (unsigned long long) g.Ap[g.m];
     for (int64_t base = (int64_t) blockIdx.x * (SX_NT / TG); base < g.m;
          base += (int64_t) gridDim.x * (SX_NT / TG))
@@ -403,6 +405,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
             else if (t <= g.wl_max) bin = BIN_WL;
             else if (t <= g.blk_max && !sx_tiled(g, f, a1 - a0)) bin = BIN_BLK;
             else bin = BIN_HVY;
+            if (f > fs && t > 0) bsum += (unsigned long long) t;
         }
         __syncthreads();
         // block-aggregated appends: LDS counters, one global atomic per bin
@@ -424,16 +427,13 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
         }
         __syncthreads();
     }
-    // flops of small rows: one atomic per workgroup
-    #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) fsum += __shfl_xor(fsum, off, 64);
-    if (lane == 0) s_red[threadIdx.x >> 6] = fsum;
-    __syncthreads();
+    // one atomic per workgroup for each sum
+    fsum = block_sum<unsigned long long, SX_NT>(fsum, s_red);
+    bsum = block_sum<unsigned long long, SX_NT>(bsum, s_red);
     if (threadIdx.x == 0)
     {
-        unsigned long long tsum = 0;
-        for (int w = 0; w < SX_NT / 64; w++) tsum += s_red[w];
-        if (tsum) atomicAdd(&g.cnt[CNT_SMALL], tsum);
+        if (fsum) atomicAdd(&g.cnt[CNT_SMALL], fsum);
+        if (bsum) atomicAdd(&g.cnt[CNT_BIGT], bsum);
     }
 }
 
@@ -1701,6 +1701,14 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         if (have_big)
         {
             GM_TRY((sx_launch_phase<SxSym, 0>(g, hc, true)));
+            // the output's room for them: their bound while that is small, else
+            // their exact sum, at the price of a kernel and a wait (about 20 us a
+            // call; with the sizes accum_mask need not fetch, four hops of one
+            // source over 60000 vertices went from 1258 to 1157 us)
+            big_total = hc[CNT_BIGT];
+        }
+        if (have_big && (double) big_total * (double) entry_bytes > (double) BIG_BOUND_MAX)
+        {
             k_sx_sum_big<<<sx_grid(nbig, SX_NT, 512), SX_NT, 0, st>>>(g, dmax);
             GM_HIP(hipGetLastError(), "k_sx_sum_big");
             GM_HIP(hipMemcpyAsync(hp, g.cnt + CNT_BIGSUM, sizeof(unsigned long long),

@@ -413,7 +413,8 @@ GrB_Info GrB_mxm(GrB_Matrix C, const GrB_Matrix Mask, const GrB_BinaryOp accum,
             GB_free_out(&R);
             return GB_error(C, info, "%s", C->err);
         }
-        rc = gm_accum_mask(&O, &vc, Mask ? &vm : NULL, mask_comp, mstruct, C_replace, &vt, accum_op);
+        rc = gm_accum_mask_sized(&O, &vc, C->nvals, Mask ? &vm : NULL, mask_comp, mstruct, C_replace, &vt,
+                                 R.nvals, accum_op);
         GB_free_out(&R);
         if (rc != GM_SUCCESS) return GB_error(C, GB_from_gm(rc), "GrB_mxm: %s", gm_last_error());
         R = O;

@@ -376,6 +376,10 @@ int gm_transpose(gm_csr_out *T, const gm_csr *A);
 // 10 LOR, 11 LAND.  Outside the mask C's entries stay unless replace.
 int gm_accum_mask(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bool mask_comp,
                   bool mask_struct, bool replace, const gm_csr *T, int32_t accum_op);
+// the same for a caller that knows the entry counts of C and T (-1: read from
+// their row pointers, which takes a wait)
+int gm_accum_mask_sized(gm_csr_out *O, const gm_csr *C, int64_t c_nvals, const gm_csr *M, bool mask_comp,
+                        bool mask_struct, bool replace, const gm_csr *T, int64_t t_nvals, int32_t accum_op);
 
 //------------------------------------------------------------------------------
 // batches: many independent requests in one launch sequence (no counterpart
