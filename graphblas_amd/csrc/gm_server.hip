@@ -37,6 +37,7 @@
 #include <mutex>
 #include <thread>
 #include <unordered_map>
+#include <new>
 #include <vector>
 #include <cstring>
 
@@ -606,7 +607,9 @@ static int sv_copy_rows(const SvSlice &sl, int64_t k, int64_t *Cp, int64_t *Cj, 
         std::lock_guard<std::mutex> lk(h.mu);
         if (h.hp.empty())
         {
-            std::vector<int64_t> hp((size_t) C.nrows + 1);
+            std::vector<int64_t> hp;
+            try { hp.resize((size_t) C.nrows + 1); }
+            catch (const std::exception &) { return set_error(GM_OUT_OF_MEMORY, "fetch: row pointers"); }
             GM_TRY(gm_memcpy_d2h(hp.data(), C.p, sizeof(int64_t) * hp.size()));
             h.hp = std::move(hp);
         }
@@ -619,19 +622,27 @@ static int sv_copy_rows(const SvSlice &sl, int64_t k, int64_t *Cp, int64_t *Cj, 
         {
             if (!h.hj)
             {
-                std::unique_ptr<uint8_t[]> hj(new uint8_t[sizeof(int64_t) * all]), hx(new uint8_t[xs * all]);
-                hipStream_t st = stream();
-                GM_HIP(hipMemcpyAsync(hj.get(), C.j, sizeof(int64_t) * all, hipMemcpyDeviceToHost, st), "fetch j");
-                GM_HIP(hipMemcpyAsync(hx.get(), C.x, C.iso ? xs : xs * all, hipMemcpyDeviceToHost, st), "fetch x");
-                GM_HIP(hipStreamSynchronize(st), "fetch sync");
-                if (C.iso)
-                    for (int64_t t = 1; t < all; t++) memcpy(hx.get() + t * xs, hx.get(), xs);
-                h.hj = std::move(hj);
-                h.hx = std::move(hx);
+                // without the host memory each request is copied by itself below
+                std::unique_ptr<uint8_t[]> hj(new (std::nothrow) uint8_t[sizeof(int64_t) * all]);
+                std::unique_ptr<uint8_t[]> hx(new (std::nothrow) uint8_t[xs * all]);
+                if (hj && hx)
+                {
+                    hipStream_t st = stream();
+                    GM_HIP(hipMemcpyAsync(hj.get(), C.j, sizeof(int64_t) * all, hipMemcpyDeviceToHost, st), "fetch j");
+                    GM_HIP(hipMemcpyAsync(hx.get(), C.x, C.iso ? xs : xs * all, hipMemcpyDeviceToHost, st), "fetch x");
+                    GM_HIP(hipStreamSynchronize(st), "fetch sync");
+                    if (C.iso)
+                        for (int64_t t = 1; t < all; t++) memcpy(hx.get() + t * xs, hx.get(), xs);
+                    h.hj = std::move(hj);
+                    h.hx = std::move(hx);
+                }
             }
-            if (Cj) memcpy(Cj, h.hj.get() + sizeof(int64_t) * base, sizeof(int64_t) * nz);
-            if (Cx) memcpy(Cx, h.hx.get() + xs * base, xs * nz);
-            return GM_SUCCESS;
+            if (h.hj)
+            {
+                if (Cj) memcpy(Cj, h.hj.get() + sizeof(int64_t) * base, sizeof(int64_t) * nz);
+                if (Cx) memcpy(Cx, h.hx.get() + xs * base, xs * nz);
+                return GM_SUCCESS;
+            }
         }
     }
     hipStream_t st = stream();
