@@ -23,6 +23,11 @@
 //          one.  Lanes reduce in lane order (= k order), so fp64 sums are
 //          deterministic and ANY keeps the first match in k order, like the
 //          reference's sequential merge.
+//  short   when no row of either operand is long, one kernel without bins
+//          looks B's rows up in LDS tables of A's rows instead of phase1 and
+//          the teams (k_dot3_short).
+//  mates   when M, A and B are one symmetric pattern (a batch of C<A> = A*A'),
+//          C(i,j) = C(j,i) is computed once and stored twice.
 //  compact one pass per 2048-entry tile: block scan of the live flags, scatter
 //          of the surviving (j, value) pairs, and the new row pointers of all
 //          rows that start in the tile.  The result has no zombies.

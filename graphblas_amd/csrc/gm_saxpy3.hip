@@ -9,23 +9,29 @@
 //
 // Layout: all operands CSR in HBM.  C(i,:) = (+)_k A(i,k) (x) B(k,:).
 //
-//  flops   one thread per row: f = sum |B(k,:)|, table size t = f (or
+//  flops   eight lanes per row (the workgroup for a long row of A, the device
+//          for few rows): f = sum |B(k,:)|, table size t = f (or
 //          min(f, |M(i,:)|) for C<M>, and <= ncols).  Rows are binned:
 //            single  |A(i,:)| == 1: C(i,:) is B(k,:) filtered by the mask,
 //                    already sorted; no hash table at all
 //            wave S  t <= 64   : one wavefront, 128-slot LDS table
 //            wave L  t <= 512  : one wavefront, 1024-slot LDS table
 //            block   t <= 2048 : one 256-thread workgroup, 4096-slot table
-//            global  larger    : one workgroup, table of 2^ceil(log2 2t) slots
-//                                in HBM (sub-allocated by an atomic bump)
+//            heavy   larger    : dealt out by k_sx_classify to tiles of C's
+//                    columns in LDS (gm_sx_tile.h), to dense HBM tables that
+//                    the whole device updates (gm_sx_push.h), or to one
+//                    workgroup with a table of 2^ceil(log2 2t) slots in HBM
+//                    (sub-allocated by an atomic bump)
 //  symbolic  per row, hash-insert the allowed column indices, count new keys
 //            -> Cp[i]; device exclusive scan -> row pointers, nnz(C).
 //  numeric   the same inserts plus values; flops are enumerated in the
 //            reference's sequential order (k ascending over A(i,:), then j
-//            ascending over B(k,:)) and applied in that order (lane order
-//            inside a wavefront, wavefront order inside a workgroup), so
-//            fp64 results equal the reference's coarse-task sums bit for bit
-//            and ANY keeps the last writer, as GB_HX_UPDATE "z = t" does.
+//            ascending over B(k,:)).  fp64 sums apply them in that order (lanes
+//            that meet in a column go lowest first, wavefronts in turn), so
+//            they equal the reference's coarse-task sums bit for bit; where
+//            any order gives the same result (SX_ANY_ORDER) updates are
+//            atomics, and ANY keeps the largest k, the last writer, as
+//            GB_HX_UPDATE "z = t" does.
 //            Rows are then sorted in LDS (rank count / bitonic) and written
 //            to C: C is returned with sorted rows.
 //  Masks     M(i,j) is tested by binary search in the sorted row M(i,:).

@@ -22,8 +22,8 @@
 //
 // What bounds it: the atomics at L2 / memory, the gathers of B, and for few
 // rows the launches.  Second level of 64 searches on RMAT scale 20
-// (any_secondi, 1.9M entries of C): 53.6 ms with one workgroup per row, 1.36
-// ms here.
+// (any_secondi, 1.9M entries of C): 53.6 ms with one workgroup per row, 0.90
+// ms for the call here.
 #pragma once
 
 namespace gm
