@@ -26,8 +26,8 @@
 //  short   when no row of either operand is long, one kernel without bins
 //          looks B's rows up in LDS tables of A's rows instead of phase1 and
 //          the teams (k_dot3_short).
-//  mates   when M, A and B are one symmetric pattern (a batch of C<A> = A*A'),
-//          C(i,j) = C(j,i) is computed once and stored twice.
+//  mates   C<M> = A*A' with a structural, mostly symmetric M: C(i,j) = C(j,i)
+//          is computed once and stored twice.
 //  compact one pass per 2048-entry tile: block scan of the live flags, scatter
 //          of the surviving (j, value) pairs, and the new row pointers of all
 //          rows that start in the tile.  The result has no zombies.
@@ -854,15 +854,13 @@ __global__ __launch_bounds__(D3_NT) void k_dot3_phase1(Dot3Args g)
                 {
                     if (g.mate)
                     {
-                        // (j,i), if the mask allows it too, has this value: the
-                        // entry below the diagonal computes both
+                        // (j,i), if M holds it, has this value: the entry below
+                        // the diagonal computes both
                         uint32_t m = D3_ALONE;
                         if (i != j)
                         {
                             const int64_t m1 = g.Mp[j + 1], q = lower_bound(g.Mj, g.Mp[j], m1, i);
-                            if (q < m1 && g.Mj[q] == i &&
-                                (g.mask_struct || mask_true(g.Mx, q, g.msize, g.m_iso)))
-                                m = (uint32_t) q;
+                            if (q < m1 && g.Mj[q] == i) m = (uint32_t) q;
                         }
                         if (m != D3_ALONE && i < j) bin = 3;
                         else g.mate[p] = m;
@@ -2817,8 +2815,10 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         // C(i,j) = C(j,i) for one matrix (every multiplier here commutes): when a
         // sample of M's entries finds its transposed place three times in four,
         // one of each such pair is computed.  The search costs 3.7 ms for the 83M
-        // entries of a 256-graph batch and saves 14.6 ms of 46.0
-        const bool sym = g.one && Mnz >= ((int64_t) 1 << 16) && 4 * front->pairs >= 3 * SYM_SAMPLES;
+        // entries of a 256-graph batch and saves 14.6 ms of 46.0.  Structural
+        // masks only: with int32 mask values the search was paid without fewer
+        // entries in the bins (4096 graphs, 1.46e9 entries: 698 ms, 539 without)
+        const bool sym = g.one && g.mask_struct && Mnz >= ((int64_t) 1 << 16) && 4 * front->pairs >= 3 * SYM_SAMPLES;
         // group deferred entries by probed row: explicit, or by default for
         // masks large enough that the sort pays for itself
         const gm_dot3_params tu = dot3_tuned();
