@@ -166,8 +166,10 @@ __device__ __forceinline__ T dn_bcast(T v, int t)
     else return shfl_any<T>(v, t, G);
 }
 
-// rows of a sparse A with more than DN_HUB entries
+// rows of a sparse A with more than DN_HUB entries, among its first 2^32: the
+// list holds 32-bit row ids, and a row past them stays with its team
 constexpr int64_t DN_HUB = 512;
+constexpr int64_t DN_HUB_ROWS = (int64_t) 1 << 32;
 
 __global__ __launch_bounds__(DN_NT) void k_dn_hubs(const int64_t *__restrict__ Ap, int64_t m, uint32_t *list,
                                                    unsigned long long *cnt)
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const
             {
                 q0 = g.Ap[i];
                 q1 = g.Ap[i + 1];
-                if (q1 - q0 > DN_HUB) continue;           // done above
+                if (q1 - q0 > DN_HUB && i < DN_HUB_ROWS) continue;           // done above
             }
             else q1 = g.kdim;
         }
@@ -624,8 +626,9 @@ static int dn_mxm_run(gm_dense_out *C, const gm_csr *Ms, const gm_dense *Md, boo
             unsigned long long *ctr = g.nvals + 1;      // hub count, next hub item
             if (As)
             {
-                if (!hubs.alloc(sizeof(uint32_t) * g.m)) return set_error(GM_OUT_OF_MEMORY, "dense product: rows");
-                k_dn_hubs<<<dn_grid((g.m + DN_NT - 1) / DN_NT), DN_NT, 0, st>>>(g.Ap, g.m, hubs.as<uint32_t>(), ctr);
+                const int64_t hm = std::min(g.m, DN_HUB_ROWS);
+                if (!hubs.alloc(sizeof(uint32_t) * hm)) return set_error(GM_OUT_OF_MEMORY, "dense product: rows");
+                k_dn_hubs<<<dn_grid((hm + DN_NT - 1) / DN_NT), DN_NT, 0, st>>>(g.Ap, hm, hubs.as<uint32_t>(), ctr);
             }
 #define GM_DN_ROWS(L)                                                                        \
     case L:                                                                                  \

@@ -262,3 +262,37 @@ def test_saxbit_hub_rows(grb, handle, n):
         C = capi.Matrix(ZT[name], len(lens), n)
         capi.mxm_checked(C, None, handle, capi.Matrix.from_csr(A, vt), _matrix(B, fb, vt))
         assert_csr_equal(C.to_csr(), O.saxpy3(name, A, B), what=f"{handle} n={n} {fb}")
+
+
+def test_saxbit_hub_row_past_32_bits(grb):
+    """A hub row whose number needs 33 bits, with one bool column (34 GB of row
+    pointers): it is computed, and no row that its low bits name."""
+    import ctypes
+    print("[dense] hub row 2^32", flush=True)
+    L = capi.lib()
+    m, nz = (1 << 32) + 1, 600
+    p, j, x = L.gm_malloc(8 * (m + 1)), L.gm_malloc(8 * nz), L.gm_malloc(nz)
+    out = capi.GmDenseOut()
+    try:
+        if not (p and j and x):
+            pytest.skip("34 GB of device memory are not free")
+        tail, cols, ones = np.array([0, nz], dtype=np.int64), np.arange(nz, dtype=np.int64), np.ones(nz, dtype=np.uint8)
+        assert L.gm_memset(p, 0, 8 * (m + 1)) == 0
+        assert L.gm_memcpy_h2d(p + 8 * (m - 1), tail.ctypes.data, 16) == 0
+        assert L.gm_memcpy_h2d(j, cols.ctypes.data, cols.nbytes) == 0
+        assert L.gm_memcpy_h2d(x, ones.ctypes.data, nz) == 0
+        A, B = capi.GmCsr(), capi.GmDense(nz, 1, None, x, 0, 1)
+        A.nrows, A.ncols, A.p, A.j, A.x, A.iso, A.type = m, nz, p, j, x, 1, 1
+        sr = capi.GmSemiring(*SR["GxB_ANY_PAIR_BOOL"][1])
+        rc = L.gm_saxbit(ctypes.byref(out), None, None, False, True, ctypes.byref(A), None, None,
+                         ctypes.byref(B), ctypes.byref(sr), None)
+        assert rc == 0, capi.last_error()
+        got = np.zeros(2, dtype=np.int8)
+        assert L.gm_memcpy_d2h(got[:1].ctypes.data, out.b, 1) == 0
+        assert L.gm_memcpy_d2h(got[1:].ctypes.data, out.b + m - 1, 1) == 0
+        assert out.nvals == 1 and got.tolist() == [0, 1]
+    finally:
+        for q in (p, j, x, out.b, out.x):
+            if q:
+                L.gm_free(q)
+        L.gm_arena_trim()
