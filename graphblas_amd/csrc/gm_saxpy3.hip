@@ -159,6 +159,21 @@ template <class S>
 constexpr bool SX_ANY_ORDER = S::add == GM_ADD_MIN || S::add == GM_ADD_MAX || S::any_min_k || S::iso_out ||
                               (S::add == GM_ADD_PLUS && !std::is_same<typename S::Z, double>::value);
 
+// can t change a cell that holds cur?  A plain read of the cell may be stale:
+// it is then an earlier value, which t may seem to change and does not.  The
+// zeros are told apart by their bits, so that -0 is the smaller one whichever
+// comes first.
+template <class S>
+__device__ __forceinline__ bool sx_changes(typename S::Z cur, typename S::Z t)
+{
+    if constexpr (std::is_same<typename S::Z, double>::value)
+    {
+        if (S::add == GM_ADD_MIN ? cur < t : cur > t) return false;
+        return __builtin_bit_cast(uint64_t, cur) != __builtin_bit_cast(uint64_t, t);
+    }
+    else return S::upd(cur, t) != cur;
+}
+
 // *p = *p (+) t, atomically (SX_ANY_ORDER semirings; *p starts at the
 // identity, for ANY with the inner index at 0)
 template <class S>

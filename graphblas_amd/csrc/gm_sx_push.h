@@ -185,7 +185,7 @@ __device__ __forceinline__ void pu_update(const PushArgs &h, int64_t n, int64_t 
             {
                 if (!(*bw & bit)) atomicOr(bw, bit);
             }
-            else if (S::upd(cur, t) != cur) sx_atomic_upd<S>(c, t);
+            else if (sx_changes<S>(cur, t)) sx_atomic_upd<S>(c, t);
         }
     }
 }

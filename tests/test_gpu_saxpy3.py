@@ -338,3 +338,21 @@ def test_saxpy3_tiled_rows(grb, mask, ncols, handle):
     for mode in (1, 2):
         got = gm_saxpy3(handle, A, B, params=(8, 16, 32, mode), **kw)
         assert_csr_equal(got, ref, what=f"tiled {handle} mode={mode}")
+
+
+@pytest.mark.parametrize("first", [0.0, -0.0])
+def test_saxpy3_signed_zeros_any_order(grb, first):
+    """min_plus_fp64 entries whose least products are zeros of both signs, in a
+    row spread over the device: -0 wherever it comes among them, also when it
+    comes after every workgroup has put +0 there, as in the row's hash table."""
+    print(f"[saxpy3] signed zeros, {first} first", flush=True)
+    K, n = 140000, 64
+    # A(i,k) + B(k,j) is -0 only where both are -0
+    A = W.Csr(1, K, np.array([0, K]), np.arange(K), np.full(K, -0.0))
+    x = np.full((K, n), first)
+    x[-5000:] = -first
+    B = W.Csr(K, n, np.arange(K + 1, dtype=np.int64) * n, np.tile(np.arange(n), K), x.ravel())
+    for table in (0, 1):                     # spread over the device, one hash table
+        got = gm_saxpy3("GrB_MIN_PLUS_SEMIRING_FP64", A, B, params=(8, 16, 32, 2, table))
+        assert len(got.x) == n and np.all(got.x == 0)
+        assert np.all(np.signbit(got.x)), f"table {table}: +0 in {int((~np.signbit(got.x)).sum())} entries"
