@@ -159,6 +159,19 @@ template <class S>
 constexpr bool SX_ANY_ORDER = S::add == GM_ADD_MIN || S::add == GM_ADD_MAX || S::any_min_k || S::iso_out ||
                               (S::add == GM_ADD_PLUS && !std::is_same<typename S::Z, double>::value);
 
+// what an accumulator of the any-order updates holds before its first product:
+// the identity, or for fp64 MIN / MAX the NaN that the updates below replace
+// with any number, so that products which are all NaN leave a NaN and not an
+// infinity (as an entry's first product does elsewhere, which fmin / fmax
+// then keep only among NaNs)
+template <class S>
+__device__ __forceinline__ typename S::Z sx_cell0()
+{
+    if constexpr (std::is_same<typename S::Z, double>::value && (S::add == GM_ADD_MIN || S::add == GM_ADD_MAX))
+        return __builtin_bit_cast(double, S::add == GM_ADD_MIN ? 0x7ff8000000000000ull : 0xfff8000000000000ull);
+    else return S::identity();
+}
+
 // can t change a cell that holds cur?  A plain read of the cell may be stale:
 // it is then an earlier value, which t may seem to change and does not.  The
 // zeros are told apart by their bits, so that -0 is the smaller one whichever
@@ -174,8 +187,7 @@ __device__ __forceinline__ bool sx_changes(typename S::Z cur, typename S::Z t)
     else return S::upd(cur, t) != cur;
 }
 
-// *p = *p (+) t, atomically (SX_ANY_ORDER semirings; *p starts at the
-// identity, for ANY with the inner index at 0)
+// *p = *p (+) t, atomically (SX_ANY_ORDER semirings; *p starts at sx_cell0)
 template <class S>
 __device__ __forceinline__ void sx_atomic_upd(typename S::Z *p, typename S::Z t)
 {
@@ -185,7 +197,8 @@ __device__ __forceinline__ void sx_atomic_upd(typename S::Z *p, typename S::Z t)
     else if constexpr (std::is_same<Z, double>::value)
     {
         // fmin / fmax of the bits: a NaN changes nothing; doubles of one sign
-        // order as their bits do (negative ones in reverse)
+        // order as their bits do (negative ones in reverse), with sx_cell0
+        // beyond the infinity of its sign
         if (t != t) return;
         const long long b = __builtin_bit_cast(long long, t);
         const bool neg = b < 0;
@@ -664,7 +677,7 @@ __device__ void sx_row(const SxArgs &g, int64_t i, uint32_t *keys, typename S::Z
     for (int64_t t = tid; t < T; t += NT)
     {
         keys[t] = SX_EMPTY;
-        if (PHASE) vals[t] = S::identity();
+        if (PHASE) vals[t] = SX_ANY_ORDER<S> ? sx_cell0<S>() : S::identity();
     }
     if constexpr (PHASE == 1 && !SX_ANY_ORDER<S>)
         for (int t = lane; t < SX_OWN; t += 64) own[t] = 0xffffffffu;

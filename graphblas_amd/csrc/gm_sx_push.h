@@ -17,8 +17,9 @@
 //   write    the cells in column order, so nothing is sorted
 //
 // Cells hold the largest inner index + 1 (ANY), a count (PLUS_PAIR), or the
-// value with the identity for "none"; a bit per column says present where the
-// cell cannot (PLUS_TIMES, ANY_PAIR, a product equal to the identity).
+// value with sx_cell0 for "none"; a bit per column says present where the cell
+// cannot (PLUS_TIMES, ANY_PAIR, an integer product equal to the identity, a
+// NaN).
 //
 // What bounds it: the atomics at L2 / memory, the gathers of B, and for few
 // rows the launches.  Second level of 64 searches on RMAT scale 20
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(PU_NT) void k_sx_push_init(PushArgs h, int64_t cell
     if constexpr (!S::iso_out)
     {
         PuCell<S> *tab = (PuCell<S> *) h.tab;
-        const PuCell<S> id = PU_U32<S> ? (PuCell<S>) 0 : (PuCell<S>) S::identity();
+        const PuCell<S> id = PU_U32<S> ? (PuCell<S>) 0 : (PuCell<S>) sx_cell0<S>();
         for (int64_t t = t0; t < cells; t += stride) tab[t] = id;
     }
     if constexpr (PU_BITS<S>)
@@ -179,9 +180,9 @@ __device__ __forceinline__ void pu_update(const PushArgs &h, int64_t n, int64_t 
         }
         else
         {
-            // a product equal to the identity (or a NaN) leaves the cell as it is
+            // a NaN, or an integer equal to the identity, leaves the cell as it is
             const Z cur = *c;
-            if (t != t || t == S::identity())
+            if (t != t || t == sx_cell0<S>())
             {
                 if (!(*bw & bit)) atomicOr(bw, bit);
             }
@@ -281,7 +282,8 @@ __device__ __forceinline__ bool pu_present(const PushArgs &h, int64_t n, int64_t
         else
         {
             z = ((const Z *) h.tab)[d * n + j];
-            return bit || (S::add != GM_ADD_PLUS && !h.all_bits && z != S::identity());
+            if constexpr (std::is_same<Z, double>::value) return bit || (S::add != GM_ADD_PLUS && !h.all_bits && z == z);
+            else return bit || (S::add != GM_ADD_PLUS && !h.all_bits && z != sx_cell0<S>());
         }
     }
 }

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(TL_NT) void k_sx_tile(SxArgs g, TileArgs t)
             if constexpr (PHASE == 0)
                 for (int x = lane; x < NW; x += 64) { s_bits[wv][x] = 0; s_mask[wv][x] = 0; }
             if constexpr (VALS)
-                for (int x = lane; x < TL_W; x += 64) s_acc[wv][x] = S::identity();
+                for (int x = lane; x < TL_W; x += 64) s_acc[wv][x] = SX_ANY_ORDER<S> ? sx_cell0<S>() : S::identity();
             wave_sync();
             for (int64_t ea = a0; (PHASE == 0 || VALS) && ea < a1; ea += 64)
             {

@@ -356,3 +356,39 @@ def test_saxpy3_signed_zeros_any_order(grb, first):
         got = gm_saxpy3("GrB_MIN_PLUS_SEMIRING_FP64", A, B, params=(8, 16, 32, 2, table))
         assert len(got.x) == n and np.all(got.x == 0)
         assert np.all(np.signbit(got.x)), f"table {table}: +0 in {int((~np.signbit(got.x)).sum())} entries"
+
+
+def _nan_values(rng, A, B):
+    """min_plus values with NaN, so that a column of A*B has only NaN products,
+    some, or none, and columns whose numbers are all +inf."""
+    A.x[rng.random(A.nnz) < 0.1] = np.nan
+    B.x[B.j % 3 == 0] = np.nan
+    B.x[(B.j % 3 == 1) & (rng.random(B.nnz) < 0.6)] = np.nan
+    B.x[(B.j % 7 == 2) & ~np.isnan(B.x)] = np.inf
+    B.x[rng.random(B.nnz) < 0.1] *= -1.0
+
+
+@pytest.mark.parametrize("table", [0, 1])
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("shape", ["few rows", "many rows"])
+@pytest.mark.parametrize("bins", [(0, 0, 0), (8, 16, 32)])
+def test_saxpy3_nan_products(grb, shape, bins, mode, table):
+    """min_plus_fp64 with NaN products through the small rows' sort, the LDS
+    and HBM hash tables, the tiles and the rows spread over the device: a NaN
+    is ignored, and an entry whose products are all NaN is NaN."""
+    print(f"[saxpy3] NaN {shape} bins={bins} mode={mode} table={table}", flush=True)
+    rng = np.random.default_rng(len(shape) + mode)
+    if shape == "few rows":
+        A = rand_csr(6, 900, 0.6, rng, "fp64")
+        B = rand_csr(900, 2100, 0.01, rng, "fp64")
+    else:
+        A = power_law_csr(2000, 40, rng, values="fp64")
+        B = rand_csr(2000, 4100, 0.001, rng, "fp64")
+    _nan_values(rng, A, B)
+    ref = O.saxpy3("min_plus_fp64", A, B)
+    nan = np.isnan(ref.x)
+    assert nan.any() and (~nan).any() and np.isinf(ref.x).any()
+    got = gm_saxpy3("GrB_MIN_PLUS_SEMIRING_FP64", A, B, params=tuple(bins) + (mode, table))
+    assert np.array_equal(got.p, ref.p) and np.array_equal(got.j, ref.j)
+    assert np.array_equal(got.x, ref.x, equal_nan=True), \
+        f"{int(np.isnan(got.x).sum())} NaN entries, {int(nan.sum())} expected"

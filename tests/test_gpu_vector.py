@@ -133,3 +133,26 @@ def test_vxm_bt(grb, handle, shape, comp):
     for d in (dU, dB, dM):
         if d:
             d.free()
+
+
+def test_vxm_nan_products_both_ways(grb):
+    """min_plus_fp64 over NaN products: u'*B' read as held and u'*C with C = B'
+    held by rows agree, an entry whose products are all NaN is NaN."""
+    rng = np.random.default_rng(17)
+    B = rand_csr(400, 3000, 0.05, rng, "fp64")
+    B.x[rng.random(B.nnz) < 0.7] = np.nan
+    rows = np.repeat(np.arange(400), np.diff(B.p))
+    B.x[rows % 3 == 0] = np.nan
+    ui = np.sort(rng.choice(3000, 2000, replace=False))
+    ux = rng.random(2000)
+    u = capi.Vector.from_arrays(ui, ux, "fp64", 3000)
+    ref = O.saxpy3("min_plus_fp64", _row(ui, ux, 3000), O.transpose(B))
+    assert np.isnan(ref.x).any() and (~np.isnan(ref.x)).any()
+    Bd, Bt = capi.Matrix.from_csr(B, "fp64"), capi.Matrix.from_csr(O.transpose(B), "fp64")
+    for what, call in (("mxv", lambda w: capi.mxv(w, None, "GrB_MIN_PLUS_SEMIRING_FP64", Bd, u)),
+                       ("vxm", lambda w: capi.vxm(w, None, "GrB_MIN_PLUS_SEMIRING_FP64", u, Bt))):
+        w = capi.Vector("fp64", 400)
+        assert call(w) == 0, capi.last_error()
+        got = _got(w, 400)
+        assert np.array_equal(got.j, ref.j), what
+        assert np.array_equal(got.x, ref.x, equal_nan=True), what
