@@ -332,7 +332,8 @@ GrB_Info GrB_mxm(GrB_Matrix C, const GrB_Matrix Mask, const GrB_BinaryOp accum,
         if (pulled && GB_burble)
             printf("burble: GrB_mxm C%s=A*B' %s: one row, B as held (%lld entries)\n", Mask ? "<!M>" : "",
                    GB_sr_name(&sr, nm, sizeof(nm)), (long long) B->nvals);
-        if (rc != GM_SUCCESS && rc != GM_NO_VALUE)
+        // a shape it does not take, or no room for its dense vectors: B' and saxpy3
+        if (rc != GM_SUCCESS && rc != GM_NO_VALUE && rc != GM_OUT_OF_MEMORY)
         {
             GB_free_out(&AT);
             return GB_error(C, GB_from_gm(rc), "GrB_mxm: %s", gm_last_error());

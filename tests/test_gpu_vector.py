@@ -156,3 +156,25 @@ def test_vxm_nan_products_both_ways(grb):
         got = _got(w, 400)
         assert np.array_equal(got.j, ref.j), what
         assert np.array_equal(got.x, ref.x, equal_nan=True), what
+
+
+def test_mxv_without_room_for_dense_vectors(grb):
+    """An allocation forced to fail anywhere in the product that reads B as
+    held: B is transposed instead and the result is the same."""
+    rng = np.random.default_rng(23)
+    B = rand_csr(300, 500, 0.05, rng, "int64")
+    Bd = capi.Matrix.from_csr(B, "int64")
+    ui = np.sort(rng.choice(500, 200, replace=False))
+    ux = rng.integers(-9, 10, 200)
+    u = capi.Vector.from_arrays(ui, ux, "int64", 500)
+    ref = O.saxpy3("plus_times_int64", _row(ui, ux, 500), O.transpose(B))
+    L = capi.lib()
+    for n in range(8):
+        w = capi.Vector("int64", 300)
+        L.gm_debug_fail_after(n)
+        try:
+            rc = capi.mxv(w, None, "GrB_PLUS_TIMES_SEMIRING_INT64", Bd, u)
+        finally:
+            L.gm_debug_fail_after(-1)
+        assert rc == 0, f"allocation {n}: {capi.last_error()}"
+        assert_csr_equal(_got(w, 300), ref, what=f"allocation {n}")
