@@ -92,20 +92,30 @@ def test_vxm_transposed_with_accum_and_mask(grb):
     assert_csr_equal(_got(w, 80), ref, what="w<m> += u'A'")
 
 
+def _mostly_empty(rng):
+    """Row lengths: 70001 rows, 1 to 3 entries in 2400 of them, some long ones,
+    one longer than a chunk, the last row empty."""
+    lens = np.zeros(70001, dtype=np.int64)
+    lens[rng.choice(70000, 2400, replace=False)] = rng.integers(1, 4, 2400)
+    lens[[0, 17, 30000, 50000, 60000, 69999]] = [1, 65, 3000, 64, 100, 200]
+    return lens
+
+
 @pytest.mark.parametrize("comp", [False, True])
-@pytest.mark.parametrize("shape", ["one row", "short", "hub", "chunk"])
+@pytest.mark.parametrize("shape", ["one row", "short", "hub", "chunk", "empty rows"])
 @pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GxB_PLUS_PAIR_INT32", "GxB_ANY_PAIR_BOOL",
                                     "GxB_ANY_SECONDI_INT64", "GrB_PLUS_TIMES_SEMIRING_INT64",
                                     "GrB_MIN_PLUS_SEMIRING_INT32", "GrB_MAX_PLUS_SEMIRING_INT32",
                                     "GrB_MIN_PLUS_SEMIRING_FP64", "GrB_PLUS_TIMES_SEMIRING_FP64"])
 def test_vxm_bt(grb, handle, shape, comp):
     """u'*B' without a transpose: one row, many short and empty rows, rows that
-    span several chunks of 2048 entries, and rows that end where a chunk ends."""
+    span several chunks of 2048 entries, rows that end where a chunk ends, and
+    chunks that span more empty rows than a workgroup walks."""
     print(f"[vector] vxm_bt {handle} {shape} comp={comp}", flush=True)
     rng = np.random.default_rng(len(handle) + len(shape))
     K = 9000
     lens = {"one row": [4096], "short": rng.integers(0, 9, 3000), "chunk": [2048, 0, 1, 2047, 64, 65, 1919, 2048],
-            "hub": np.where(np.arange(300) % 97 == 5, 8500, rng.integers(0, 40, 300))}[shape]
+            "empty rows": _mostly_empty(rng), "hub": np.where(np.arange(300) % 97 == 5, 8500, rng.integers(0, 40, 300))}[shape]
     p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
     j = np.concatenate([np.sort(rng.choice(K, size=int(l), replace=False)) for l in lens]).astype(np.int64)
     n, name = len(lens), SR[handle][0]
@@ -178,3 +188,26 @@ def test_mxv_without_room_for_dense_vectors(grb):
             L.gm_debug_fail_after(-1)
         assert rc == 0, f"allocation {n}: {capi.last_error()}"
         assert_csr_equal(_got(w, 300), ref, what=f"allocation {n}")
+
+
+def test_mxv_empty_rows_cost(grb):
+    """Empty rows are not walked one workgroup at a time: 2000 entries in 2^24
+    rows take at most 10 times a call on 2^12 rows (2.3 times as measured)."""
+    import time
+    best = {}
+    for lg in (12, 24):
+        n, rng = 1 << lg, np.random.default_rng(lg)
+        key = np.sort(rng.choice(n, 2000, replace=False))
+        B = W.Csr(n, n, np.searchsorted(key, np.arange(n + 1)).astype(np.int64), rng.permutation(key), rng.random(2000))
+        Bd = capi.Matrix.from_csr(B, "fp64")
+        u = capi.Vector.from_arrays(key, np.ones(2000), "fp64", n)
+        w = capi.Vector("fp64", n)
+        ts = []
+        for _ in range(8):
+            t = time.perf_counter()
+            assert capi.mxv(w, None, "GrB_PLUS_TIMES_SEMIRING_FP64", Bd, u) == 0, capi.last_error()
+            ts.append(time.perf_counter() - t)
+        best[lg] = min(ts)
+        got = _got(w, n)
+        assert np.array_equal(got.j, key) and np.array_equal(got.x, B.x)
+    assert best[24] <= 10 * best[12], best
