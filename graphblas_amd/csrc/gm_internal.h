@@ -54,6 +54,16 @@ struct DevBuf
     void *release() { void *p = ptr; ptr = nullptr; return p; }
 };
 
+// Results may be written at their bound while that is at most this many bytes;
+// a larger one waits for its entry count first.
+constexpr int64_t OUT_BOUND_MAX = (int64_t) 64 << 20;
+
+// b, allocated at `cap` bytes, holds `used`: moved to a block of that size if
+// the rest is more than 1 MB and more than what is used, so that an object
+// keeps at most twice its entries.  True if a copy was queued on the library
+// stream; without room b stays as it is.
+bool fit_block(DevBuf &b, size_t used, size_t cap);
+
 // pinned host staging for small device->host reads
 void *pinned_scratch(size_t bytes);
 

@@ -17,6 +17,7 @@
 #include "gm_internal.h"
 #include "gm_block.h"
 
+#include <algorithm>
 #include <mutex>
 #include <map>
 #include <unordered_map>
@@ -210,6 +211,20 @@ void *pinned_scratch(size_t bytes)
     if (hipHostMalloc(&g_pinned, want, hipHostMallocDefault) != hipSuccess) return nullptr;
     g_pinned_bytes = want;
     return g_pinned;
+}
+
+bool fit_block(DevBuf &b, size_t used, size_t cap)
+{
+    if (cap - used <= std::max(used, (size_t) 1 << 20)) return false;
+    DevBuf t;
+    if (!t.alloc(used)) return false;
+    if (used > 0 && hipMemcpyAsync(t.ptr, b.ptr, used, hipMemcpyDeviceToDevice, stream()) != hipSuccess)
+    {
+        (void) hipGetLastError();
+        return false;
+    }
+    std::swap(t.ptr, b.ptr);
+    return true;
 }
 
 //------------------------------------------------------------------------------

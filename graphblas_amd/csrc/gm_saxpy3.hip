@@ -273,7 +273,6 @@ namespace gm
 //------------------------------------------------------------------------------
 
 constexpr int TG = 8;          // lanes per row in the flop-count and fused kernels
-constexpr int64_t BIG_BOUND_MAX = (int64_t) 64 << 20;   // bytes of C held at the big rows' bound
 constexpr int FEW_ROWS = 256;             // A with at most this many rows: k_sx_rowflops
 constexpr int64_t FLOPS_TEAM_MAX = 256;   // longer rows of A: counted by the workgroup
 constexpr int FMAX = 64;       // largest flop count of a "small" row
@@ -1726,7 +1725,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     push.h.dflops = dflops;
     if constexpr (SX_ANY_ORDER<S>)
         if (hc[BIN_DNS] > 0) GM_TRY(sx_push_build<S>(g, push, hc[BIN_DNS], hc[CNT_NNZA], hc[CNT_HFLOPS]));
-    int64_t nvals = 0;
+    int64_t nvals = 0, held = 0;        // held: entries C has room for, if at the big rows' bound and small
     DevBuf Ci, Cx;
     if (fused)
     {
@@ -1741,7 +1740,8 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             // source over 60000 vertices went from 1258 to 1157 us)
             big_total = hc[CNT_BIGT];
         }
-        if (have_big && (double) big_total * (double) entry_bytes > (double) BIG_BOUND_MAX)
+        const bool at_bound = have_big && (double) big_total * (double) entry_bytes <= (double) OUT_BOUND_MAX;
+        if (have_big && !at_bound)
         {
             k_sx_sum_big<<<sx_grid(nbig, SX_NT, 512), SX_NT, 0, st>>>(g, dmax);
             GM_HIP(hipGetLastError(), "k_sx_sum_big");
@@ -1751,6 +1751,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
             big_total = (int64_t) hp[0];
         }
         const int64_t cap = cap_small + big_total;
+        if (at_bound && (double) cap * (double) entry_bytes <= 2.0 * (double) OUT_BOUND_MAX) held = cap;
         if (!Ci.alloc(sizeof(int64_t) * (cap > 0 ? cap : 1)) ||
             !Cx.alloc(S::iso_out ? zs : zs * (cap > 0 ? cap : 1)))
             return set_error(GM_OUT_OF_MEMORY, "saxpy3: output (%lld entries)", (long long) cap);
@@ -1838,6 +1839,11 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
         k_sx_iso_one<<<1, 1, 0, st>>>(Cx.ptr, (int) zs);
         GM_HIP(hipGetLastError(), "k_sx_iso_one");
     }
+    if (held > 0)
+    {
+        (void) fit_block(Ci, sizeof(int64_t) * nvals, sizeof(int64_t) * held);
+        if (!S::iso_out) (void) fit_block(Cx, zs * nvals, zs * held);
+    }
     GM_HIP(hipStreamSynchronize(st), "saxpy3 sync");
     C->nrows = m;
     C->ncols = n;
@@ -1882,13 +1888,21 @@ static int vxm_bt_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm
     // its 32-bit cells
     const int64_t words = 2 + kw + (M ? nw : 0) + (PU_U32<S> ? n : nw);
     DevBuf Cp, Ci, Cx, zero, val, tab, part, seg;
-    if (!Cp.alloc(2 * sizeof(int64_t)) || !Ci.alloc(sizeof(int64_t) * n) ||
-        !Cx.alloc(S::iso_out ? sizeof(Z) : sizeof(Z) * n) || !zero.alloc(sizeof(uint32_t) * (words + 1)) ||
+    // the result at its bound of n entries, or once they are counted
+    const size_t xs = S::iso_out ? 0 : sizeof(Z);
+    const bool bound = n * (int64_t) (sizeof(int64_t) + xs) <= OUT_BOUND_MAX;
+    auto result = [&](int64_t entries) {
+        if (!Ci.alloc(sizeof(int64_t) * entries) || !Cx.alloc(S::iso_out ? sizeof(Z) : sizeof(Z) * entries)) return false;
+        g.Ci = Ci.as<int64_t>();
+        g.Cx = Cx.ptr;
+        return true;
+    };
+    if (!Cp.alloc(2 * sizeof(int64_t)) || (bound && !result(n)) || !zero.alloc(sizeof(uint32_t) * (words + 1)) ||
         (!S::pattern && !val.alloc(sizeof(Z) * k)) || (!PU_U32<S> && !S::iso_out && !tab.alloc(sizeof(Z) * n)) ||
         !part.alloc((size_t) p.nch * (2 * sizeof(Z) + sizeof(int64_t) + 2) + 8) ||
         !seg.alloc(sizeof(int64_t) * (h.nseg + 1)))
         return set_error(GM_OUT_OF_MEMORY, "one-row product: workspace");
-    g.Cp = Cp.as<int64_t>(); g.Ci = Ci.as<int64_t>(); g.Cx = Cx.ptr;
+    g.Cp = Cp.as<int64_t>();
     uint32_t *w = zero.as<uint32_t>();
     h.drow = w;
     p.ubits = w + 2;
@@ -1916,12 +1930,25 @@ static int vxm_bt_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm
         k_sx_push_count<S><<<sx_grid(h.nseg, 1, cap), PU_NT, 0, st>>>(g, h);
         GM_TRY(scan_exclusive_i64(h.seg, h.seg, h.nseg));
         k_pull_ptr<<<1, 64, 0, st>>>(g.Cp, h.seg, h.nseg);
+        if (!bound)
+        {
+            GM_HIP(hipMemcpyAsync(hp, g.Cp + 1, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
+            GM_HIP(hipStreamSynchronize(st), "one-row product nnz sync");
+            if (!result(hp[0]))
+                return set_error(GM_OUT_OF_MEMORY, "one-row product: output (%lld entries)", (long long) hp[0]);
+        }
         k_sx_push_write<S><<<sx_grid(h.nseg, 1, cap), PU_NT, 0, st>>>(g, h);
         if (S::iso_out) k_sx_iso_one<<<1, 1, 0, st>>>(Cx.ptr, (int) sizeof(Z));
         GM_HIP(hipGetLastError(), "one-row product");
     }
     GM_HIP(hipMemcpyAsync(hp, g.Cp + 1, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
     GM_HIP(hipStreamSynchronize(st), "one-row product sync");
+    if (bound)
+    {
+        bool moved = fit_block(Ci, sizeof(int64_t) * hp[0], sizeof(int64_t) * n);
+        moved |= fit_block(Cx, xs * hp[0], xs * n);
+        if (moved) GM_HIP(hipStreamSynchronize(st), "one-row product fit sync");
+    }
     C->nrows = 1;
     C->ncols = n;
     C->nvals = hp[0];

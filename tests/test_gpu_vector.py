@@ -211,3 +211,38 @@ def test_mxv_empty_rows_cost(grb):
         got = _got(w, n)
         assert np.array_equal(got.j, key) and np.array_equal(got.x, B.x)
     assert best[24] <= 10 * best[12], best
+
+
+@pytest.mark.parametrize("handle", ["GrB_PLUS_TIMES_SEMIRING_FP64", "GxB_ANY_PAIR_BOOL"])
+@pytest.mark.parametrize("lg", [18, 22, 23])
+def test_mxv_result_memory(grb, lg, handle):
+    """A sparse result of a long one-row product keeps about its entries'
+    memory, below and above the size that is written at its bound (2^22 fp64
+    entries), also as the product of a spread row."""
+    n, L = 1 << lg, capi.lib()
+    rng = np.random.default_rng(lg)
+    vt = "fp64" if "FP64" in handle else "bool"
+    key = np.sort(rng.choice(n, 2000, replace=False))
+    one = np.ones(2000, dtype=np.float64 if vt == "fp64" else bool)
+    B = W.Csr(n, n, np.searchsorted(key, np.arange(n + 1)).astype(np.int64), rng.permutation(key),
+              rng.random(2000) if vt == "fp64" else one.astype(np.uint8))
+    Bd = capi.Matrix.from_csr(B, vt)
+    u = capi.Vector.from_arrays(key, one, vt, n)
+    w = capi.Vector(vt, n)
+    before = L.gm_arena_bytes_in_use()
+    assert capi.mxv(w, None, handle, Bd, u) == 0, capi.last_error()
+    held = L.gm_arena_bytes_in_use() - before
+    got = _got(w, n)
+    assert np.array_equal(got.j, key) and (vt == "bool" or np.array_equal(got.x, B.x))
+    assert held <= 5 << 20, f"{held} bytes for 2000 entries"
+    # 50000 rows with the same 40 columns: 2 million products, 40 entries
+    D = W.Csr(50000, n, np.arange(50001) * 40, np.tile(np.arange(40) * (n // 40), 50000),
+              rng.random(2000000) if vt == "fp64" else np.ones(2000000, dtype=np.uint8))
+    Dd = capi.Matrix.from_csr(D, vt)
+    v = capi.Vector.from_arrays(np.arange(50000), np.ones(50000, dtype=one.dtype), vt, 50000)
+    w = capi.Vector(vt, n)
+    before = L.gm_arena_bytes_in_use()
+    assert capi.vxm(w, None, handle, v, Dd) == 0, capi.last_error()
+    held = L.gm_arena_bytes_in_use() - before
+    assert np.array_equal(_got(w, n).j, np.arange(40) * (n // 40))
+    assert held <= 5 << 20, f"{held} bytes for 40 entries"
