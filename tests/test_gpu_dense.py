@@ -296,3 +296,29 @@ def test_saxbit_hub_row_past_32_bits(grb):
             if q:
                 L.gm_free(q)
         L.gm_arena_trim()
+
+
+@pytest.mark.parametrize("fa", ["sparse", "bitmap"])
+def test_saxbit_few_long_rows_cost(grb, fa):
+    """16 long rows of A spread over the device: at most four times one row's
+    time (1.0 times as measured, 16 on one workgroup), and the same values."""
+    import time
+    rng = np.random.default_rng(3)
+    k, n = (100000, 64) if fa == "sparse" else (20000, 64)
+    x = rng.random(k)
+    B = capi.Matrix.from_dense(rng.random((k, n)), None, "fp64")
+    best, rows = {}, {}
+    for m in (1, 16):
+        if fa == "sparse":
+            A = capi.Matrix.from_csr(Csr(m, k, np.arange(m + 1, dtype=np.int64) * k, np.tile(np.arange(k), m),
+                                         np.tile(x, m)), "fp64")
+        else:
+            A = capi.Matrix.from_dense(np.tile(x, (m, 1)), np.ones((m, k), dtype=bool), "fp64")
+        C, ts = capi.Matrix("fp64", m, n), []
+        for _ in range(5):
+            t = time.perf_counter()
+            capi.mxm_checked(C, None, "GrB_PLUS_TIMES_SEMIRING_FP64", A, B)
+            ts.append(time.perf_counter() - t)
+        best[m], rows[m] = min(ts), C.to_dense()[0]
+    assert np.array_equal(rows[16], np.tile(rows[1], (16, 1)))
+    assert best[16] <= 4 * best[1], best
