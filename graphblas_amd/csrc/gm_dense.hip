@@ -178,6 +178,20 @@ __global__ __launch_bounds__(DN_NT) void k_dn_hubs(const int64_t *__restrict__ A
         if (Ap[i + 1] - Ap[i] > DN_HUB) list[atomicAdd(cnt, 1ull)] = (uint32_t) i;
 }
 
+// does the mask allow entry (i,c)
+__device__ __forceinline__ bool dn_allowed(const DnArgs &g, int64_t i, int64_t c)
+{
+    const int64_t d = i * g.n + c;
+    bool in;
+    if (g.mkind == 2) in = (!g.Mb || g.Mb[d] != 0) && (g.mstruct || dn_mask_value(g.Mx, d, g.msize, g.m_iso));
+    else
+    {
+        const int64_t m1 = g.Mp[i + 1], q = lower_bound(g.Mj, g.Mp[i], m1, c);
+        in = q < m1 && g.Mj[q] == c && (g.mstruct || dn_mask_value(g.Mx, q, g.msize, g.m_iso));
+    }
+    return in != (g.mcomp != 0);
+}
+
 // the result of entry (i,c): stored; returns 1 if C holds it
 template <class S>
 __device__ __forceinline__ int dn_put(const DnArgs &g, int64_t i, int64_t c, bool e, typename S::Z z)
@@ -190,17 +204,6 @@ __device__ __forceinline__ int dn_put(const DnArgs &g, int64_t i, int64_t c, boo
         const Z cin = ((const Z *) g.Cin)[d];
         ((Z *) g.Cx)[d] = e ? S::upd(cin, z) : cin;
         return 1;
-    }
-    if (e && g.mkind)
-    {
-        bool in;
-        if (g.mkind == 2) in = (!g.Mb || g.Mb[d] != 0) && (g.mstruct || dn_mask_value(g.Mx, d, g.msize, g.m_iso));
-        else
-        {
-            const int64_t m1 = g.Mp[i + 1], q = lower_bound(g.Mj, g.Mp[i], m1, c);
-            in = q < m1 && g.Mj[q] == c && (g.mstruct || dn_mask_value(g.Mx, q, g.msize, g.m_iso));
-        }
-        e = in != (g.mcomp != 0);
     }
     g.Cb[d] = e ? 1 : 0;
     if constexpr (!S::iso_out) ((Z *) g.Cx)[d] = e ? z : (Z) 0;
@@ -218,14 +221,19 @@ __device__ __forceinline__ int dn_put(const DnArgs &g, int64_t i, int64_t c, boo
 // the device beside them.
 // RMAT n = 65536, 1.82M entries, times 64 full columns, fp64: 7.2 ms with a
 // workgroup per row, LDS accumulators and one read in flight; 2.2 ms without
-// the hub stages; 0.75 ms here.  B's rows, 931 MB, come from L2 and the
+// the hub stages; 0.69 ms here.  B's rows, 931 MB, come from L2 and the
 // Infinity Cache.
 constexpr int DN_UN = 16;
 constexpr int DN_RT = 1024;                 // threads
 constexpr int DN_SPT = 8;                   // products of a stage per thread
 constexpr int DN_STG = DN_RT * DN_SPT;
 
-template <class S, bool ASP, int G>
+// MASK: there is a mask (a template parameter: its fields and tests cost the
+// products without one up to 17%, in spilled registers).  Excluded columns are
+// not gathered, nor rows all of whose are: 60000 rows of 30 times 1000 columns
+// with a hundredth of them allowed 2.93 -> 1.82 ms, none 2.91 -> 0.50; a mask
+// that allows all costs 3% more than one tested at the store.
+template <class S, bool ASP, int G, bool MASK>
 __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const uint32_t *hubs,
                                                    const unsigned long long *nhubs, unsigned long long *next)
 {
@@ -250,11 +258,11 @@ __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const
             if (it >= items) break;
             const int64_t i = hubs[it / nseg], c0 = (it - it / nseg * nseg) * G;
             const int64_t q0 = g.Ap[i], q1 = g.Ap[i + 1];
-            const int64_t stages = (q1 - q0 + SE - 1) / SE;
             // this thread's products of a stage: entries er, er + DN_RT/G, ...,
             // always of column c0 + sub
             const int er = (int) threadIdx.x / G;
-            const bool col = c0 + sub < g.n;
+            bool col = c0 + sub < g.n;
+            if constexpr (MASK) col = col && dn_allowed(g, i, c0 + sub);
             int64_t k[DN_SPT];
             Z a[DN_SPT], b[DN_SPT], t[DN_SPT];
             bool p[DN_SPT];
@@ -298,9 +306,15 @@ __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const
             };
             bool e = false;
             Z z = S::identity();
-            entries(0);
-            rows();
-            products();
+            int64_t stages = (q1 - q0 + SE - 1) / SE;
+            if constexpr (MASK)
+                if (!__syncthreads_or(col)) stages = 0;       // every column excluded
+            if (!MASK || stages > 0)
+            {
+                entries(0);
+                rows();
+                products();
+            }
             if (stages > 1) entries(1);
             for (int64_t s = 0; s < stages; s++)
             {
@@ -331,7 +345,7 @@ __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const
                     if (s + 2 < stages) entries(s + 2);
                 }
             }
-            if (threadIdx.x < G && col) cnt += (unsigned long long) dn_put<S>(g, i, c0 + sub, e, z);
+            if (threadIdx.x < G && c0 + sub < g.n) cnt += (unsigned long long) dn_put<S>(g, i, c0 + sub, e, z);
             __syncthreads();
         }
     }
@@ -354,6 +368,14 @@ __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const
                 if (q1 - q0 > DN_HUB && i < DN_HUB_ROWS) continue;           // done above
             }
             else q1 = g.kdim;
+        }
+        // the columns that the mask excludes are not read, nor a row all of whose are
+        bool want = own;
+        if constexpr (MASK)
+        {
+            want = own && dn_allowed(g, i, c);
+            const unsigned long long any = __ballot(want) >> (team * G);
+            if (!(any & (~0ull >> (64 - G)))) q1 = q0;
         }
         bool e = false;
         Z z = S::identity();
@@ -411,13 +433,13 @@ __global__ __launch_bounds__(DN_RT) void k_dn_rows(DnArgs g, int64_t nseg, const
                         has = (!g.Ab || g.Ab[d] != 0) ? 1 : 0;
                         av[u] = S::geta(Ax, d, g.a_iso);
                     }
-                    p[u] = own && t0 + u < nb && has != 0;
+                    p[u] = want && t0 + u < nb && has != 0;
                 }
                 #pragma unroll
                 for (int u = 0; u < UN; u++)
                 {
                     b[u] = Z(0);
-                    if (own)
+                    if (want)
                     {
                         const int64_t d = kv[u] * g.n + c;
                         if (g.Bb) p[u] = p[u] && g.Bb[d] != 0;
@@ -632,16 +654,22 @@ static int dn_mxm_run(gm_dense_out *C, const gm_csr *Ms, const gm_dense *Md, boo
                 if (!hubs.alloc(sizeof(uint32_t) * hm)) return set_error(GM_OUT_OF_MEMORY, "dense product: rows");
                 k_dn_hubs<<<dn_grid((hm + DN_NT - 1) / DN_NT), DN_NT, 0, st>>>(g.Ap, hm, hubs.as<uint32_t>(), ctr);
             }
-#define GM_DN_ROWS(L)                                                                        \
-    case L:                                                                                  \
-        if (As) k_dn_rows<S, true, 1 << L><<<grid, DN_RT, 0, st>>>(g, nseg, hubs.as<uint32_t>(), ctr, ctr + 1); \
-        else k_dn_rows<S, false, 1 << L><<<grid, DN_RT, 0, st>>>(g, nseg, nullptr, ctr, ctr + 1); \
+            const bool masked = g.mkind != 0;
+#define GM_DN_RUN(L, ASP, MASK) \
+    k_dn_rows<S, ASP, 1 << L, MASK><<<grid, DN_RT, 0, st>>>(g, nseg, hubs.as<uint32_t>(), ctr, ctr + 1)
+#define GM_DN_ROWS(L)                            \
+    case L:                                      \
+        if (As && masked) GM_DN_RUN(L, true, true);   \
+        else if (As) GM_DN_RUN(L, true, false);  \
+        else if (masked) GM_DN_RUN(L, false, true);   \
+        else GM_DN_RUN(L, false, false);         \
         break;
             switch (lg)
             {
                 GM_DN_ROWS(0) GM_DN_ROWS(1) GM_DN_ROWS(2) GM_DN_ROWS(3) GM_DN_ROWS(4) GM_DN_ROWS(5) GM_DN_ROWS(6)
             }
 #undef GM_DN_ROWS
+#undef GM_DN_RUN
         }
         GM_HIP(hipGetLastError(), "k_dn_mxm");
     }
