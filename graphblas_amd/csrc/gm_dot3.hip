@@ -2818,7 +2818,7 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         // entries of a 256-graph batch and saves 14.6 ms of 46.0.  Structural
         // masks only: with int32 mask values the search was paid without fewer
         // entries in the bins (4096 graphs, 1.46e9 entries: 698 ms, 539 without)
-        const bool sym = g.one && g.mask_struct && Mnz >= ((int64_t) 1 << 16) && 4 * front->pairs >= 3 * SYM_SAMPLES;
+        bool sym = g.one && g.mask_struct && Mnz >= ((int64_t) 1 << 16) && 4 * front->pairs >= 3 * SYM_SAMPLES;
         // group deferred entries by probed row: explicit, or by default for
         // masks large enough that the sort pays for itself
         const gm_dot3_params tu = dot3_tuned();
@@ -2838,13 +2838,20 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         // the workspace in one block: row summaries (columns below 2^31), bins,
         // grouping keys, index offsets and list, tile offsets, results, flags
         const bool shared = (A->p == B->p && A->j == B->j && A->nrows == B->nrows);
-        const bool use_desc = A->ncols < ((int64_t) 1 << 31);
+        bool use_desc = A->ncols < ((int64_t) 1 << 31);
         const size_t nr = (size_t) A->nrows + (shared ? 0 : (size_t) B->nrows);
         const int64_t ntiles = (Mnz + D3_CT_TILE - 1) / D3_CT_TILE;
         const size_t wbytes = S::iso_out ? 0 : (zs * (size_t) Mnz + 7) / 8 * 8;
-        if (!work.alloc((use_desc ? sizeof(RowDesc) * nr : 0) + 8 * 3 * (size_t) Mnz * (grouped ? 2 : 1) + 16 * nr +
-                        8 * (size_t) (ntiles + 1) + wbytes + (sym ? 4 * (size_t) Mnz : 0) + (size_t) Mnz))
-            return set_error(GM_OUT_OF_MEMORY, "dot3: workspace");
+        auto room = [&](bool with_desc, bool with_mates) {
+            return work.alloc((with_desc ? sizeof(RowDesc) * nr : 0) + 8 * 3 * (size_t) Mnz * (grouped ? 2 : 1) +
+                              16 * nr + 8 * (size_t) (ntiles + 1) + wbytes + (with_mates ? 4 * (size_t) Mnz : 0) +
+                              (size_t) Mnz);
+        };
+        // without room for them the product does without mates, then without summaries
+        bool have = room(use_desc, sym);
+        if (!have && sym) { sym = false; have = room(use_desc, sym); }
+        if (!have && use_desc) { use_desc = false; have = room(use_desc, sym); }
+        if (!have) return set_error(GM_OUT_OF_MEMORY, "dot3: workspace");
         RowDesc *desc = use_desc ? work.as<RowDesc>() : nullptr;
         g.bins = use_desc ? (uint64_t *) (desc + nr) : work.as<uint64_t>();
         uint64_t *at = g.bins + 3 * (size_t) Mnz;

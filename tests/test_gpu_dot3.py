@@ -385,3 +385,36 @@ def test_dot3_one_matrix(grb, handle, mask, order):
     assert_csr_equal(got, ref, fp_tol=FP_TOL if "fp64" in name else None, what=f"{handle} {mask}")
     for d in (dA, dM):
         d.free()
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("one", [True, False])
+@pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GrB_MIN_PLUS_SEMIRING_INT32", "GxB_ANY_SECONDI_INT64"])
+def test_dot3_without_room_for_helpers(grb, handle, one, order):
+    """The workspace (the fifth allocation) forced not to fit: the product does
+    without the mates of symmetric pairs (one matrix), or without the row
+    summaries, and gives the same result."""
+    import ctypes
+    from helpers import ZT, download
+    print(f"[dot3] without room {handle} one={one} order={order}", flush=True)
+    rng = np.random.default_rng(len(handle))
+    vt = _vals(handle)
+    G = W.rmat_sym(11, 40, seed=6)
+    x = rng.integers(-50, 50, G.nnz).astype(np.int32) if vt else None
+    A = W.Csr(G.nrows, G.ncols, G.p, G.j, x)
+    name, trip = SR[handle]
+    dA, dB, dM = DevCsr(A, trip[2]), DevCsr(A, trip[2]), DevCsr(G, 1)
+    out, sr = capi.GmCsrOut(), capi.GmSemiring(*trip)
+    prm = capi.GmDot3Params(0, 0, 0, 0, order, 0)
+    L = capi.lib()
+    L.gm_debug_fail_after(4)
+    try:
+        rc = L.gm_dot3(ctypes.byref(out), ctypes.byref(dM.view), True, ctypes.byref(dA.view),
+                       ctypes.byref((dA if one else dB).view), ctypes.byref(sr), ctypes.byref(prm))
+    finally:
+        L.gm_debug_fail_after(-1)
+    assert rc == 0, capi.last_error()
+    got = download(out, ZT[{8: "int64", 6: "int32"}[trip[2]]])
+    assert_csr_equal(got, O.dot3(name, G, A, A), what=handle)
+    for d in (dA, dB, dM):
+        d.free()
