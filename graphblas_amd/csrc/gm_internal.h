@@ -48,7 +48,8 @@ struct DevBuf
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() { if (ptr) gm_free(ptr); }
+    ~DevBuf() { drop(); }
+    void drop() { if (ptr) gm_free(ptr); ptr = nullptr; }
     bool alloc(size_t bytes) { ptr = gm_malloc(bytes ? bytes : 8); return ptr != nullptr; }
     template <class T> T *as() const { return (T *) ptr; }
     void *release() { void *p = ptr; ptr = nullptr; return p; }

@@ -1385,6 +1385,10 @@ struct SxPush
 {
     PushArgs h;
     DevBuf pre, coff, it_d, it_e, tab, bits, mbits, seg;
+    void drop()
+    {
+        pre.drop(); coff.drop(); it_d.drop(); it_e.drop(); tab.drop(); bits.drop(); mbits.drop(); seg.drop();
+    }
 };
 
 // bytes of one dense row
@@ -1452,6 +1456,7 @@ struct SxTile
 {
     TileArgs t;
     DevBuf tpos, bits, seg, next;
+    void drop() { tpos.drop(); bits.drop(); seg.drop(); next.drop(); }
 };
 
 static int64_t sx_tile_row_bytes(int64_t n) { return (n + TL_W - 1) / TL_W * (TL_W / 8 + 8); }
@@ -1706,25 +1711,42 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     }
 
     DevBuf gkeys, gvals, glist;
-    const int64_t gslots = hc[CNT_SLOTS];
-    if (gslots > 0)
-    {
-        if (!gkeys.alloc(sizeof(uint32_t) * gslots) || !gvals.alloc(zs * gslots) ||
-            !glist.alloc(sizeof(uint64_t) * gslots))
-            return set_error(GM_OUT_OF_MEMORY, "saxpy3: global hash tables (%lld slots)",
-                             (long long) gslots);
-        g.gkeys = gkeys.as<uint32_t>(); g.gvals = gvals.ptr; g.glist = glist.as<uint64_t>();
-    }
-    const int64_t nbig = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB] + hc[BIN_DNS] +
-                         hc[BIN_TIL];
-    const bool have_big = nbig > 0;
     SxTile tiles;
-    if (hc[BIN_TIL] > 0) GM_TRY(sx_tile_build(g, tiles, hc, B->nrows));
     SxPush push;
     memset(&push.h, 0, sizeof(push.h));
     push.h.dflops = dflops;
-    if constexpr (SX_ANY_ORDER<S>)
-        if (hc[BIN_DNS] > 0) GM_TRY(sx_push_build<S>(g, push, hc[BIN_DNS], hc[CNT_NNZA], hc[CNT_HFLOPS]));
+    // the heavy rows' tables, and the counts of the tiled and dense ones
+    auto tables = [&]() -> int {
+        const int64_t gslots = hc[CNT_SLOTS];
+        if (gslots > 0)
+        {
+            if (!gkeys.alloc(sizeof(uint32_t) * gslots) || !gvals.alloc(zs * gslots) ||
+                !glist.alloc(sizeof(uint64_t) * gslots))
+                return set_error(GM_OUT_OF_MEMORY, "saxpy3: global hash tables (%lld slots)",
+                                 (long long) gslots);
+            g.gkeys = gkeys.as<uint32_t>(); g.gvals = gvals.ptr; g.glist = glist.as<uint64_t>();
+        }
+        if (hc[BIN_TIL] > 0) GM_TRY(sx_tile_build(g, tiles, hc, B->nrows));
+        if constexpr (SX_ANY_ORDER<S>)
+            if (hc[BIN_DNS] > 0) GM_TRY(sx_push_build<S>(g, push, hc[BIN_DNS], hc[CNT_NNZA], hc[CNT_HFLOPS]));
+        return GM_SUCCESS;
+    };
+    int trc = tables();
+    if (trc == GM_OUT_OF_MEMORY && hc[BIN_TIL] + hc[BIN_DNS] > 0)
+    {
+        // no room for the tiles' bits or the dense tables: a hash table for
+        // every heavy row, which is as large as its own products
+        gkeys.drop(); gvals.drop(); glist.drop();
+        tiles.drop();
+        push.drop();
+        k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
+        GM_TRY(sx_count(g, fs, fused ? 0 : 1, 0, 0, dflops, hc, hp));
+        trc = tables();
+    }
+    GM_TRY(trc);
+    const int64_t nbig = hc[BIN_SINGLE] + hc[BIN_WL] + hc[BIN_BLK] + hc[BIN_GLB] + hc[BIN_DNS] +
+                         hc[BIN_TIL];
+    const bool have_big = nbig > 0;
     int64_t nvals = 0, held = 0;        // held: entries C has room for, if at the big rows' bound and small
     DevBuf Ci, Cx;
     if (fused)

@@ -392,3 +392,47 @@ def test_saxpy3_nan_products(grb, shape, bins, mode, table):
     assert np.array_equal(got.p, ref.p) and np.array_equal(got.j, ref.j)
     assert np.array_equal(got.x, ref.x, equal_nan=True), \
         f"{int(np.isnan(got.x).sum())} NaN entries, {int(nan.sum())} expected"
+
+
+@pytest.mark.parametrize("mask", ["none", "!M"])
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("rows,handle", [("spread", "GrB_MIN_PLUS_SEMIRING_INT32"), ("spread", "GxB_ANY_SECONDI_INT64"),
+                                         ("tiled", "GrB_PLUS_TIMES_SEMIRING_FP64")])
+def test_saxpy3_without_room_for_tables(grb, rows, handle, mode, mask):
+    """Every allocation of a product with heavy rows forced to fail in turn:
+    without room for dense tables or tiles the rows take hash tables, so that
+    only what every product needs (counters, lists, row pointers, the result)
+    ends the call."""
+    import ctypes
+    from helpers import ZT, DevCsr, download
+    print(f"[saxpy3] without room {rows} {handle} mode={mode} mask={mask}", flush=True)
+    rng = np.random.default_rng(mode)
+    vt = _vals(handle)
+    m, n = (5, 3000) if rows == "spread" else (300, 3000)
+    A, B = rand_csr(m, 400, 0.4, rng, vt), rand_csr(400, n, 0.03, rng, vt)
+    M = rand_csr(m, n, 0.2, rng, "int64") if mask != "none" else None
+    kw = {} if M is None else {"M": M, "mask_comp": True, "mask_struct": True}
+    name, trip = SR[handle]
+    ref = O.saxpy3(name, A, B, **kw)
+    L, refused, n = capi.lib(), [], 0
+    dA, dB, dM = DevCsr(A, trip[2]), DevCsr(B, trip[2]), DevCsr(M, 8) if M is not None else None
+    sr, prm = capi.GmSemiring(*trip), capi.GmSaxpy3Params(8, 16, 32, mode, 0)
+    for at in range(24):
+        out = capi.GmCsrOut()
+        L.gm_debug_fail_after(at)
+        try:
+            rc = L.gm_saxpy3(ctypes.byref(out), ctypes.byref(dM.view) if dM else None, M is not None, True,
+                             ctypes.byref(dA.view), ctypes.byref(dB.view), ctypes.byref(sr), ctypes.byref(prm))
+        finally:
+            L.gm_debug_fail_after(-1)
+        if rc == capi.GrB_OUT_OF_MEMORY:
+            refused.append(at)
+            continue
+        assert rc == 0, capi.last_error()
+        got = download(out, ZT[{8: "int64", 6: "int32", 11: "fp64"}[trip[2]]])
+        assert_csr_equal(got, ref, what=f"allocation {at}")
+    # row pointers, counters, lists, the few rows' flops; columns, values and the pass over more than one tile
+    assert len(refused) <= 7, refused
+    for d in (dA, dB, dM):
+        if d:
+            d.free()
