@@ -177,7 +177,8 @@ struct AccArgs
     const int64_t *Mp, *Mj; const void *Mx; int32_t m_iso, msize;
     int32_t has_mask, mask_comp, mask_struct, replace, op;
     int64_t ntc, ntt;     // tiles of C's and T's entries (one entry past the end included)
-    uint32_t *rank;       // per entry (C's tiles, then T's): output entries before it in its tile
+    uint64_t *bits;       // LEAN: a bit per entry (C's tiles, then T's), set for an output entry
+    uint32_t *rank;       // per entry (the same order): output entries before it in its tile
     uint8_t *state;       // per entry: AC_*
     int64_t *other;       // per entry: its place in the other operand
     int64_t *toff;        // ntc + ntt + 1: output entries before each tile
@@ -199,10 +200,39 @@ enum { AC_NONE = 0, AC_OWN = 1, AC_BOTH = 2, AC_OTHER = 3 };
 // us with a thread per row walking it twice, 680 us here; four hops of a
 // shortest-path vector that grows to 44000 entries (one row): 66 ms and 1.4
 // ms with their products.
+// LEAN, for merges whose 13 bytes of state an entry do not fit: a bit an entry
+// is kept, and the writing pass searches again.
 constexpr int AC_NT = 256;
 constexpr int AC_IPT = 8;
 constexpr int AC_TILE = AC_NT * AC_IPT;
 
+// what becomes of entry e of C (of T), in row i; y: its place in the other operand
+__device__ __forceinline__ int ac_fate(const AccArgs &g, bool isC, int64_t i, int64_t e, int64_t &y)
+{
+    const int64_t *Yp = isC ? g.Tp : g.Cp, *Yj = isC ? g.Tj : g.Cj;
+    const int64_t j = isC ? g.Cj[e] : g.Tj[e];
+    bool both = false;
+    y = 0;
+    if (Yp)
+    {
+        const int64_t y1 = Yp[i + 1];
+        y = lower_bound(Yj, Yp[i], y1, j);
+        both = y < y1 && Yj[y] == j;
+    }
+    bool allow = true;
+    if (g.has_mask)
+    {
+        const int64_t m1 = g.Mp[i + 1], q = lower_bound(g.Mj, g.Mp[i], m1, j);
+        const bool in = q < m1 && g.Mj[q] == j && (g.mask_struct || mask_true(g.Mx, q, g.msize, g.m_iso));
+        allow = g.mask_comp ? !in : in;
+    }
+    if (!isC) return (allow && !both) ? AC_OWN : AC_NONE;
+    if (!allow) return g.replace ? AC_NONE : AC_OWN;
+    if (g.op) return both ? AC_BOTH : AC_OWN;
+    return both ? AC_OTHER : AC_NONE;
+}
+
+template <bool LEAN>
 __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
 {
     constexpr int NW = AC_NT / 64;
@@ -211,8 +241,7 @@ __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
     const bool isC = (int64_t) blockIdx.x < g.ntc;
     const int64_t t0 = ((int64_t) blockIdx.x - (isC ? 0 : g.ntc)) * AC_TILE;
     const int64_t n = isC ? g.nc : g.nt;
-    const int64_t *Xp = isC ? g.Cp : g.Tp, *Xj = isC ? g.Cj : g.Tj;
-    const int64_t *Yp = isC ? g.Tp : g.Cp, *Yj = isC ? g.Tj : g.Cj;
+    const int64_t *Xp = isC ? g.Cp : g.Tp;
     const int64_t t1 = t0 + AC_TILE < n ? t0 + AC_TILE : n;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const size_t slot = (size_t) blockIdx.x * AC_TILE;
@@ -228,33 +257,16 @@ __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
         if (e < t1)
         {
             const int64_t i = tr_row_of(Xp, s_r[0], s_r[1], e);
-            const int64_t j = Xj[e];
-            bool both = false;
-            if (Yp)
-            {
-                const int64_t y1 = Yp[i + 1];
-                y = lower_bound(Yj, Yp[i], y1, j);
-                both = y < y1 && Yj[y] == j;
-            }
-            bool allow = true;
-            if (g.has_mask)
-            {
-                const int64_t m1 = g.Mp[i + 1], q = lower_bound(g.Mj, g.Mp[i], m1, j);
-                const bool in = q < m1 && g.Mj[q] == j && (g.mask_struct || mask_true(g.Mx, q, g.msize, g.m_iso));
-                allow = g.mask_comp ? !in : in;
-            }
-            if (!isC) st = (allow && !both) ? AC_OWN : AC_NONE;
-            else if (!allow) st = g.replace ? AC_NONE : AC_OWN;
-            else if (g.op) st = both ? AC_BOTH : AC_OWN;
-            else st = both ? AC_OTHER : AC_NONE;
+            st = ac_fate(g, isC, i, e, y);
         }
-        if (e <= n)
+        if (!LEAN && e <= n)
         {
             g.state[slot + t * AC_NT + threadIdx.x] = (uint8_t) st;
             g.other[slot + t * AC_NT + threadIdx.x] = y;
         }
         bal[t] = __ballot(st != AC_NONE);
         if (lane == 0) s_cnt[t * NW + wv] = __popcll(bal[t]);
+        if (LEAN && lane == 0) g.bits[(slot >> 6) + t * NW + wv] = bal[t];
     }
     __syncthreads();
     int run = 0, total = 0;
@@ -264,7 +276,7 @@ __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
         total += s_cnt[q];
     }
     #pragma unroll
-    for (int t = 0; t < AC_IPT; t++)
+    for (int t = 0; t < AC_IPT && !LEAN; t++)
     {
         if (t0 + t * AC_NT + threadIdx.x <= n)
             g.rank[slot + t * AC_NT + threadIdx.x] = (uint32_t) (run + __popcll(bal[t] & ((1ull << lane) - 1ull)));
@@ -274,18 +286,44 @@ __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
     if (threadIdx.x == 0) g.toff[blockIdx.x] = total;
 }
 
+// output entries in slot s's tile before s
+template <bool LEAN>
+__device__ __forceinline__ int64_t ac_rank(const AccArgs &g, int64_t s)
+{
+    if constexpr (!LEAN) return (int64_t) g.rank[s];
+    int64_t r = 0;
+    for (int64_t w = s / AC_TILE * (AC_TILE / 64); w < s >> 6; w++) r += __popcll(g.bits[w]);
+    return r + __popcll(g.bits[s >> 6] & ((1ull << (s & 63)) - 1ull));
+}
+
 // output entries of C (T) before its entry p, p up to the entry count
+template <bool LEAN>
 __device__ __forceinline__ int64_t ac_before_c(const AccArgs &g, int64_t p)
 {
-    return g.toff[p / AC_TILE] + (int64_t) g.rank[p];
+    return g.toff[p / AC_TILE] + ac_rank<LEAN>(g, p);
 }
+template <bool LEAN>
 __device__ __forceinline__ int64_t ac_before_t(const AccArgs &g, int64_t p)
 {
-    return g.toff[g.ntc + p / AC_TILE] - g.toff[g.ntc] + (int64_t) g.rank[g.ntc * AC_TILE + p];
+    return g.toff[g.ntc + p / AC_TILE] - g.toff[g.ntc] + ac_rank<LEAN>(g, g.ntc * AC_TILE + p);
+}
+
+// the fate of entry p of C (of T) as k_accum_state found it
+template <bool LEAN>
+__device__ __forceinline__ int ac_again(const AccArgs &g, bool isC, int64_t p, int64_t &y)
+{
+    const int64_t s = isC ? p : g.ntc * AC_TILE + p;
+    if constexpr (!LEAN)
+    {
+        y = g.other[s];
+        return g.state[s];
+    }
+    if (!((g.bits[s >> 6] >> (s & 63)) & 1ull)) return AC_NONE;
+    return ac_fate(g, isC, tr_row_of(isC ? g.Cp : g.Tp, 0, g.m - 1, p), p, y);
 }
 
 // every output entry to its place: the entries of both operands before it
-template <class Z>
+template <class Z, bool LEAN>
 __global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g)
 {
     const Z *Cx = (const Z *) g.Cx, *Tx = (const Z *) g.Tx;
@@ -293,9 +331,10 @@ __global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g)
     const int64_t stride = (int64_t) gridDim.x * AC_NT, t0 = (int64_t) blockIdx.x * AC_NT + threadIdx.x;
     for (int64_t p = t0; p < g.nc; p += stride)
     {
-        const int st = g.state[p];
+        int64_t q;
+        const int st = ac_again<LEAN>(g, true, p, q);
         if (st == AC_NONE) continue;
-        const int64_t q = g.other[p], o = ac_before_c(g, p) + ac_before_t(g, q);
+        const int64_t o = ac_before_c<LEAN>(g, p) + ac_before_t<LEAN>(g, q);
         g.Oj[o] = g.Cj[p];
         if (st == AC_OTHER) Ox[o] = Tx[g.t_iso ? 0 : q];
         else
@@ -306,13 +345,84 @@ __global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g)
     }
     for (int64_t q = t0; q < g.nt; q += stride)
     {
-        if (g.state[g.ntc * AC_TILE + q] == AC_NONE) continue;
-        const int64_t o = ac_before_t(g, q) + ac_before_c(g, g.other[g.ntc * AC_TILE + q]);
+        int64_t p;
+        if (ac_again<LEAN>(g, false, q, p) == AC_NONE) continue;
+        const int64_t o = ac_before_t<LEAN>(g, q) + ac_before_c<LEAN>(g, p);
         g.Oj[o] = g.Tj[q];
         Ox[o] = Tx[g.t_iso ? 0 : q];
     }
     for (int64_t i = t0; i <= g.m; i += stride)
-        g.Op[i] = ac_before_c(g, g.Cp ? g.Cp[i] : 0) + ac_before_t(g, g.Tp[i]);
+        g.Op[i] = ac_before_c<LEAN>(g, g.Cp ? g.Cp[i] : 0) + ac_before_t<LEAN>(g, g.Tp[i]);
+}
+
+// the merge of operands whose entry counts are known; hp: pinned
+template <class Z, bool LEAN>
+static int accum_try(gm_csr_out *O, AccArgs g, const gm_csr *T, int64_t *hp)
+{
+    hipStream_t st = stream();
+    const int64_t m = g.m;
+    g.ntc = g.nc / AC_TILE + 1;
+    g.ntt = g.nt / AC_TILE + 1;
+    const int64_t tiles = g.ntc + g.ntt;
+    const size_t slots = (size_t) tiles * AC_TILE;
+    DevBuf Op, Oj, Ox, work;
+    auto output = [&](int64_t entries) {
+        if (!Oj.alloc(sizeof(int64_t) * (size_t) (entries > 0 ? entries : 1)) ||
+            !Ox.alloc(sizeof(Z) * (size_t) (entries > 0 ? entries : 1)))
+            return set_error(GM_OUT_OF_MEMORY, "accum: output (%lld entries)", (long long) entries);
+        g.Oj = Oj.as<int64_t>();
+        g.Ox = Ox.ptr;
+        return GM_SUCCESS;
+    };
+    // a small output at its bound, so that its size needs no wait of its own
+    const int64_t most = g.nc + g.nt;
+    const bool bound = most * (int64_t) (sizeof(int64_t) + sizeof(Z)) <= OUT_BOUND_MAX;
+    if (bound) GM_TRY(output(most));
+    const size_t tbytes = sizeof(int64_t) * (size_t) (tiles + 1);
+    if (!Op.alloc(sizeof(int64_t) * (m + 1))) return set_error(GM_OUT_OF_MEMORY, "accum: row pointers");
+    if (!work.alloc(tbytes + (LEAN ? slots / 8 : slots * 13))) return set_error(GM_OUT_OF_MEMORY, "accum: workspace");
+    g.toff = work.as<int64_t>();
+    g.bits = (uint64_t *) (g.toff + tiles + 1);
+    g.other = g.toff + tiles + 1;
+    g.rank = (uint32_t *) (g.other + slots);
+    g.state = (uint8_t *) (g.rank + slots);
+    g.Op = Op.as<int64_t>();
+    {
+        ProfScope ps("accum_mask_state");
+        k_accum_state<LEAN><<<(unsigned) tiles, AC_NT, 0, st>>>(g);
+        GM_HIP(hipGetLastError(), "k_accum_state");
+    }
+    GM_TRY(scan_exclusive_i64(g.toff, g.toff, tiles));
+    GM_HIP(hipMemcpyAsync(hp, g.toff + tiles, sizeof(int64_t), hipMemcpyDeviceToHost, st), "accum nnz");
+    if (!bound)
+    {
+        GM_HIP(hipStreamSynchronize(st), "accum nnz sync");
+        GM_TRY(output(hp[0]));
+    }
+    {
+        ProfScope ps("accum_mask_write");
+        int64_t items = g.nc > g.nt ? g.nc : g.nt;
+        if (m + 1 > items) items = m + 1;
+        k_accum_write<Z, LEAN><<<post_grid(items, AC_NT, (int64_t) cu_count() * 16), AC_NT, 0, st>>>(g);
+        GM_HIP(hipGetLastError(), "k_accum_write");
+    }
+    GM_HIP(hipStreamSynchronize(st), "accum sync");
+    const int64_t nz = hp[0];
+    if (bound)
+    {
+        bool moved = fit_block(Oj, sizeof(int64_t) * nz, sizeof(int64_t) * most);
+        moved |= fit_block(Ox, sizeof(Z) * nz, sizeof(Z) * most);
+        if (moved) GM_HIP(hipStreamSynchronize(st), "accum fit sync");
+    }
+    O->nrows = m;
+    O->ncols = T->ncols;
+    O->nvals = nz;
+    O->p = (int64_t *) Op.release();
+    O->j = (int64_t *) Oj.release();
+    O->x = Ox.release();
+    O->iso = 0;
+    O->type = T->type;
+    return GM_SUCCESS;
 }
 
 template <class Z>
@@ -349,49 +459,9 @@ static int accum_mask_run(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bool 
     }
     g.nc = hp[0];
     g.nt = hp[1];
-    g.ntc = g.nc / AC_TILE + 1;
-    g.ntt = g.nt / AC_TILE + 1;
-    const int64_t tiles = g.ntc + g.ntt;
-    const size_t slots = (size_t) tiles * AC_TILE;
-    // the output at its bound, so that its size needs no wait of its own
-    const int64_t most = g.nc + g.nt > 0 ? g.nc + g.nt : 1;
-    DevBuf Op, Oj, Ox, work;
-    if (!Oj.alloc(sizeof(int64_t) * most) || !Ox.alloc(sizeof(Z) * most))
-        return set_error(GM_OUT_OF_MEMORY, "accum: output (%lld entries)", (long long) most);
-    if (!Op.alloc(sizeof(int64_t) * (m + 1)) || !work.alloc(sizeof(int64_t) * (size_t) (tiles + 1) + slots * 13))
-        return set_error(GM_OUT_OF_MEMORY, "accum: workspace");
-    g.toff = work.as<int64_t>();
-    g.other = g.toff + tiles + 1;
-    g.rank = (uint32_t *) (g.other + slots);
-    g.state = (uint8_t *) (g.rank + slots);
-    g.Op = Op.as<int64_t>();
-    {
-        ProfScope ps("accum_mask_state");
-        k_accum_state<<<(unsigned) tiles, AC_NT, 0, st>>>(g);
-        GM_HIP(hipGetLastError(), "k_accum_state");
-    }
-    GM_TRY(scan_exclusive_i64(g.toff, g.toff, tiles));
-    g.Oj = Oj.as<int64_t>();
-    g.Ox = Ox.ptr;
-    {
-        ProfScope ps("accum_mask_write");
-        int64_t items = g.nc > g.nt ? g.nc : g.nt;
-        if (m + 1 > items) items = m + 1;
-        k_accum_write<Z><<<post_grid(items, AC_NT, (int64_t) cu_count() * 16), AC_NT, 0, st>>>(g);
-        GM_HIP(hipGetLastError(), "k_accum_write");
-    }
-    GM_HIP(hipMemcpyAsync(hp, g.toff + tiles, sizeof(int64_t), hipMemcpyDeviceToHost, st), "accum nnz");
-    GM_HIP(hipStreamSynchronize(st), "accum sync");
-    const int64_t nz = hp[0];
-    O->nrows = m;
-    O->ncols = T->ncols;
-    O->nvals = nz;
-    O->p = (int64_t *) Op.release();
-    O->j = (int64_t *) Oj.release();
-    O->x = Ox.release();
-    O->iso = 0;
-    O->type = T->type;
-    return GM_SUCCESS;
+    int rc = accum_try<Z, false>(O, g, T, hp);
+    if (rc == GM_OUT_OF_MEMORY) rc = accum_try<Z, true>(O, g, T, hp);
+    return rc;
 }
 
 } // namespace gm

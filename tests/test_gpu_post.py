@@ -256,3 +256,62 @@ def test_accum_mask_long_rows(grb, rows, nc, nt, mask):
         for d in (dC, dT, dM):
             if d:
                 d.free()
+
+
+def _long_rows(rng, rows, n, nnz):
+    key = np.sort(rng.choice(rows * n, size=nnz, replace=False))
+    p = np.searchsorted(key // n, np.arange(rows + 1)).astype(np.int64)
+    return W.Csr(rows, n, p, (key % n).astype(np.int64), rng.integers(-9, 9, nnz).astype(np.int64))
+
+
+@pytest.mark.parametrize("mask", ["none", "M", "!M"])
+@pytest.mark.parametrize("nc,nt", [(0, 2048), (2047, 1), (2048, 2049), (4096, 0), (5000, 7000)])
+@pytest.mark.parametrize("rows", [1, 3, 900])
+def test_accum_mask_without_room(grb, rows, nc, nt, mask):
+    """Any allocation forced to fail: the merge is done with a bit an entry in
+    place of its state, and gives the same result."""
+    print(f"[post] accum without room rows={rows} nc={nc} nt={nt} mask={mask}", flush=True)
+    rng = np.random.default_rng(nc + nt + rows)
+    n = 12000
+    C, T = _long_rows(rng, rows, n, nc), _long_rows(rng, rows, n, nt)
+    M = _long_rows(rng, rows, n, 6000) if mask != "none" else None
+    L = capi.lib()
+    for at, (op, replace) in enumerate(((1, False), (0, False), (0, True), (2, True))):
+        ref = O.accum_mask(C, M, T, mask_comp=mask == "!M", mask_struct=False, replace=replace, op=op,
+                           dtype=np.int64)
+        dC, dT = DevCsr(C, 8), DevCsr(T, 8)
+        dM = DevCsr(M, 8) if M is not None else None
+        out = capi.GmCsrOut()
+        L.gm_debug_fail_after(at)            # columns, values, row pointers, workspace
+        try:
+            rc = L.gm_accum_mask(ctypes.byref(out), ctypes.byref(dC.view),
+                                 ctypes.byref(dM.view) if dM else None, mask == "!M", False, replace,
+                                 ctypes.byref(dT.view), op)
+        finally:
+            L.gm_debug_fail_after(-1)
+        assert rc == 0, capi.last_error()
+        assert_csr_equal(download(out, np.int64), ref, what=f"op={op} replace={replace}")
+        for d in (dC, dT, dM):
+            if d:
+                d.free()
+
+
+@pytest.mark.parametrize("nnz", [100000, 1000000, 3000000])
+def test_accum_mask_result_memory(grb, nnz):
+    """C<M, replace> = T with a small mask keeps about its entries' memory, below
+    and above the size (64 MB) that is written at its bound."""
+    rng = np.random.default_rng(nnz)
+    C, T = _long_rows(rng, 2, 4 * nnz, nnz), _long_rows(rng, 2, 4 * nnz, nnz)
+    M = _long_rows(rng, 2, 4 * nnz, 5000)
+    ref = O.accum_mask(C, M, T, mask_struct=True, replace=True, op=0, dtype=np.int64)
+    dC, dT, dM = DevCsr(C, 8), DevCsr(T, 8), DevCsr(M, 8)
+    out, L = capi.GmCsrOut(), capi.lib()
+    before = L.gm_arena_bytes_in_use()
+    rc = L.gm_accum_mask(ctypes.byref(out), ctypes.byref(dC.view), ctypes.byref(dM.view), False, True, True,
+                         ctypes.byref(dT.view), 0)
+    assert rc == 0, capi.last_error()
+    held = L.gm_arena_bytes_in_use() - before
+    for d in (dC, dT, dM):
+        d.free()
+    assert_csr_equal(download(out, np.int64), ref, what="C<M> = T")
+    assert held <= 5 << 20, f"{held} bytes for {ref.nnz} entries"
