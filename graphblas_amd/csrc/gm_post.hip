@@ -19,6 +19,7 @@
 #include <cstring>
 #include <rocprim/device/device_radix_sort.hpp>
 #include "gm_internal.h"
+#include "gm_block.h"
 
 namespace gm
 {
@@ -192,7 +193,7 @@ struct AccArgs
 // put out by C's entry alone.
 enum { AC_NONE = 0, AC_OWN = 1, AC_BOTH = 2, AC_OTHER = 3 };
 
-// One tile per workgroup: the fate of AC_TILE entries of C or of T and their
+// One tile per workgroup: the fate of AC_NT * IPT entries of C or of T and their
 // ranks among the tile's output entries.  A row may hold all the entries (a
 // vector is one row), so the unit is the entry: the rows of a tile's ends are
 // searched once, each entry searches only between them.  Bound by the searches'
@@ -200,11 +201,13 @@ enum { AC_NONE = 0, AC_OWN = 1, AC_BOTH = 2, AC_OTHER = 3 };
 // us with a thread per row walking it twice, 680 us here; four hops of a
 // shortest-path vector that grows to 44000 entries (one row): 66 ms and 1.4
 // ms with their products.
+// IPT is AC_IPT, or 1 for a merge of at most AC_FEW such tiles, which would leave
+// most CUs idle: a thread's eight searches follow one another.
 // LEAN, for merges whose 13 bytes of state an entry do not fit: a bit an entry
 // is kept, and the writing pass searches again.
 constexpr int AC_NT = 256;
 constexpr int AC_IPT = 8;
-constexpr int AC_TILE = AC_NT * AC_IPT;
+constexpr int AC_FEW = 4 * AC_NT;
 
 // what becomes of entry e of C (of T), in row i; y: its place in the other operand
 __device__ __forceinline__ int ac_fate(const AccArgs &g, bool isC, int64_t i, int64_t e, int64_t &y)
@@ -232,24 +235,24 @@ __device__ __forceinline__ int ac_fate(const AccArgs &g, bool isC, int64_t i, in
     return both ? AC_OTHER : AC_NONE;
 }
 
-template <bool LEAN>
+template <bool LEAN, int IPT>
 __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
 {
-    constexpr int NW = AC_NT / 64;
+    constexpr int NW = AC_NT / 64, TILE = AC_NT * IPT;
     __shared__ int64_t s_r[2];
-    __shared__ int s_cnt[AC_IPT * NW];
+    __shared__ int s_cnt[IPT * NW];
     const bool isC = (int64_t) blockIdx.x < g.ntc;
-    const int64_t t0 = ((int64_t) blockIdx.x - (isC ? 0 : g.ntc)) * AC_TILE;
+    const int64_t t0 = ((int64_t) blockIdx.x - (isC ? 0 : g.ntc)) * TILE;
     const int64_t n = isC ? g.nc : g.nt;
     const int64_t *Xp = isC ? g.Cp : g.Tp;
-    const int64_t t1 = t0 + AC_TILE < n ? t0 + AC_TILE : n;
+    const int64_t t1 = t0 + TILE < n ? t0 + TILE : n;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const size_t slot = (size_t) blockIdx.x * AC_TILE;
+    const size_t slot = (size_t) blockIdx.x * TILE;
     if (threadIdx.x < 2 && t0 < t1) s_r[threadIdx.x] = tr_row_of(Xp, 0, g.m - 1, threadIdx.x == 0 ? t0 : t1 - 1);
     __syncthreads();
-    unsigned long long bal[AC_IPT];
+    unsigned long long bal[IPT];
     #pragma unroll
-    for (int t = 0; t < AC_IPT; t++)
+    for (int t = 0; t < IPT; t++)
     {
         const int64_t e = t0 + t * AC_NT + threadIdx.x;
         int st = AC_NONE;
@@ -270,49 +273,49 @@ __global__ __launch_bounds__(AC_NT) void k_accum_state(AccArgs g)
     }
     __syncthreads();
     int run = 0, total = 0;
-    for (int q = 0; q < AC_IPT * NW; q++)
+    for (int q = 0; q < IPT * NW; q++)
     {
         if (q < wv) run += s_cnt[q];
         total += s_cnt[q];
     }
     #pragma unroll
-    for (int t = 0; t < AC_IPT && !LEAN; t++)
+    for (int t = 0; t < IPT && !LEAN; t++)
     {
         if (t0 + t * AC_NT + threadIdx.x <= n)
             g.rank[slot + t * AC_NT + threadIdx.x] = (uint32_t) (run + __popcll(bal[t] & ((1ull << lane) - 1ull)));
         for (int q = 0; q < NW; q++)
-            if (t * NW + wv + q < AC_IPT * NW) run += s_cnt[t * NW + wv + q];
+            if (t * NW + wv + q < IPT * NW) run += s_cnt[t * NW + wv + q];
     }
     if (threadIdx.x == 0) g.toff[blockIdx.x] = total;
 }
 
 // output entries in slot s's tile before s
-template <bool LEAN>
+template <bool LEAN, int IPT>
 __device__ __forceinline__ int64_t ac_rank(const AccArgs &g, int64_t s)
 {
     if constexpr (!LEAN) return (int64_t) g.rank[s];
     int64_t r = 0;
-    for (int64_t w = s / AC_TILE * (AC_TILE / 64); w < s >> 6; w++) r += __popcll(g.bits[w]);
+    for (int64_t w = s / (AC_NT * IPT) * ((AC_NT * IPT) / 64); w < s >> 6; w++) r += __popcll(g.bits[w]);
     return r + __popcll(g.bits[s >> 6] & ((1ull << (s & 63)) - 1ull));
 }
 
 // output entries of C (T) before its entry p, p up to the entry count
-template <bool LEAN>
-__device__ __forceinline__ int64_t ac_before_c(const AccArgs &g, int64_t p)
+template <bool LEAN, int IPT>
+__device__ __forceinline__ int64_t ac_before_c(const AccArgs &g, const int64_t *toff, int64_t p)
 {
-    return g.toff[p / AC_TILE] + ac_rank<LEAN>(g, p);
+    return toff[p / (AC_NT * IPT)] + ac_rank<LEAN, IPT>(g, p);
 }
-template <bool LEAN>
-__device__ __forceinline__ int64_t ac_before_t(const AccArgs &g, int64_t p)
+template <bool LEAN, int IPT>
+__device__ __forceinline__ int64_t ac_before_t(const AccArgs &g, const int64_t *toff, int64_t p)
 {
-    return g.toff[g.ntc + p / AC_TILE] - g.toff[g.ntc] + ac_rank<LEAN>(g, g.ntc * AC_TILE + p);
+    return toff[g.ntc + p / (AC_NT * IPT)] - toff[g.ntc] + ac_rank<LEAN, IPT>(g, g.ntc * (AC_NT * IPT) + p);
 }
 
 // the fate of entry p of C (of T) as k_accum_state found it
-template <bool LEAN>
+template <bool LEAN, int IPT>
 __device__ __forceinline__ int ac_again(const AccArgs &g, bool isC, int64_t p, int64_t &y)
 {
-    const int64_t s = isC ? p : g.ntc * AC_TILE + p;
+    const int64_t s = isC ? p : g.ntc * (AC_NT * IPT) + p;
     if constexpr (!LEAN)
     {
         y = g.other[s];
@@ -322,19 +325,51 @@ __device__ __forceinline__ int ac_again(const AccArgs &g, bool isC, int64_t p, i
     return ac_fate(g, isC, tr_row_of(isC ? g.Cp : g.Tp, 0, g.m - 1, p), p, y);
 }
 
-// every output entry to its place: the entries of both operands before it
-template <class Z, bool LEAN>
-__global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g)
+// Every output entry to its place: the entries of both operands before it.
+// IPT = 1: toff holds the tiles' counts, which every workgroup scans for itself,
+// as a scan's launch costs a small merge more.  The total is left in host[0].
+// 1000 rows of 8 entries in C and T, sizes unknown: 56.9 us with a thread a row
+// counting and filling, 68.9 with large tiles, a scan and the sizes and the
+// total copied, 50.5 here.
+template <class Z, bool LEAN, int IPT>
+__global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g, int64_t *host)
 {
+    constexpr bool FEW = IPT == 1;
+    constexpr int PER = AC_FEW / AC_NT;
+    __shared__ int64_t s_toff[FEW ? AC_FEW + 1 : 1], s_scan[AC_NT / 64 + 1];
+    const int64_t tiles = g.ntc + g.ntt;
+    const int64_t *toff = g.toff;
+    if constexpr (FEW)
+    {
+        int64_t c[PER], sum = 0, total;
+        #pragma unroll
+        for (int u = 0; u < PER; u++)
+        {
+            const int t = (int) threadIdx.x * PER + u;
+            c[u] = t < tiles ? g.toff[t] : 0;
+            sum += c[u];
+        }
+        int64_t run = block_exclusive_scan<int64_t, AC_NT>(sum, s_scan, &total);
+        #pragma unroll
+        for (int u = 0; u < PER; u++)
+        {
+            s_toff[(int) threadIdx.x * PER + u] = run;
+            run += c[u];
+        }
+        if (threadIdx.x == 0) s_toff[AC_FEW] = total;
+        __syncthreads();
+        toff = s_toff;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) host[0] = toff[tiles];
     const Z *Cx = (const Z *) g.Cx, *Tx = (const Z *) g.Tx;
     Z *Ox = (Z *) g.Ox;
     const int64_t stride = (int64_t) gridDim.x * AC_NT, t0 = (int64_t) blockIdx.x * AC_NT + threadIdx.x;
     for (int64_t p = t0; p < g.nc; p += stride)
     {
         int64_t q;
-        const int st = ac_again<LEAN>(g, true, p, q);
+        const int st = ac_again<LEAN, IPT>(g, true, p, q);
         if (st == AC_NONE) continue;
-        const int64_t o = ac_before_c<LEAN>(g, p) + ac_before_t<LEAN>(g, q);
+        const int64_t o = ac_before_c<LEAN, IPT>(g, toff, p) + ac_before_t<LEAN, IPT>(g, toff, q);
         g.Oj[o] = g.Cj[p];
         if (st == AC_OTHER) Ox[o] = Tx[g.t_iso ? 0 : q];
         else
@@ -346,25 +381,33 @@ __global__ __launch_bounds__(AC_NT) void k_accum_write(AccArgs g)
     for (int64_t q = t0; q < g.nt; q += stride)
     {
         int64_t p;
-        if (ac_again<LEAN>(g, false, q, p) == AC_NONE) continue;
-        const int64_t o = ac_before_t<LEAN>(g, q) + ac_before_c<LEAN>(g, p);
+        if (ac_again<LEAN, IPT>(g, false, q, p) == AC_NONE) continue;
+        const int64_t o = ac_before_t<LEAN, IPT>(g, toff, q) + ac_before_c<LEAN, IPT>(g, toff, p);
         g.Oj[o] = g.Tj[q];
         Ox[o] = Tx[g.t_iso ? 0 : q];
     }
     for (int64_t i = t0; i <= g.m; i += stride)
-        g.Op[i] = ac_before_c<LEAN>(g, g.Cp ? g.Cp[i] : 0) + ac_before_t<LEAN>(g, g.Tp[i]);
+        g.Op[i] = ac_before_c<LEAN, IPT>(g, toff, g.Cp ? g.Cp[i] : 0) + ac_before_t<LEAN, IPT>(g, toff, g.Tp[i]);
+}
+
+// nnz(C) and nnz(T) to the host
+__global__ void k_accum_sizes(const int64_t *Cp, const int64_t *Tp, int64_t m, int64_t *host)
+{
+    if (threadIdx.x == 0) host[0] = Cp ? Cp[m] : 0;
+    if (threadIdx.x == 1) host[1] = Tp[m];
 }
 
 // the merge of operands whose entry counts are known; hp: pinned
-template <class Z, bool LEAN>
+template <class Z, bool LEAN, int IPT>
 static int accum_try(gm_csr_out *O, AccArgs g, const gm_csr *T, int64_t *hp)
 {
     hipStream_t st = stream();
     const int64_t m = g.m;
-    g.ntc = g.nc / AC_TILE + 1;
-    g.ntt = g.nt / AC_TILE + 1;
+    constexpr int64_t TILE = AC_NT * IPT;
+    g.ntc = g.nc / TILE + 1;
+    g.ntt = g.nt / TILE + 1;
     const int64_t tiles = g.ntc + g.ntt;
-    const size_t slots = (size_t) tiles * AC_TILE;
+    const size_t slots = (size_t) tiles * TILE;
     DevBuf Op, Oj, Ox, work;
     auto output = [&](int64_t entries) {
         if (!Oj.alloc(sizeof(int64_t) * (size_t) (entries > 0 ? entries : 1)) ||
@@ -389,13 +432,13 @@ static int accum_try(gm_csr_out *O, AccArgs g, const gm_csr *T, int64_t *hp)
     g.Op = Op.as<int64_t>();
     {
         ProfScope ps("accum_mask_state");
-        k_accum_state<LEAN><<<(unsigned) tiles, AC_NT, 0, st>>>(g);
+        k_accum_state<LEAN, IPT><<<(unsigned) tiles, AC_NT, 0, st>>>(g);
         GM_HIP(hipGetLastError(), "k_accum_state");
     }
-    GM_TRY(scan_exclusive_i64(g.toff, g.toff, tiles));
-    GM_HIP(hipMemcpyAsync(hp, g.toff + tiles, sizeof(int64_t), hipMemcpyDeviceToHost, st), "accum nnz");
+    if (IPT != 1) GM_TRY(scan_exclusive_i64(g.toff, g.toff, tiles));
     if (!bound)
     {
+        GM_HIP(hipMemcpyAsync(hp, g.toff + tiles, sizeof(int64_t), hipMemcpyDeviceToHost, st), "accum nnz");
         GM_HIP(hipStreamSynchronize(st), "accum nnz sync");
         GM_TRY(output(hp[0]));
     }
@@ -403,7 +446,7 @@ static int accum_try(gm_csr_out *O, AccArgs g, const gm_csr *T, int64_t *hp)
         ProfScope ps("accum_mask_write");
         int64_t items = g.nc > g.nt ? g.nc : g.nt;
         if (m + 1 > items) items = m + 1;
-        k_accum_write<Z, LEAN><<<post_grid(items, AC_NT, (int64_t) cu_count() * 16), AC_NT, 0, st>>>(g);
+        k_accum_write<Z, LEAN, IPT><<<post_grid(items, AC_NT, (int64_t) cu_count() * 16), AC_NT, 0, st>>>(g, hp);
         GM_HIP(hipGetLastError(), "k_accum_write");
     }
     GM_HIP(hipStreamSynchronize(st), "accum sync");
@@ -453,14 +496,16 @@ static int accum_mask_run(gm_csr_out *O, const gm_csr *C, const gm_csr *M, bool 
     hp[1] = nt;
     if (!known)
     {
-        if (g.Cp) GM_HIP(hipMemcpyAsync(hp, g.Cp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(C)");
-        GM_HIP(hipMemcpyAsync(hp + 1, g.Tp + m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(T)");
+        k_accum_sizes<<<1, 64, 0, st>>>(g.Cp, g.Tp, m, hp);
+        GM_HIP(hipGetLastError(), "k_accum_sizes");
         GM_HIP(hipStreamSynchronize(st), "accum sizes sync");
     }
     g.nc = hp[0];
     g.nt = hp[1];
-    int rc = accum_try<Z, false>(O, g, T, hp);
-    if (rc == GM_OUT_OF_MEMORY) rc = accum_try<Z, true>(O, g, T, hp);
+    // (a merge of few tiles is below OUT_BOUND_MAX)
+    const bool few = g.nc / AC_NT + g.nt / AC_NT + 2 <= AC_FEW;
+    int rc = few ? accum_try<Z, false, 1>(O, g, T, hp) : accum_try<Z, false, AC_IPT>(O, g, T, hp);
+    if (rc == GM_OUT_OF_MEMORY) rc = accum_try<Z, true, AC_IPT>(O, g, T, hp);
     return rc;
 }
 

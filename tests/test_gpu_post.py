@@ -315,3 +315,27 @@ def test_accum_mask_result_memory(grb, nnz):
         d.free()
     assert_csr_equal(download(out, np.int64), ref, what="C<M> = T")
     assert held <= 5 << 20, f"{held} bytes for {ref.nnz} entries"
+
+
+@pytest.mark.parametrize("mask", ["none", "M"])
+@pytest.mark.parametrize("nc,nt", [(200000, 61695), (200000, 61696), (200000, 61952), (264192, 1), (0, 270335)])
+def test_accum_mask_tile_sizes(grb, nc, nt, mask):
+    """Merges on both sides of the number of small tiles (1024), and of the large
+    tiles' ends."""
+    print(f"[post] accum tiles nc={nc} nt={nt} mask={mask}", flush=True)
+    rng = np.random.default_rng(nc + nt)
+    n = 200000
+    C, T = _long_rows(rng, 3, n, nc), _long_rows(rng, 3, n, nt)
+    M = _long_rows(rng, 3, n, 100000) if mask != "none" else None
+    for op, replace in ((1, False), (0, False), (0, True)):
+        ref = O.accum_mask(C, M, T, mask_struct=False, replace=replace, op=op, dtype=np.int64)
+        dC, dT = DevCsr(C, 8), DevCsr(T, 8)
+        dM = DevCsr(M, 8) if M is not None else None
+        out = capi.GmCsrOut()
+        rc = capi.lib().gm_accum_mask(ctypes.byref(out), ctypes.byref(dC.view), ctypes.byref(dM.view) if dM else None,
+                                      False, False, replace, ctypes.byref(dT.view), op)
+        assert rc == 0, capi.last_error()
+        assert_csr_equal(download(out, np.int64), ref, what=f"op={op} replace={replace}")
+        for d in (dC, dT, dM):
+            if d:
+                d.free()
