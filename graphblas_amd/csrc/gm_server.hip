@@ -187,7 +187,7 @@ static int sv_level(gm_server *s, std::vector<std::shared_ptr<SvRequest>> &batch
     const bool valued = !(s->sr.mult_op == GM_MULT_PAIR || s->sr.mult_op == GM_MULT_K);
     hipStream_t st = stream();
     bool want_v = false, all_host = true;
-    int64_t K = 0;
+    int64_t K = 0, vnz = 0;
     // the first-level requests' rows, stacked on the host in batch order and
     // uploaded at once (F: one entry per source, iso one; V with its values)
     std::vector<int64_t> hfp(1, 0), hfj, hvp(1, 0), hvj;
@@ -196,6 +196,7 @@ static int sv_level(gm_server *s, std::vector<std::shared_ptr<SvRequest>> &batch
     {
         want_v |= r->needs_visited();
         K += r->k;
+        vnz += r->V.nnz;
         if (r->F.h) { all_host = false; continue; }
         for (int64_t t = 0; t < r->k; t++)
         {
@@ -276,7 +277,7 @@ static int sv_level(gm_server *s, std::vector<std::shared_ptr<SvRequest>> &batch
         vc.iso = 0;
         tc.nrows = C->M.nrows; tc.ncols = C->M.ncols; tc.p = C->M.p; tc.j = C->M.j;
         tc.x = C->M.x; tc.iso = C->M.iso; tc.type = zt;
-        GM_TRY(gm_accum_mask(&Vn->M, &vc, nullptr, false, true, false, &tc, 6));
+        GM_TRY(gm_accum_mask_sized(&Vn->M, &vc, vnz, nullptr, false, true, false, &tc, C->M.nvals, 6));
     }
     // the result's row pointers and the next level's flop bound per row
     std::vector<int64_t> hp(K + 1), hf(K > 0 ? K : 1);
