@@ -50,20 +50,25 @@ static double now_us()
     return (double) duration_cast<nanoseconds>(steady_clock::now().time_since_epoch()).count() * 1e-3;
 }
 
-// bytes of a held result's entries that are brought to the host at once (64
-// requests on RMAT 20, 66000 entries in 3 batches: 4.5 ms with three waits
-// for every request, 1.06 ms with two for every batch)
+// A held result's entries are brought to the host at once, for all requests of
+// its batch, when that is no more than the waits it saves: 1 MB (100 us) for
+// every request that was copied by itself before, and as much, and at most 8
+// MB; or when most of them are this request's.  64 requests on RMAT 20 (66000
+// entries in 3 batches): 4.5 ms with three waits for every request, 1.03 ms
+// here.  A request of three rows from a batch of 7.9 MB: 516 us with the batch
+// brought at once, 54 us here (86 with three waits).
 constexpr int64_t SV_HOST_MAX = (int64_t) 8 << 20;
+constexpr int64_t SV_HOST_STEP = (int64_t) 1 << 20;
 
 // a device CSR whose row slices belong to one or more requests; freed with
 // the last request that refers to it
 struct SvHold
 {
     gm_csr_out M;
-    // host copies for fetches: the row pointers, and, once a request of a small
-    // result (SV_HOST_MAX) is fetched, all of its entries, so that a batch's
-    // requests take one transfer together instead of three each
+    // host copies for fetches: the row pointers, and all entries once that pays
+    // (SV_HOST_STEP), so that a batch's requests take one transfer together
     std::mutex mu;
+    int64_t singles = 0;                // fetches that copied their own rows
     std::vector<int64_t> hp;
     std::unique_ptr<uint8_t[]> hj, hx;
     SvHold() { memset(&M, 0, sizeof(M)); }
@@ -619,7 +624,8 @@ static int sv_copy_rows(const SvSlice &sl, int64_t k, int64_t *Cp, int64_t *Cj, 
         for (int64_t t = 0; t <= k; t++) Cp[t] = h.hp[sl.row0 + t] - base;
         const int64_t all = h.hp[C.nrows];
         if ((!Cj && !Cx) || nz == 0) return GM_SUCCESS;
-        if (all * (int64_t) (sizeof(int64_t) + xs) <= SV_HOST_MAX)
+        const int64_t bytes = all * (int64_t) (sizeof(int64_t) + xs);
+        if (h.hj || (bytes <= SV_HOST_MAX && (bytes <= SV_HOST_STEP * (1 + h.singles) || all <= 2 * nz)))
         {
             if (!h.hj)
             {
@@ -645,6 +651,7 @@ static int sv_copy_rows(const SvSlice &sl, int64_t k, int64_t *Cp, int64_t *Cj, 
                 return GM_SUCCESS;
             }
         }
+        h.singles++;
     }
     hipStream_t st = stream();
     if (Cj) GM_HIP(hipMemcpyAsync(Cj, C.j + base, sizeof(int64_t) * nz, hipMemcpyDeviceToHost, st), "fetch j");
