@@ -44,12 +44,7 @@ using PuCell = std::conditional_t<PU_U32<S>, uint32_t, typename S::Z>;
 
 struct PushArgs
 {
-    // heavy rows before classification: row, products
-    const uint32_t *hrow;
-    const int64_t *hflops;
-    int64_t dmax;                      // dense rows at most (memory)
-    // the dense rows
-    uint32_t *drow;
+    uint32_t *drow;                    // the dense rows
     int64_t *dflops;
     int64_t D, nw;                     // rows; 32-bit words of a bit row
     const int64_t *pre;                // nnz(A) + 1 running products

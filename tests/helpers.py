@@ -82,6 +82,17 @@ def assert_csr_equal(got: Csr, ref: Csr, fp_tol=None, what=""):
         assert err <= fp_tol, f"{what}: max rel err {err}"
 
 
+def kernels_of(call):
+    """(call's result, the names of the kernel groups that it ran)."""
+    capi.prof_reset()
+    capi.prof_enable(True)
+    try:
+        got = call()
+    finally:
+        capi.prof_enable(False)
+    return got, set(capi.prof_get())
+
+
 # ---------------------------------------------------------------------------
 # direct C-ABI (gm_*) calls on device copies of host CSR arrays
 # ---------------------------------------------------------------------------

@@ -11,7 +11,7 @@ import scipy.sparse as sp
 import pyoracle as O
 from graphblas_amd import capi
 from graphblas_amd import workloads as W
-from helpers import SR, DevCsr, assert_csr_equal, gm_dot3, power_law_csr, rand_csr
+from helpers import SR, DevCsr, assert_csr_equal, gm_dot3, kernels_of, power_law_csr, rand_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -315,10 +315,11 @@ def test_dot3_row_slices(grb, slice_max):
 @pytest.mark.parametrize("valued", [False, True])
 @pytest.mark.parametrize("handle", list(SR))
 def test_dot3_no_long_rows(grb, handle, valued):
-    """Operands whose rows are all shorter than the index length and too large
-    for the no-histogram case: rows of 0, 1 and 127 entries, mask rows with
-    more entries than a wavefront takes, and stretches of more than 64 empty
-    mask rows."""
+    """Operands whose rows are all shorter than the index length, and whose
+    entries and columns are too many for the no-histogram case, through the
+    kernel of LDS tables: rows of 0, 1 and 127 entries, mask rows with more
+    entries than a wavefront takes, and stretches of more than 64 empty mask
+    rows."""
     print(f"[dot3] no long rows {handle} valued={valued}", flush=True)
     rng = np.random.default_rng(len(handle))
     vt = _vals(handle)
@@ -329,17 +330,21 @@ def test_dot3_no_long_rows(grb, handle, valued):
         x = {"fp64": rng.random(len(j)), "int32": rng.integers(-50, 50, len(j)).astype(np.int32),
              "int64": rng.integers(-50, 50, len(j)).astype(np.int64)}.get(values)
         return W.Csr(len(lens), ncols, p, j, x)
-    n, K = 3001, 700
+    n, K, far = 3001, 700, 1500
     A = rows(rng.choice([0, 1, 30, 64, 65, 100, 127], n, p=[.05, .05, .2, .2, .2, .2, .1]), K, vt)
     B = rows(rng.choice([0, 1, 15, 16, 17, 64, 127], n, p=[.05, .05, .1, .1, .1, .3, .3]), K, vt)
-    assert 32 * 8 * (A.nnz + B.nnz) > 64 << 20
+    # the operands' columns far apart, the mask's are B's rows
+    A, B = (W.Csr(X.nrows, K * far, X.p, X.j * far, X.x) for X in (A, B))
+    nz = A.nnz + B.nnz
+    assert 8 * min(32 * nz, 4 * nz + (nz / 128 + 1) * (K * far / 64 + 2)) > 64 << 20
     ml = rng.integers(0, 6, n)
     ml[100:400] = 0
     ml[500] = 1000
     M = rows(ml, n, "int64" if valued else None)
     name, _ = SR[handle]
     ref = O.dot3(name, M, A, B, mask_struct=not valued)
-    got = gm_dot3(handle, M, A, B, mask_struct=not valued)
+    got, ran = kernels_of(lambda: gm_dot3(handle, M, A, B, mask_struct=not valued))
+    assert "dot3_short" in ran and "dot3_phase1" not in ran, ran
     assert_csr_equal(got, ref, fp_tol=FP_TOL if "fp64" in name else None, what=handle)
 
 
@@ -348,8 +353,10 @@ def test_dot3_no_long_rows(grb, handle, valued):
 @pytest.mark.parametrize("handle", list(SR))
 def test_dot3_one_matrix(grb, handle, mask, order):
     """C<M> = A*A' with a mask that is symmetric but for a few entries, whose
-    values (valued mask) differ between the two sides, with diagonal entries:
-    each pair computed once, the others alone; and the mask that is A itself."""
+    values (valued mask) differ between the two sides, with diagonal entries,
+    and the mask that is A itself: with the structural masks an entry and its
+    transposed one are computed together where both are there, with the valued
+    one every entry is computed by itself."""
     import ctypes
     from helpers import ZT, download
     print(f"[dot3] one matrix {handle} {mask} order={order}", flush=True)
@@ -417,4 +424,38 @@ def test_dot3_without_room_for_helpers(grb, handle, one, order):
     got = download(out, ZT[{8: "int64", 6: "int32"}[trip[2]]])
     assert_csr_equal(got, O.dot3(name, G, A, A), what=handle)
     for d in (dA, dB, dM):
+        d.free()
+
+
+@pytest.mark.parametrize("mask", ["A", "lower"])
+@pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GxB_ANY_PAIR_BOOL", "GxB_ANY_SECONDI_INT64",
+                                    "GxB_PLUS_PAIR_INT32"])
+def test_dot3_one_matrix_wide_rows(grb, handle, mask):
+    """C<M> = A*A' with rows that span more than 65536 columns, grouped by the
+    long row: the LDS hash tables of one matrix's rows, which serve an entry
+    whichever operand the long row is read as."""
+    import ctypes
+    from helpers import ZT, download
+    print(f"[dot3] one matrix, wide rows {handle} {mask}", flush=True)
+    rng = np.random.default_rng(len(handle))
+    n, hubs = 90001, 70
+    r = np.concatenate([np.repeat(rng.choice(n, hubs, replace=False), 1500), rng.integers(0, n, 3 * n)])
+    c = rng.integers(0, n, len(r))
+    g = sp.coo_matrix((np.ones(len(r)), (r, c)), shape=(n, n)).tocsr()
+    g = ((g + g.T) > 0).astype(np.float64).tocsr()
+    A = W.Csr.from_scipy(g, keep_values=False)
+    M = A if mask == "A" else W.Csr.from_scipy(sp.tril(g).tocsr(), keep_values=False)
+    name, trip = SR[handle]
+    dA = DevCsr(A, trip[2])
+    dM = dA if mask == "A" else DevCsr(M, 1)
+    out, sr = capi.GmCsrOut(), capi.GmSemiring(*trip)
+    prm = capi.GmDot3Params(0, 0, 0, 0, 2, 0)
+    rc, ran = kernels_of(lambda: capi.lib().gm_dot3(
+        ctypes.byref(out), ctypes.byref(dM.view), True, ctypes.byref(dA.view), ctypes.byref(dA.view),
+        ctypes.byref(sr), ctypes.byref(prm)))
+    assert rc == 0, capi.last_error()
+    assert "dot3_team16_lh" in ran, ran
+    got = download(out, ZT[{8: "int64", 6: "int32", 1: "bool"}[trip[2]]])
+    assert_csr_equal(got, O.dot3(name, M, A, A), what=f"{handle} {mask}")
+    for d in {id(x): x for x in (dA, dM)}.values():
         d.free()

@@ -11,7 +11,7 @@ import pytest
 import pyoracle as O
 from graphblas_amd import capi
 from graphblas_amd import workloads as W
-from helpers import SR, assert_csr_equal, gm_saxpy3, power_law_csr, rand_csr
+from helpers import SR, assert_csr_equal, gm_saxpy3, kernels_of, power_law_csr, rand_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -307,36 +307,43 @@ def test_saxpy3_spread_rows(grb, mask, mode, ncols, handle):
     name, _ = SR[handle]
     kw = {} if M is None else {"M": M, "mask_comp": mask == "!M", "mask_struct": False}
     ref = O.saxpy3(name, A, B, **kw)
-    got = gm_saxpy3(handle, A, B, params=(8, 16, 32, mode), **kw)
+    got, ran = kernels_of(lambda: gm_saxpy3(handle, A, B, params=(8, 16, 32, mode), **kw))
+    # (one column needs no table beyond the LDS; fp64 sums keep their order)
+    if ncols != 31:
+        assert ("sx_push" in ran) == (ncols > 31 and handle != "GrB_PLUS_TIMES_SEMIRING_FP64"), ran
     tol = FP_TOL if handle == "GrB_PLUS_TIMES_SEMIRING_FP64" else None
     assert_csr_equal(got, ref, fp_tol=tol, what=f"spread {handle}")
 
 
 @pytest.mark.parametrize("mask", ["none", "M", "!M"])
+@pytest.mark.parametrize("rows", ["heavy", "light"])
 @pytest.mark.parametrize("ncols", [1023, 1025, 4100])
 @pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GxB_ANY_PAIR_BOOL", "GxB_ANY_SECONDI_INT64",
                                     "GrB_PLUS_TIMES_SEMIRING_INT64", "GrB_MIN_PLUS_SEMIRING_FP64",
                                     "GrB_PLUS_TIMES_SEMIRING_FP64"])
-def test_saxpy3_tiled_rows(grb, mask, ncols, handle):
-    """Rows of C cut into tiles of 1024 columns: none of them heavy enough to be
-    spread over the device, a few very heavy ones, entries of A on both sides
-    of the 64 read at a time, columns on both sides of a tile's end; fp64 sums
-    in the oracle's order, bit for bit."""
-    print(f"[saxpy3] tiled {handle} n={ncols} mask={mask}", flush=True)
+def test_saxpy3_tiled_rows(grb, mask, ncols, rows, handle):
+    """Rows of C cut into tiles of 1024 columns, a few very heavy ones among
+    them, entries of A on both sides of the 64 read at a time, columns on both
+    sides of a tile's end; fp64 sums in the oracle's order, bit for bit.  Heavy
+    rows, with many products a tile, are the fp64 sums' only (the others spread
+    them over the device); light ones, of which there are more, everyone's."""
+    print(f"[saxpy3] tiled {handle} n={ncols} {rows} mask={mask}", flush=True)
     rng = np.random.default_rng(ncols + len(mask))
     vt = _vals(handle)
-    K, m = 400, 900
+    K, m = 400, 900 if rows == "heavy" else 4500
     lens = np.where(np.arange(m) % 300 == 7, K, rng.choice([0, 1, 40, 63, 64, 65, 100], m))
     p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
     j = np.concatenate([np.sort(rng.choice(K, size=int(l), replace=False)) for l in lens]).astype(np.int64)
     x = {"fp64": rng.random(len(j)), "int64": rng.integers(-9, 9, len(j)).astype(np.int64)}.get(vt)
     A = W.Csr(m, K, p, j, x)
-    B = rand_csr(K, ncols, 60.0 / ncols, rng, vt, empty_rows=0.1)
+    B = rand_csr(K, ncols, (60.0 if rows == "heavy" else 1.5) / ncols, rng, vt, empty_rows=0.1)
     M = rand_csr(m, ncols, 0.2, rng, "int64") if mask != "none" else None
     kw = {} if M is None else {"M": M, "mask_comp": mask == "!M", "mask_struct": False}
     ref = O.saxpy3(SR[handle][0], A, B, **kw)
     for mode in (1, 2):
-        got = gm_saxpy3(handle, A, B, params=(8, 16, 32, mode), **kw)
+        got, ran = kernels_of(lambda: gm_saxpy3(handle, A, B, params=(8, 16, 32, mode), **kw))
+        tiled = rows == "light" or handle == "GrB_PLUS_TIMES_SEMIRING_FP64"
+        assert ("sx_tile_num" in ran) == tiled, ran
         assert_csr_equal(got, ref, what=f"tiled {handle} mode={mode}")
 
 
