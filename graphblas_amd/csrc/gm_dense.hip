@@ -651,7 +651,16 @@ static int dn_mxm_run(gm_dense_out *C, const gm_csr *Ms, const gm_dense *Md, boo
             if (As)
             {
                 const int64_t hm = std::min(g.m, DN_HUB_ROWS);
-                if (!hubs.alloc(sizeof(uint32_t) * hm)) return set_error(GM_OUT_OF_MEMORY, "dense product: rows");
+                if (!hubs.alloc(sizeof(uint32_t) * hm))
+                {
+                    // without room for every row, for as many hubs as A's entries make
+                    int64_t *nz = (int64_t *) pinned_scratch(sizeof(int64_t));
+                    if (!nz) return set_error(GM_OUT_OF_MEMORY, "pinned scratch");
+                    GM_HIP(hipMemcpyAsync(nz, g.Ap + g.m, sizeof(int64_t), hipMemcpyDeviceToHost, st), "nnz(A)");
+                    GM_HIP(hipStreamSynchronize(st), "nnz(A) sync");
+                    if (!hubs.alloc(sizeof(uint32_t) * (nz[0] / (DN_HUB + 1) + 1)))
+                        return set_error(GM_OUT_OF_MEMORY, "dense product: rows");
+                }
                 k_dn_hubs<<<dn_grid((hm + DN_NT - 1) / DN_NT), DN_NT, 0, st>>>(g.Ap, hm, hubs.as<uint32_t>(), ctr);
             }
             const bool masked = g.mkind != 0;

@@ -405,3 +405,32 @@ def test_saxbit_excluded_columns_cost(grb):
         best[what] = min(ts)
         assert C.nvals == (m * n if M is None else 0)
     assert best["none"] <= 0.6 * best["all"], best
+
+
+def test_saxbit_without_room_for_hub_list(grb):
+    """The hub rows' list (the fourth allocation) forced not to fit: one of the
+    size that A's entries allow takes its place."""
+    import ctypes
+    rng = np.random.default_rng(8)
+    A = _hub_csr(rng, 1500, [0, 513, 3, 1500, 512, 700], "fp64")
+    B = rand_csr(1500, 65, 1.0, rng, "fp64")
+    L = capi.lib()
+    dA, dB = capi.DeviceCsr(A, 11), L.gm_malloc(8 * 1500 * 65)
+    x = np.ascontiguousarray(_dense_of(B, np.float64)[0])
+    assert L.gm_memcpy_h2d(dB, x.ctypes.data, x.nbytes) == 0
+    out, sr = capi.GmDenseOut(), capi.GmSemiring(*SR["GrB_PLUS_TIMES_SEMIRING_FP64"][1])
+    bd = capi.GmDense(1500, 65, None, dB, 0, 11)
+    L.gm_debug_fail_after(3)
+    try:
+        rc = L.gm_saxbit(ctypes.byref(out), None, None, False, True, ctypes.byref(dA.view), None, None,
+                         ctypes.byref(bd), ctypes.byref(sr), None)
+    finally:
+        L.gm_debug_fail_after(-1)
+    assert rc == 0, capi.last_error()
+    got, b = np.zeros((6, 65)), np.zeros((6, 65), dtype=np.int8)
+    assert L.gm_memcpy_d2h(got.ctypes.data, out.x, got.nbytes) == 0
+    assert L.gm_memcpy_d2h(b.ctypes.data, out.b, b.nbytes) == 0
+    assert_csr_equal(_csr_of(got, b != 0), O.saxpy3("plus_times_fp64", A, B), what="without a hub list")
+    for q in (dB, out.x, out.b):
+        L.gm_free(q)
+    dA.free()
