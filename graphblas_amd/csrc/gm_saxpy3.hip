@@ -82,7 +82,8 @@ struct SxArgs
     int64_t *Cp;
     int64_t *Ci;
     void *Cx;
-    uint32_t *rows;               // SX_NBINS x m row ids
+    uint32_t *rows;               // SX_NBINS x ls row ids, or NULL: rows are only counted
+    int64_t ls;
     unsigned long long *cnt;      // bin counters and totals (CNT_*)
     int64_t *hflops;              // per BIN_HVY row: its flops
     const unsigned long long *rowf;   // NULL, or the rows' flops (few-row A)
@@ -451,10 +452,10 @@ __global__ __launch_bounds__(SX_NT) void k_sx_flops(SxArgs g, int64_t fs, int li
         if (bin >= 0)
         {
             const unsigned long long slot = s_base[bin] + local;
-            g.rows[(int64_t) bin * g.m + (int64_t) slot] = (uint32_t) i;
+            if (g.rows) g.rows[(int64_t) bin * g.ls + (int64_t) slot] = (uint32_t) i;
             if (bin == BIN_HVY)
             {
-                g.hflops[slot] = f;
+                if (g.rows) g.hflops[slot] = f;
                 atomicAdd(&g.cnt[CNT_HFLOPS], (unsigned long long) f);
             }
         }
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops
     const int64_t nt = (g.n + TL_W - 1) / TL_W;
     for (int64_t q = (int64_t) blockIdx.x * SX_NT + threadIdx.x; q < count; q += (int64_t) gridDim.x * SX_NT)
     {
-        const uint32_t i = g.rows[(int64_t) BIN_HVY * g.m + q];
+        const uint32_t i = g.rows[(int64_t) BIN_HVY * g.ls + q];
         const int64_t f = g.hflops[q], la = g.Ap[i + 1] - g.Ap[i];
         const bool most = (double) f * 512 > total;
         const bool push = dmax > 0 && g.table != 1;
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops
             const int64_t d = (int64_t) atomicAdd(&g.cnt[BIN_DNS], 1ull);
             if (d < dmax)
             {
-                g.rows[(int64_t) BIN_DNS * g.m + d] = i;
+                g.rows[(int64_t) BIN_DNS * g.ls + d] = i;
                 dflops[d] = f;
                 continue;
             }
@@ -512,8 +513,8 @@ __global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops
         {
             if ((int64_t) atomicAdd(&g.cnt[BIN_TIL], 1ull) < tmax)
             {
-                if (most) g.rows[(int64_t) BIN_TIL * g.m + atomicAdd(&g.cnt[CNT_TILF], 1ull)] = i;
-                else g.rows[(int64_t) (BIN_TIL + 1) * g.m - 1 - atomicAdd(&g.cnt[CNT_TILB], 1ull)] = i;
+                if (most) g.rows[(int64_t) BIN_TIL * g.ls + atomicAdd(&g.cnt[CNT_TILF], 1ull)] = i;
+                else g.rows[(int64_t) (BIN_TIL + 1) * g.ls - 1 - atomicAdd(&g.cnt[CNT_TILB], 1ull)] = i;
                 atomicAdd(&g.cnt[CNT_TILA], (unsigned long long) la);
                 continue;
             }
@@ -527,7 +528,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_classify(SxArgs g, int64_t *dflops
                         (g.table == 2 && lgd <= lg + 4);
         if (dn && lgd > lg) lg = lgd;
         const int64_t slot = (int64_t) atomicAdd(&g.cnt[BIN_GLB], 1ull);
-        g.rows[(int64_t) BIN_GLB * g.m + slot] = i;
+        g.rows[(int64_t) BIN_GLB * g.ls + slot] = i;
         g.gtab_off[slot] = (int64_t) atomicAdd(&g.cnt[CNT_SLOTS], 1ull << lg);
         g.gtab_log2[slot] = lg;
     }
@@ -544,8 +545,8 @@ __global__ __launch_bounds__(SX_NT) void k_sx_sum_big(SxArgs g, int64_t dmax)
     {
         int64_t count = (int64_t) g.cnt[b < 5 ? bins[b] : b == 5 ? CNT_TILF : CNT_TILB];
         if (bins[b] == BIN_DNS && count > dmax) count = dmax;
-        const uint32_t *list = g.rows + (int64_t) bins[b] * g.m;
-        if (b == 6) list += g.m - count;
+        const uint32_t *list = g.rows + (int64_t) bins[b] * g.ls;
+        if (b == 6) list += g.ls - count;
         for (int64_t q = (int64_t) blockIdx.x * SX_NT + threadIdx.x; q < count;
              q += (int64_t) gridDim.x * SX_NT)
             sum += (unsigned long long) g.Cp[list[q]];
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_single(SxArgs g)
     using Z = typename S::Z;
     const int lane = threadIdx.x & 63;
     const int64_t count = (int64_t) g.cnt[BIN_SINGLE];
-    const uint32_t *list = g.rows + (int64_t) BIN_SINGLE * g.m;
+    const uint32_t *list = g.rows + (int64_t) BIN_SINGLE * g.ls;
     for (int64_t q = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6); q < count;
          q += (int64_t) gridDim.x * 4)
     {
@@ -847,7 +848,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_wave(SxArgs g, int bin)
     __shared__ uint32_t s_own[NWV][SX_OWN];
     const int wv = threadIdx.x >> 6;
     const int64_t count = (int64_t) g.cnt[bin];
-    const uint32_t *list = g.rows + (int64_t) bin * g.m;
+    const uint32_t *list = g.rows + (int64_t) bin * g.ls;
     for (int64_t q = (int64_t) blockIdx.x * NWV + wv; q < count; q += (int64_t) gridDim.x * NWV)
     {
         sx_row<S, 64, PHASE>(g, (int64_t) list[q], s_keys[wv], s_vals[wv], s_list[wv], LOGT,
@@ -869,7 +870,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_block(SxArgs g)
     __shared__ uint32_t s_own[SX_NT / 64][SX_OWN];
     __shared__ int64_t s_red[SX_NT / 64 + 1];
     const int64_t count = (int64_t) g.cnt[BIN_BLK];
-    const uint32_t *list = g.rows + (int64_t) BIN_BLK * g.m;
+    const uint32_t *list = g.rows + (int64_t) BIN_BLK * g.ls;
     for (int64_t q = blockIdx.x; q < count; q += gridDim.x)
     {
         sx_row<S, SX_NT, PHASE>(g, (int64_t) list[q], s_keys, s_vals, s_list, LOGT,
@@ -887,7 +888,7 @@ __global__ __launch_bounds__(SX_NT) void k_sx_global(SxArgs g)
     __shared__ uint32_t s_own[SX_NT / 64][SX_OWN];
     __shared__ int64_t s_red[SX_NT / 64 + 1];
     const int64_t count = (int64_t) g.cnt[BIN_GLB];
-    const uint32_t *list = g.rows + (int64_t) BIN_GLB * g.m;
+    const uint32_t *list = g.rows + (int64_t) BIN_GLB * g.ls;
     for (int64_t q = blockIdx.x; q < count; q += gridDim.x)
     {
         const int64_t off = g.gtab_off[q];
@@ -1407,7 +1408,7 @@ static int sx_push_build(SxArgs &g, SxPush &p, int64_t D, int64_t nnzA, int64_t 
     const int64_t cap = (int64_t) cu_count() * 8;
     PushArgs &h = p.h;
     h.D = D;
-    h.drow = g.rows + (int64_t) BIN_DNS * g.m;
+    h.drow = g.rows + (int64_t) BIN_DNS * g.ls;
     h.nw = (g.n + 31) >> 5;
     h.nseg = (g.n + PU_SEG - 1) / PU_SEG;
     const int64_t items = hflops / PU_CH + D + 1;
@@ -1481,8 +1482,8 @@ static int sx_tile_build(SxArgs &g, SxTile &x, const int64_t *hc, int64_t kb)
     t.nf = hc[CNT_TILF];
     t.T = hc[BIN_TIL];
     t.nt = (g.n + TL_W - 1) / TL_W;
-    t.front = g.rows + (int64_t) BIN_TIL * g.m;
-    t.back = t.front + g.m - 1;
+    t.front = g.rows + (int64_t) BIN_TIL * g.ls;
+    t.back = t.front + g.ls - 1;
     if (!x.bits.alloc((size_t) (t.T * t.nt) * (TL_W / 8)) || !x.seg.alloc(sizeof(int64_t) * (size_t) (t.T * t.nt + 1)) ||
         !x.next.alloc(128 * sizeof(unsigned long long)))
         return set_error(GM_OUT_OF_MEMORY, "saxpy3: tiled rows (%lld)", (long long) t.T);
@@ -1527,7 +1528,7 @@ static int sx_count(SxArgs &g, int64_t fs, int list_small, int64_t dmax, int64_t
         }
         k_sx_flops<<<sx_grid(g.m, SX_NT / TG, (int64_t) cu_count() * 16), SX_NT, 0, st>>>(g, fs, list_small);
         g.rowf = nullptr;
-        k_sx_classify<<<sx_grid(g.m, SX_NT, (int64_t) cu_count()), SX_NT, 0, st>>>(g, dflops, dmax, tmax);
+        if (g.rows) k_sx_classify<<<sx_grid(g.m, SX_NT, (int64_t) cu_count()), SX_NT, 0, st>>>(g, dflops, dmax, tmax);
         GM_HIP(hipGetLastError(), "k_sx_flops");
     }
     GM_HIP(hipMemcpyAsync(hp, g.cnt, SX_NCNT * sizeof(unsigned long long), hipMemcpyDeviceToHost, st), "bin counts");
@@ -1610,7 +1611,7 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     g.mask_struct = (mask_struct || !M || !M->x) ? 1 : 0;
     g.mode = !M ? MODE_NONE : (mask_comp ? MODE_NOTMASK : MODE_MASK);
     g.Cp = Cp.as<int64_t>(); g.Ci = nullptr; g.Cx = nullptr;
-    g.rows = nullptr; g.cnt = cnt.as<unsigned long long>();
+    g.rows = nullptr; g.ls = 0; g.cnt = cnt.as<unsigned long long>();
     g.hflops = nullptr; g.rowf = nullptr;
     g.gtab_off = nullptr; g.gtab_log2 = nullptr;
     g.gkeys = nullptr; g.gvals = nullptr; g.glist = nullptr;
@@ -1691,13 +1692,31 @@ static int saxpy3_run(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_
     if (!all_small)
     {
         // the bins' row lists and the heavy rows' records, in one block
-        if (!lists.alloc((size_t) m * (3 * sizeof(int64_t) + (SX_NBINS + 1) * sizeof(uint32_t))))
-            return set_error(GM_OUT_OF_MEMORY, "saxpy3: row lists");
-        g.gtab_off = lists.as<int64_t>();
-        g.hflops = g.gtab_off + m;
-        dflops = g.hflops + m;
-        g.rows = (uint32_t *) (dflops + m);
-        g.gtab_log2 = (int32_t *) (g.rows + SX_NBINS * m);
+        auto place = [&](int64_t ls) {
+            if (!lists.alloc((size_t) ls * (3 * sizeof(int64_t) + (SX_NBINS + 1) * sizeof(uint32_t)))) return false;
+            g.ls = ls;
+            g.gtab_off = lists.as<int64_t>();
+            g.hflops = g.gtab_off + ls;
+            dflops = g.hflops + ls;
+            g.rows = (uint32_t *) (dflops + ls);
+            g.gtab_log2 = (int32_t *) (g.rows + SX_NBINS * ls);
+            return true;
+        };
+        if (!place(m))
+        {
+            // without room for every row in every bin the rows are counted first
+            GM_TRY(sx_count(g, fs, fused ? 0 : 1, dmax, tmax, nullptr, hc, hp));
+            if (fused && (double) hc[CNT_SMALL] * (double) entry_bytes > budget)
+            {
+                fused = false;
+                k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
+                GM_TRY(sx_count(g, fs, 1, dmax, tmax, nullptr, hc, hp));
+            }
+            int64_t ls = 1;
+            for (int bin : {BIN_SINGLE, BIN_WS, BIN_WL, BIN_BLK, BIN_HVY}) ls = hc[bin] > ls ? hc[bin] : ls;
+            k_sx_fill_u64<<<1, 64, 0, st>>>(g.cnt, SX_NCNT);
+            if (!place(ls)) return set_error(GM_OUT_OF_MEMORY, "saxpy3: row lists");
+        }
         GM_TRY(sx_count(g, fs, fused ? 0 : 1, dmax, tmax, dflops, hc, hp));
         cap_small = hc[CNT_SMALL];
         if (fused && (double) cap_small * (double) entry_bytes > budget)

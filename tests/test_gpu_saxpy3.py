@@ -443,3 +443,35 @@ def test_saxpy3_without_room_for_tables(grb, rows, handle, mode, mask):
     for d in (dA, dB, dM):
         if d:
             d.free()
+
+
+@pytest.mark.parametrize("mask", ["none", "M", "!M"])
+@pytest.mark.parametrize("bins,mode", [((0, 0, 0), 0), ((8, 16, 64), 1), ((8, 16, 64), 2)])
+@pytest.mark.parametrize("handle", ["GxB_PLUS_PAIR_INT64", "GrB_PLUS_TIMES_SEMIRING_FP64"])
+def test_saxpy3_without_room_for_row_lists(grb, handle, bins, mode, mask):
+    """The row lists (the third allocation) forced not to fit: the rows are
+    counted and the lists sized by their bins; rows of every bin."""
+    import ctypes
+    from helpers import ZT, DevCsr, download
+    rng = np.random.default_rng(mode)
+    vt = _vals(handle)
+    A = power_law_csr(1500, 12, rng, values=vt)
+    B = power_law_csr(1500, 12, rng, values=vt)
+    M = rand_csr(1500, 1500, 0.1, rng, "int64") if mask != "none" else None
+    kw = {} if M is None else {"M": M, "mask_comp": mask == "!M", "mask_struct": True}
+    name, trip = SR[handle]
+    L = capi.lib()
+    dA, dB, dM = DevCsr(A, trip[2]), DevCsr(B, trip[2]), DevCsr(M, 8) if M is not None else None
+    out, sr, prm = capi.GmCsrOut(), capi.GmSemiring(*trip), capi.GmSaxpy3Params(*bins, mode, 0)
+    L.gm_debug_fail_after(2)
+    try:
+        rc = L.gm_saxpy3(ctypes.byref(out), ctypes.byref(dM.view) if dM else None, mask == "!M", True,
+                         ctypes.byref(dA.view), ctypes.byref(dB.view), ctypes.byref(sr), ctypes.byref(prm))
+    finally:
+        L.gm_debug_fail_after(-1)
+    assert rc == 0, capi.last_error()
+    got = download(out, ZT[{8: "int64", 11: "fp64"}[trip[2]]])
+    assert_csr_equal(got, O.saxpy3(name, A, B, **kw), what=f"{handle} {mask}")
+    for d in (dA, dB, dM):
+        if d:
+            d.free()
