@@ -221,8 +221,8 @@ __device__ __forceinline__ int dn_put(const DnArgs &g, int64_t i, int64_t c, boo
 // the device beside them.
 // RMAT n = 65536, 1.82M entries, times 64 full columns, fp64: 7.2 ms with a
 // workgroup per row, LDS accumulators and one read in flight; 2.2 ms without
-// the hub stages; 0.69 ms here.  B's rows, 931 MB, come from L2 and the
-// Infinity Cache.
+// the hub stages; 0.69 ms here.  Of B's rows, 931 MB, 450 MB are
+// read past L2.
 constexpr int DN_UN = 16;
 constexpr int DN_RT = 1024;                 // threads
 constexpr int DN_SPT = 8;                   // products of a stage per thread

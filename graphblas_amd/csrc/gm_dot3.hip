@@ -1073,9 +1073,10 @@ __global__ __launch_bounds__(D3_NT) void k_dot3_block_grp(Dot3Args g, const uint
 // A(i,:) into an LDS hash table of columns and positions once; teams of 16
 // lanes then look their B(j,:) up there, SR_UN reads ahead.  Neighbouring
 // entries share the table, and an entry costs its B row's elements instead of
-// the merge of both lists.  Bound by the reads' latency, covered by 24
-// wavefronts per CU.  720000 valued mask entries, rows of 40, fp64: phase1 and
-// the team merges took 222 us of a 310 us call; 179 us for the call here.
+// the merge of both lists.  Bound by the reads' latency (its wavefronts wait
+// two thirds of their cycles, at 20 per CU and 2.3 TB/s past L2).  720000
+// valued mask entries, rows of 40, fp64: phase1 and the team merges took 222
+// us of a 310 us call; 179 us for the call here.
 constexpr int64_t SR_MAX = 128;
 constexpr int SR_SLOTS = 256;
 constexpr int SR_G = 16;
@@ -2505,7 +2506,9 @@ static int dot3_bitmaps(Dot3Args &g, D3Front &f, const gm_csr *A, const gm_csr *
     const int64_t gcap = (int64_t) cu_count() * 8;
     const double wbytes = 8.0 + (need_rank ? 4.0 : 0.0);
     int64_t T = INT64_MAX, total_words = 0;
-    no_long = false;              // known: every row is shorter than minlen
+    // known: every row is shorter than minlen (small operands, whose indexes need
+    // no histogram, are not looked at for it and take the bins)
+    no_long = false;
     if (minlen > 0)
     {
         const double nz = (double) f.nza + (shared ? 0.0 : (double) f.nzb);
@@ -2816,8 +2819,12 @@ static int dot3_run(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_c
         // sample of M's entries finds its transposed place three times in four,
         // one of each such pair is computed.  The search costs 3.7 ms for the 83M
         // entries of a 256-graph batch and saves 14.6 ms of 46.0.  Structural
-        // masks only: with int32 mask values the search was paid without fewer
-        // entries in the bins (4096 graphs, 1.46e9 entries: 698 ms, 539 without)
+        // masks only: a mask's value at the mate's place must be tested as well,
+        // and with mask_true in phase1's search the compiler (clang of ROCm 7.2)
+        // lost the assignment of the place that follows it: of 54M entries, each
+        // with its mate in M and true, none got one (by counters, and the
+        // register stays at D3_ALONE in the assembly), so the search was paid
+        // for nothing (4096 graphs, int32 masks: 698 ms, 539 without it)
         bool sym = g.one && g.mask_struct && Mnz >= ((int64_t) 1 << 16) && 4 * front->pairs >= 3 * SYM_SAMPLES;
         // group deferred entries by probed row: explicit, or by default for
         // masks large enough that the sort pays for itself

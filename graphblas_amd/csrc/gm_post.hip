@@ -198,8 +198,8 @@ enum { AC_NONE = 0, AC_OWN = 1, AC_BOTH = 2, AC_OTHER = 3 };
 // vector is one row), so the unit is the entry: the rows of a tile's ends are
 // searched once, each entry searches only between them.  Bound by the searches'
 // dependent reads.  C and T of 2^20 rows with 8 entries each, int64, PLUS: 1043
-// us with a thread per row walking it twice, 680 us here; four hops of a
-// shortest-path vector that grows to 44000 entries (one row): 66 ms and 1.4
+// us with a thread per row walking it twice, 685 us here; four hops of a
+// shortest-path vector that grows to 44000 entries (one row): 66 ms and 1.1
 // ms with their products.
 // IPT is AC_IPT, or 1 for a merge of at most AC_FEW such tiles, which would leave
 // most CUs idle: a thread's eight searches follow one another.
