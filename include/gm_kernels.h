@@ -347,7 +347,9 @@ int gm_saxpy3(gm_csr_out *C, const gm_csr *M, bool mask_comp, bool mask_struct,
 // C = A*B', or C<!M> = A*B' when M is given, for an A of one row (a vector) and
 // B by rows with nnz_b entries: the product GrB_mxv runs, without the transpose
 // of B that saxpy3 needs.  The result is saxpy3's (ANY keeps the largest k;
-// fp64 sums are tree sums).  Returns GM_NO_VALUE for a shape it does not take.
+// fp64 sums are tree sums).  Returns GM_NO_VALUE for a shape it does not take and
+// GM_OUT_OF_MEMORY where its vectors, as long as B's dimensions, do not fit;
+// GrB_mxm transposes B in either case.
 // The reference transposes or uses its dot products here
 // (Source/mxm/GrB_mxv.c, GB_AxB_meta.c).
 int gm_vxm_bt(gm_csr_out *C, const gm_csr *M, bool mask_struct, const gm_csr *A, const gm_csr *B,
